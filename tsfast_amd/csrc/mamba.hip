@@ -12,7 +12,8 @@
 // and LDS traffic and keeps every SIMD busy:
 //
 //  * Workgroup = one batch row b x a tile of DT=32 channels, all N states, walking the whole
-//    sequence. NG lanes share a channel, each holding NPT = NS/NG states in VGPRs (NG = 8 for
+//    sequence, or one time segment of it where the rows and tiles alone leave the chip idle
+//    (see segments below). NG lanes share a channel, each holding NPT = NS/NG states in VGPRs (NG = 8 for
 //    N >= 8), so the grid B * D/32 (768 workgroups of 4 waves at config 3) puts three
 //    workgroups on every CU with no tail; workgroups are renumbered so that each XCD works on a
 //    contiguous range of tiles (neighbouring tiles share L2 lines).
@@ -203,6 +204,163 @@ TSF_DEV float row_bcast(float x, int k) {
   }
 }
 
+// ----------------------------------------------------------------------------------- segments
+// A walk over the whole sequence has B x ceil(D / 32) workgroups. Where that leaves the chip idle
+// (a recording of a few batch rows, an identification model's width) the sequence is cut into
+// segments that run side by side: mamba_segment_kernel reduces each segment to its state map
+// (every state decays by exp(A S) over it, S the segment's sum of delta, and gains the segment's
+// own end state), and each workgroup of the main kernel starts from the composition of the maps
+// before (adjoint: behind) its segment. The maps cost about half of the forward's work again.
+// Layout of the maps: per segment, sums S [B, D], then end states [B, N, D].
+TSF_HOST_DEV int64_t segment_floats(int64_t B, int64_t D, int64_t N) { return B * D * (N + 1); }
+
+// x_j <- exp(A S_k) x_j + e_k over the segments k = first, first + step, .. before last, in order.
+// `state(j)` is the state this lane holds in slot j, A2 its decay rate times log2(e).
+template <int NPT, typename F>
+TSF_DEV void compose_segments(const float* __restrict__ segs, int64_t first, int64_t last, int64_t step, int64_t B,
+                              int64_t b, int64_t D, int64_t d, int N, F state, bool act, const float* A2, float* x) {
+  if (first == last || !act) return;
+  const int64_t stride = segment_floats(B, D, N);
+  const int64_t so = b * D + d, eo = B * D + b * N * D + d;
+  for (int64_t k = first; k != last;) {
+    // the maps of up to four segments are loaded together, ahead of the chain of multiply-adds
+    float S[4], e[4][NPT];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int64_t kk = (last - k) * step > q ? k + q * step : k;
+      const float* p = segs + kk * stride;
+      S[q] = p[so];
+#pragma unroll
+      for (int j = 0; j < NPT; ++j) e[q][j] = state(j) < N ? p[eo + state(j) * D] : 0.0f;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (k == last) break;
+#pragma unroll
+      for (int j = 0; j < NPT; ++j) x[j] = fmaf(fast_exp2(A2[j] * S[q]), x[j], e[q][j]);
+      k += step;
+    }
+  }
+}
+
+// The map of one segment: forward, the state after it from a zero state; ADJ, the adjoint that
+// leaves its first step to the left (lam_t G_t) with none entering from the right. Same tiling as
+// the forward (32 channels, NG lanes a channel), two LDS buffers, so one barrier per round of TF
+// steps. Bound by the exp and three multiply-adds per state element.
+template <typename TIO, int NS, bool ADJ>
+__global__ void __launch_bounds__(FCfg<NS>::TH) mamba_segment_kernel(
+    const TIO* __restrict__ draw, const float* __restrict__ A, const TIO* __restrict__ V, const TIO* __restrict__ u,
+    const TIO* __restrict__ z, float* __restrict__ segs, int64_t B, int64_t L, int64_t D, int N, int64_t seg_len) {
+  using C = FCfg<NS>;
+  constexpr int NPT = C::NPT, NG = C::NG, DT = C::DT, TH = C::TH, TF = C::TF;
+  constexpr int IT = C::IT_F, BCI = C::BC_F;
+  __shared__ float2 s_sc[2][TF][DT];  // (delta, delta * u) or (delta, gy)
+  __shared__ float s_v[2][TF][NS];    // B, or C
+  const int tid = threadIdx.x;
+  int64_t tile, b;
+  xcd_remap((D + DT - 1) / DT, tile, b);
+  // the forward composes every segment but the last one, the adjoint every one but the first
+  const int64_t seg = b / B + (ADJ ? 1 : 0);
+  b %= B;
+  const int64_t t_begin = seg * seg_len, t_end = t_begin + seg_len < L ? t_begin + seg_len : L;
+  const int64_t d0 = tile * DT;
+  const int pr = tid & 1;
+  const int dl = (tid >> 1) & (DT - 1);
+  const int n0 = (2 * (tid / (2 * DT)) + pr) * NPT;
+  const int64_t d = d0 + dl;
+  const bool act = d < D;
+  const int od = tid % DT;
+  const bool oact = d0 + od < D;
+  const int64_t rowD = b * L * D + d0, rowN = b * L * N;
+  const uint32_t Du = (uint32_t)D, Nu = (uint32_t)N;
+  const TIO* __restrict__ drw = draw + rowD;
+  const TIO* __restrict__ urw = u + rowD;
+  const TIO* __restrict__ zrw = ADJ ? z + rowD : nullptr;
+  const TIO* __restrict__ vrw = V + rowN;
+  float A2[NPT], x[NPT];
+#pragma unroll
+  for (int j = 0; j < NPT; ++j) {
+    A2[j] = (act && n0 + j < N) ? A[d * N + n0 + j] * kLog2e : 0.0f;
+    x[j] = 0.0f;
+  }
+  TIO r_dr[IT], r_u[IT], r_z[IT], r_v[BCI];
+  auto load_round = [&](int64_t t0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < IT; ++k) {
+      const int idx = tid + k * TH, t = idx / DT;
+      const bool v = idx < TF * DT && oact && t0 + t < t_end;
+      const uint32_t o = ((uint32_t)t0 + (uint32_t)t) * Du + (uint32_t)od;
+      r_dr[k] = v ? ld32(drw, o) : io_zero<TIO>();
+      r_u[k] = v ? ld32(urw, o) : io_zero<TIO>();
+      if (ADJ) r_z[k] = v ? ld32(zrw, o) : io_zero<TIO>();
+    }
+#pragma unroll
+    for (int k = 0; k < BCI; ++k) {
+      const int idx = tid + k * TH, t = idx / NS, n = idx % NS;
+      const bool v = idx < TF * NS && n < N && t0 + t < t_end;
+      r_v[k] = v ? ld32(vrw, ((uint32_t)t0 + (uint32_t)t) * Nu + (uint32_t)n) : io_zero<TIO>();
+    }
+  };
+  const int64_t rounds = (t_end - t_begin + TF - 1) / TF;
+  auto round_start = [&](int64_t r) { return t_begin + (ADJ ? rounds - 1 - r : r) * TF; };
+  load_round(round_start(0));
+  float S = 0.0f;  // this owner's share of its channel's sum of delta
+  for (int64_t r = 0; r < rounds; ++r) {
+    const int buf = (int)(r & 1);
+    const int64_t t0 = round_start(r);
+#pragma unroll
+    for (int k = 0; k < IT; ++k) {
+      const int idx = tid + k * TH;
+      if ((TF * DT) % TH == 0 || idx < TF * DT) {
+        // steps past the end and idle channels: delta = 0 and no input, an identity step
+        const bool live = oact && t0 + idx / DT < t_end;
+        const float delta = live ? softplus_ref(to_f32(r_dr[k])) : 0.0f;
+        const float uu = to_f32(r_u[k]);
+        float w = delta * uu;
+        if (ADJ) {
+          const float zz = to_f32(r_z[k]);
+          w = live ? uu * zz * sigmoid_fast(zz) : 0.0f;
+        }
+        S += delta;
+        s_sc[buf][idx / DT][idx % DT] = make_float2(delta, w);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < BCI; ++k) {
+      const int idx = tid + k * TH;
+      if (idx < TF * NS) s_v[buf][idx / NS][idx % NS] = to_f32(r_v[k]);
+    }
+    if (r + 1 < rounds) load_round(round_start(r + 1));
+    __syncthreads();
+#pragma unroll 8
+    for (int i = 0; i < TF; ++i) {
+      const int t = ADJ ? TF - 1 - i : i;
+      const float2 sc = s_sc[buf][t][dl];
+#pragma unroll
+      for (int j = 0; j < NPT; ++j) {
+        const float lam = fast_exp2(sc.x * A2[j]), v = s_v[buf][t][n0 + j];
+        x[j] = ADJ ? lam * fmaf(sc.y, v, x[j]) : fmaf(lam, x[j], sc.y * v);
+      }
+    }
+  }
+  float* __restrict__ out = segs + seg * segment_floats(B, D, N);
+  if (act) {
+#pragma unroll
+    for (int j = 0; j < NPT; ++j)
+      if (n0 + j < N) out[B * D + (b * N + n0 + j) * D + d] = x[j];
+  }
+  // the owners' shares of S through the buffer of the round before the last
+  float* red = reinterpret_cast<float*>(&s_sc[rounds & 1][0][0]);
+  red[tid] = S;
+  __syncthreads();
+  if (tid < DT && oact) {
+    float s = 0.0f;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) s += red[g * DT + tid];
+    out[b * D + d0 + tid] = s;
+  }
+}
+
 // ------------------------------------------------------------------------------------ forward
 // SAVE: training forward (writes the checkpoints and y to chk); chk is unused otherwise.
 template <typename TIO, int NS, bool SAVE>
@@ -210,7 +368,8 @@ __global__ void __launch_bounds__(FCfg<NS>::TH, FCfg<NS>::WAVES >= 8 ? 3 : 1) ma
     const TIO* __restrict__ draw, const float* __restrict__ A, const TIO* __restrict__ Bt,
     const TIO* __restrict__ Ct, const TIO* __restrict__ u, const TIO* __restrict__ z, const float* __restrict__ Dp,
     const float* __restrict__ h0, TIO* __restrict__ out, float* __restrict__ h_last, float* __restrict__ chk,
-    int64_t L, int64_t D, int N, int64_t NC, unsigned cus) {
+    const float* __restrict__ segs, int64_t B, int64_t L, int64_t D, int N, int64_t NC, int64_t seg_len,
+    unsigned cus) {
   using C = FCfg<NS>;
   constexpr int NPT = C::NPT, NG = C::NG, DT = C::DT, TH = C::TH, CHK = C::CHK, TF = C::TF;
   constexpr int IT = C::IT_F, BCI = C::BC_F;
@@ -225,6 +384,10 @@ __global__ void __launch_bounds__(FCfg<NS>::TH, FCfg<NS>::WAVES >= 8 ? 3 : 1) ma
   const int tid = threadIdx.x;
   int64_t tile, b;
   xcd_remap((D + DT - 1) / DT, tile, b);
+  // this workgroup's time segment [t_begin, t_end) of its batch row (the whole row when unsplit)
+  const int64_t seg = b / B;
+  b -= seg * B;
+  const int64_t t_begin = seg * seg_len, t_end = t_begin + seg_len < L ? t_begin + seg_len : L;
   const int64_t d0 = tile * DT;
   // recurrence mapping: adjacent lanes hold the two halves of a state pair
   const int pr = tid & 1;
@@ -249,6 +412,7 @@ __global__ void __launch_bounds__(FCfg<NS>::TH, FCfg<NS>::WAVES >= 8 ? 3 : 1) ma
     h[j] = (act && h0 && n < N) ? h0[(b * D + d) * N + n] : 0.0f;
     co[j] = (uint32_t)n * Du + (uint32_t)dl;
   }
+  compose_segments<NPT>(segs, 0, seg, 1, B, b, D, d, N, [&](int j) { return n0 + j; }, act, A2, h);
   const uint32_t slot_floats = Nu * Du;
   const float dp_o = oact ? Dp[d0 + od] : 0.0f;
 
@@ -292,11 +456,11 @@ __global__ void __launch_bounds__(FCfg<NS>::TH, FCfg<NS>::WAVES >= 8 ? 3 : 1) ma
   // FULL loads (no per-element guard): all TF steps in the sequence, all DT channels in range
   // and N == NS; workgroup-uniform
   const bool wg_full = d0 + DT <= D && N == NS;
-  if (L > 0) {
-    if (TF <= L && wg_full)
-      load_chunk(0u, Bool<true>());
+  if (t_begin < t_end) {
+    if (t_begin + TF <= L && wg_full)
+      load_chunk((uint32_t)t_begin, Bool<true>());
     else
-      load_chunk(0u, Bool<false>());
+      load_chunk((uint32_t)t_begin, Bool<false>());
   }
 
   float o_u[IT], o_z[IT];
@@ -322,7 +486,7 @@ __global__ void __launch_bounds__(FCfg<NS>::TH, FCfg<NS>::WAVES >= 8 ? 3 : 1) ma
     }
     // prefetch the next round while this one computes
     const uint32_t t1 = t0 + TF;
-    if ((int64_t)t1 < L) {
+    if ((int64_t)t1 < t_end) {
       if ((int64_t)t1 + TF <= L && wg_full)
         load_chunk(t1, Bool<true>());
       else
@@ -392,12 +556,12 @@ __global__ void __launch_bounds__(FCfg<NS>::TH, FCfg<NS>::WAVES >= 8 ? 3 : 1) ma
   // races ahead and the last ones finish alone; rotating the issue priority among the slots
   // every four rounds evens their progress and shortens the tail.
   const unsigned slot = blockIdx.x / cus;
-  for (int64_t t0 = 0; t0 < L; t0 += TF) {
+  for (int64_t t0 = t_begin; t0 < t_end; t0 += TF) {
     if (((t0 / TF) & 3) == 0) set_wave_priority((slot + (unsigned)(t0 / TF / 4)) % 3);
-    chunk((uint32_t)t0, (int)((L - t0) < TF ? (L - t0) : TF));
+    chunk((uint32_t)t0, (int)((t_end - t0) < TF ? (t_end - t0) : TF));
   }
   (void)NG;
-  if (act) {
+  if (act && t_end == L) {
 #pragma unroll
     for (int j = 0; j < NPT; ++j)
       if (n0 + j < N) h_last[(b * D + d) * N + n0 + j] = h[j];
@@ -441,7 +605,8 @@ __global__ void __launch_bounds__((BCfg<NS, DT_>::TH), (BCfg<NS, DT_>::OCC)) mam
     const float* __restrict__ h0, const float* __restrict__ saved, const TIO* __restrict__ gout,
     const float* __restrict__ ghlast, TIO* __restrict__ gdraw, TIO* __restrict__ gu, TIO* __restrict__ gz,
     float* __restrict__ gA_part, float* __restrict__ gDp_part, TIO* __restrict__ gBC_part, float* __restrict__ gh0,
-    int64_t B, int64_t L, int64_t D, int N, int64_t NC, unsigned cus) {
+    const float* __restrict__ segs, int64_t B, int64_t L, int64_t D, int N, int64_t NC, int64_t n_segs,
+    int64_t seg_chunks, unsigned cus) {
   using C = BCfg<NS, DT_>;
   constexpr int NPT = C::NPT, NG = C::NG, DT = C::DT, TH = C::TH, CHK = C::CHK, IT = C::IT;
   constexpr int W2 = C::W2, NBV = C::NBV, NSL = C::NSL, RPG = C::RPG;
@@ -457,6 +622,10 @@ __global__ void __launch_bounds__((BCfg<NS, DT_>::TH), (BCfg<NS, DT_>::OCC)) mam
   const int tid = threadIdx.x;
   int64_t tile, b;
   xcd_remap((D + DT - 1) / DT, tile, b);
+  // this workgroup's segment, chunks [c_begin, c_end) of its batch row (all of them when unsplit)
+  const int64_t part_row = b, seg = b / B;
+  b -= seg * B;
+  const int64_t c_begin = seg * seg_chunks, c_end = c_begin + seg_chunks < NC ? c_begin + seg_chunks : NC;
   const int64_t d0 = tile * DT;
   const int rw = tid >> 4, lk = tid & 15;
   const int ng = rw / RPG;
@@ -477,8 +646,9 @@ __global__ void __launch_bounds__((BCfg<NS, DT_>::TH), (BCfg<NS, DT_>::OCC)) mam
     A2[j] = Av[j] * kLog2e;
     G[j] = (v && ghlast) ? ghlast[(b * D + d) * N + n] : 0.0f;
     gA[j] = 0.0f;
-    lam_next[j] = 1.0f;  // no step after the last one
+    lam_next[j] = 1.0f;  // no step after the last one; a segment's G starts as lam_{t+1} G_{t+1}
   }
+  compose_segments<NPT>(segs, n_segs - 1, seg, -1, B, b, D, d, N, [&](int j) { return j * NG + ng; }, act, A2, G);
   float gdp = 0.0f;
 
   // Row streams through buffer resources (see make_rsrc): a per-lane byte offset fixed for the
@@ -601,9 +771,9 @@ __global__ void __launch_bounds__((BCfg<NS, DT_>::TH), (BCfg<NS, DT_>::OCC)) mam
     for (int j = 0; j < NPT; ++j) hst[j] = r_hs[j];
   };
 
-  if (NC > 0) {
-    load_chunk(NC - 1);
-    prepare(NC - 1);
+  if (c_end > c_begin) {
+    load_chunk(c_end - 1);
+    prepare(c_end - 1);
   }
   __syncthreads();
 
@@ -611,14 +781,14 @@ __global__ void __launch_bounds__((BCfg<NS, DT_>::TH), (BCfg<NS, DT_>::OCC)) mam
   // The forward's issue-priority rotation among the workgroups sharing a CU (every 16 chunks =
   // 128 steps): without it the oldest workgroup races ahead and the last one finishes alone.
   const unsigned slot = blockIdx.x / cus;
-  for (int64_t c = NC - 1; c >= 0; --c) {
-    const int64_t r = NC - 1 - c;
+  for (int64_t c = c_end - 1; c >= c_begin; --c) {
+    const int64_t r = c_end - 1 - c;
     if (C::OCC > 1 && (r & 15) == 0) set_wave_priority((slot + (unsigned)(r / 16)) % C::OCC);
     const uint32_t t0 = (uint32_t)(c * CHK);
     const int wb = (int)(c & 1);
     // the previous chunk's inputs, consumed at the end of this iteration (D): loads issued and
     // used within one iteration, so no pending load is carried around the loop
-    if (c > 0) load_chunk(c - 1);
+    if (c > c_begin) load_chunk(c - 1);
 
     // A: recompute this chunk's states into registers: lam_t, lam_t h_{t-1} and h_t (the chunk's
     // (delta, delta u) stay in registers for B: one LDS read per step instead of two)
@@ -715,17 +885,17 @@ __global__ void __launch_bounds__((BCfg<NS, DT_>::TH), (BCfg<NS, DT_>::OCC)) mam
                 ((uint32_t)ii * W2 + (uint32_t)col) * esz, t0 * (uint32_t)W2 * esz);
     }
     // D: the previous chunk's inputs (loaded during this one) into place
-    if (c > 0) prepare(c - 1);
+    if (c > c_begin) prepare(c - 1);
     __syncthreads();
   }
 
   if (act) {
 #pragma unroll
     for (int j = 0; j < NPT; ++j)
-      if (j * NG + ng < N) gA_part[(b * D + d) * N + j * NG + ng] = gA[j];
+      if (j * NG + ng < N) gA_part[(part_row * D + d) * N + j * NG + ng] = gA[j];
   }
   // gh0 = lam_0 G_0 (lam_next now holds lam_0; an empty sequence passes the state through)
-  if (gh0 && act) {
+  if (gh0 && act && seg == 0) {
 #pragma unroll
     for (int j = 0; j < NPT; ++j)
       if (j * NG + ng < N) gh0[(b * D + d) * N + j * NG + ng] = lam_next[j] * G[j];
@@ -738,7 +908,7 @@ __global__ void __launch_bounds__((BCfg<NS, DT_>::TH), (BCfg<NS, DT_>::OCC)) mam
   if (tid < DT && d0 + tid < D) {
     float s = 0.0f;
     for (int k = tid; k < TH; k += DT) s += red[k];
-    gDp_part[b * D + d0 + tid] = s;
+    gDp_part[part_row * D + d0 + tid] = s;
   }
 }
 
@@ -793,54 +963,117 @@ TSF_DEV void reduce_bc_vec(const TIO* __restrict__ part, TIO* __restrict__ gBt, 
   *reinterpret_cast<uint4*>(dst) = o;
 }
 
-// Sum [B, X] partials over the batch into [X] (gA with X = D*N, gDp with X = D), in batch order.
-TSF_DEV void reduce_batch(const float* __restrict__ part, float* __restrict__ dst, int64_t B, int64_t X,
-                          unsigned block) {
-  const int64_t i = block * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= X) return;
+// Sum [R, X] partials (one row per batch row and segment) into [X] (gA with X = D*N, gDp with
+// X = D). A block takes 64 outputs; each of its four waves adds 16 rows (a quarter of them beyond
+// 64 rows) in order, eight loads ahead, and the waves' sums are added in order: a fixed order, so
+// bitwise reproducible, and up to 16 rows the plain ordered sum.
+TSF_DEV void reduce_rows(const float* __restrict__ part, float* __restrict__ dst, int64_t R, int64_t X, unsigned block,
+                         float (&red)[4][64]) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t i = block * (int64_t)64 + lane;
+  const int64_t per = R > 64 ? (R + 3) / 4 : 16, r0 = w * per, r1 = r0 + per < R ? r0 + per : R;
   float s = 0.0f;
-  for (int64_t b = 0; b < B; ++b) s += part[b * X + i];
-  dst[i] = s;
+  if (i < X) {
+    int64_t r = r0;
+    for (; r + 8 <= r1; r += 8) {
+      float v[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] = part[(r + q) * X + i];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) s += v[q];
+    }
+    for (; r < r1; ++r) s += part[r * X + i];
+  }
+  red[w][lane] = s;
+  __syncthreads();
+  if (w == 0 && i < X) dst[i] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
 }
-__global__ void __launch_bounds__(256) mamba_reduce_batch(const float* __restrict__ part, float* __restrict__ dst,
-                                                          int64_t B, int64_t X) {
-  reduce_batch(part, dst, B, X, blockIdx.x);
+__global__ void __launch_bounds__(256) mamba_reduce_rows(const float* __restrict__ gA_part, float* __restrict__ gA,
+                                                         const float* __restrict__ gDp_part, float* __restrict__ gDp,
+                                                         int64_t R, int64_t XA, int64_t XD, unsigned nb_a) {
+  __shared__ float red[4][64];
+  if (blockIdx.x < nb_a)
+    reduce_rows(gA_part, gA, R, XA, blockIdx.x, red);
+  else
+    reduce_rows(gDp_part, gDp, R, XD, blockIdx.x - nb_a, red);
 }
 
 // The backward's three sums in one launch (each a few microseconds of work, so the launches
 // themselves were most of their time): blocks [0, nb_bc) the grad B_t / grad C_t sum over channel
-// tiles (reduce_bc_vec), the next nb_a blocks grad A over the batch, the rest grad Dp.
+// tiles (reduce_bc_vec), the next nb_a blocks grad A over its rows, the rest grad Dp.
 template <typename TIO>
 __global__ void __launch_bounds__(256) mamba_reduce_all(const TIO* __restrict__ part, TIO* __restrict__ gBt,
                                                         TIO* __restrict__ gCt, int64_t nT, int64_t BL, int NS,
                                                         unsigned nb_bc, const float* __restrict__ gA_part,
                                                         float* __restrict__ gA, const float* __restrict__ gDp_part,
-                                                        float* __restrict__ gDp, int64_t B, int64_t XA, int64_t XD,
+                                                        float* __restrict__ gDp, int64_t R, int64_t XA, int64_t XD,
                                                         unsigned nb_a) {
+  __shared__ float red[4][64];
   if (blockIdx.x < nb_bc) {
     reduce_bc_vec<TIO>(part, gBt, gCt, nT, BL, NS, blockIdx.x);
   } else if (blockIdx.x - nb_bc < nb_a) {
-    reduce_batch(gA_part, gA, B, XA, blockIdx.x - nb_bc);
+    reduce_rows(gA_part, gA, R, XA, blockIdx.x - nb_bc, red);
   } else {
-    reduce_batch(gDp_part, gDp, B, XD, blockIdx.x - nb_bc - nb_a);
+    reduce_rows(gDp_part, gDp, R, XD, blockIdx.x - nb_bc - nb_a, red);
   }
+}
+
+// Time segments of a walk: `segs` of `len` steps (a multiple of 32, so of every round and
+// checkpoint interval; the last one may be shorter).
+struct Split {
+  int64_t segs, len;
+};
+// Segments for a walk of `wgs` workgroups per segment of which `occ` fit a CU: as many as fill the
+// chip once, of at least 64 steps. Past that the maps cost more than the segments give (64 rows of
+// 1000 steps at D 256, two workgroups a CU: forward 91 us whole, 120 us in three segments).
+// Measured (fp32, N 16, whole -> split): 4 x 16384 x 256 inference 1120 -> 146 us and training
+// forward 1293 -> 184, backward 2970 -> 293 us; 8 x 2000 x 128 140 -> 31, 161 -> 32, 370 -> 54 us;
+// 64 x 512 x 128 44 -> 42, 48 -> 44, 107 -> 79 us.
+// Below 256 steps the second launch costs what the segments give. Rows of more than 1024 channels
+// are walked whole whatever the batch, so that such a row gives the same bits alone and in a batch.
+inline Split split_for(int64_t wgs, int64_t L, int64_t D, int occ) {
+  constexpr int64_t kStep = 32, kMin = 64;
+  int64_t segs = wgs > 0 ? (int64_t)device_cus() * occ / wgs : 1;
+  if (D > 1024 || segs < 2 || L < 4 * kMin) return {1, L};
+  int64_t len = ((L + segs - 1) / segs + kStep - 1) / kStep * kStep;
+  if (len < kMin) len = kMin;
+  segs = (L + len - 1) / len;
+  if (segs < 2) return {1, L};
+  return {segs, len};
+}
+template <int NS>
+Split fwd_split(int64_t B, int64_t L, int64_t D) {
+  using C = FCfg<NS>;
+  return split_for((D + C::DT - 1) / C::DT * B, L, D, C::OCC);
+}
+
+template <typename TIO, int NS, bool ADJ>
+void launch_segments(int64_t B, int64_t L, int64_t D, int64_t N, const Split& sp, const void* draw, const float* A,
+                     const void* V, const void* u, const void* z, float* segs, hipStream_t s) {
+  using C = FCfg<NS>;
+  hipLaunchKernelGGL((mamba_segment_kernel<TIO, NS, ADJ>),
+                     dim3((unsigned)((D + C::DT - 1) / C::DT * B * (sp.segs - 1))), dim3(C::TH), 0, s, (const TIO*)draw,
+                     A, (const TIO*)V, (const TIO*)u, (const TIO*)z, segs, B, L, D, (int)N, sp.len);
 }
 
 template <typename TIO, int NS>
 int launch_fwd(int64_t B, int64_t L, int64_t D, int64_t N, const void* draw, const float* A, const void* Bt,
                const void* Ct, const void* u, const void* z, const float* Dp, const float* h0, void* out,
-               float* h_last, float* chk, hipStream_t s) {
+               float* h_last, float* chk, float* segs, hipStream_t s) {
   using C = FCfg<NS>;
   const int64_t NC = (L + C::CHK - 1) / C::CHK;
-  dim3 grid((unsigned)((D + C::DT - 1) / C::DT * B));
+  // without a workspace for the segments' maps the rows are walked whole
+  const Split sp = segs ? fwd_split<NS>(B, L, D) : Split{1, L};
+  if (sp.segs > 1) launch_segments<TIO, NS, false>(B, L, D, N, sp, draw, A, Bt, u, nullptr, segs, s);
+  dim3 grid((unsigned)((D + C::DT - 1) / C::DT * B * sp.segs));
   if (chk)
     hipLaunchKernelGGL((mamba_fwd_kernel<TIO, NS, true>), grid, dim3(C::TH), 0, s, (const TIO*)draw, A,
-                       (const TIO*)Bt, (const TIO*)Ct, (const TIO*)u, (const TIO*)z, Dp, h0, (TIO*)out, h_last, chk, L,
-                       D, (int)N, NC, device_cus());
+                       (const TIO*)Bt, (const TIO*)Ct, (const TIO*)u, (const TIO*)z, Dp, h0, (TIO*)out, h_last, chk,
+                       segs, B, L, D, (int)N, NC, sp.len, device_cus());
   else
     hipLaunchKernelGGL((mamba_fwd_kernel<TIO, NS, false>), grid, dim3(C::TH), 0, s, (const TIO*)draw, A,
-                       (const TIO*)Bt, (const TIO*)Ct, (const TIO*)u, (const TIO*)z, Dp, h0, (TIO*)out, h_last, chk, L,
-                       D, (int)N, NC, device_cus());
+                       (const TIO*)Bt, (const TIO*)Ct, (const TIO*)u, (const TIO*)z, Dp, h0, (TIO*)out, h_last, chk,
+                       segs, B, L, D, (int)N, NC, sp.len, device_cus());
   return tsf_launch_status();
 }
 
@@ -857,8 +1090,15 @@ constexpr int bwd_dt() {
   return NS >= 32 ? 16 : kBwdDT;
 }
 
+template <int NS>
+Split bwd_split(int64_t B, int64_t L, int64_t D) {
+  constexpr int DT = bwd_dt<NS>();
+  return split_for((D + DT - 1) / DT * B, L, D, NS == 64 ? 2 : BCfg<NS, DT>::OCC);  // N 64: one wave per SIMD
+}
+
 // Backward workspace: grad-B/C partials [nT, B, L, 2*NS] in the I/O type (padded to 256 bytes),
-// then the fp32 per-row partials of gA [B, D, N] and gDp [B, D].
+// then the fp32 partials of gA [segs * B, D, N] and gDp [segs * B, D], then (when the rows are
+// split) the segments' maps.
 template <int NS>
 int64_t bwd_partial_bytes(int64_t B, int64_t L, int64_t D, int64_t esz) {
   const int64_t nT = (D + bwd_dt<NS>() - 1) / bwd_dt<NS>();
@@ -866,20 +1106,14 @@ int64_t bwd_partial_bytes(int64_t B, int64_t L, int64_t D, int64_t esz) {
 }
 template <int NS>
 int64_t bwd_workspace_bytes(int64_t B, int64_t L, int64_t D, int64_t N, int64_t esz) {
-  return bwd_partial_bytes<NS>(B, L, D, esz) + 4 * (B * D * N + B * D);
+  const Split sp = bwd_split<NS>(B, L, D);
+  const int64_t maps = sp.segs > 1 ? sp.segs * segment_floats(B, D, N) : 0;
+  return bwd_partial_bytes<NS>(B, L, D, esz) + 4 * (sp.segs * (B * D * N + B * D) + maps);
 }
-
-template <typename TIO, int NS, int DT>
-void launch_bwd_tile(int64_t B, int64_t L, int64_t D, int64_t N, int64_t NC, const void* draw, const float* A,
-                     const void* Bt, const void* Ct, const void* u, const void* z, const float* Dp, const float* h0,
-                     const float* chk, const void* gout, const float* ghlast, void* gdraw, void* gu, void* gz,
-                     float* gA_part, float* gDp_part, TIO* gBC_part, float* gh0, hipStream_t s) {
-  using C = BCfg<NS, DT>;
-  const int64_t nT = (D + DT - 1) / DT;
-  hipLaunchKernelGGL((mamba_bwd_kernel<TIO, NS, DT>), dim3((unsigned)(nT * B)), dim3(C::TH), 0, s,
-                     (const TIO*)draw, A, (const TIO*)Bt, (const TIO*)Ct, (const TIO*)u, (const TIO*)z, Dp, h0, chk,
-                     (const TIO*)gout, ghlast, (TIO*)gdraw, (TIO*)gu, (TIO*)gz, gA_part, gDp_part, gBC_part, gh0, B,
-                     L, D, (int)N, NC, device_cus());
+template <int NS>
+int64_t fwd_workspace_bytes(int64_t B, int64_t L, int64_t D, int64_t N) {
+  const Split sp = fwd_split<NS>(B, L, D);
+  return sp.segs > 1 ? 4 * sp.segs * segment_floats(B, D, N) : 0;
 }
 
 template <typename TIO, int NS>
@@ -887,23 +1121,31 @@ int launch_bwd(int64_t B, int64_t L, int64_t D, int64_t N, const void* draw, con
                const void* Ct, const void* u, const void* z, const float* Dp, const float* h0, const float* chk,
                const void* gout, const float* ghlast, void* gdraw, float* gA, void* gBt, void* gCt, void* gu, void* gz,
                float* gDp, float* gh0, void* workspace, hipStream_t s) {
-  using C = MCfg<NS>;
+  constexpr int DT = bwd_dt<NS>();
+  using C = BCfg<NS, DT>;
   const int64_t NC = (L + C::CHK - 1) / C::CHK;
-  const int64_t nT = (D + bwd_dt<NS>() - 1) / bwd_dt<NS>();
+  const int64_t nT = (D + DT - 1) / DT;
+  const Split sp = bwd_split<NS>(B, L, D);
+  const int64_t rows = sp.segs * B;
   TIO* gBC_part = static_cast<TIO*>(workspace);
   float* gA_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + bwd_partial_bytes<NS>(B, L, D, sizeof(TIO)));
-  float* gDp_part = gA_part + B * D * N;
-  if (B > 0 && D > 0)
-    launch_bwd_tile<TIO, NS, bwd_dt<NS>()>(B, L, D, N, NC, draw, A, Bt, Ct, u, z, Dp, h0, chk, gout, ghlast, gdraw, gu, gz,
-                                     gA_part, gDp_part, gBC_part, gh0, s);
+  float* gDp_part = gA_part + rows * D * N;
+  float* segs = gDp_part + rows * D;
+  if (B > 0 && D > 0) {
+    if (sp.segs > 1) launch_segments<TIO, NS, true>(B, L, D, N, sp, draw, A, Ct, gout, z, segs, s);
+    hipLaunchKernelGGL((mamba_bwd_kernel<TIO, NS, DT>), dim3((unsigned)(nT * rows)), dim3(C::TH), 0, s,
+                       (const TIO*)draw, A, (const TIO*)Bt, (const TIO*)Ct, (const TIO*)u, (const TIO*)z, Dp, h0, chk,
+                       (const TIO*)gout, ghlast, (TIO*)gdraw, (TIO*)gu, (TIO*)gz, gA_part, gDp_part, gBC_part, gh0,
+                       segs, B, L, D, (int)N, NC, sp.segs, (sp.len + C::CHK - 1) / C::CHK, device_cus());
+  }
   const int64_t BLN = B * L * N;
   constexpr int V = 16 / sizeof(TIO);
+  const unsigned nb_a = (unsigned)((D * N + 63) / 64), nb_d = (unsigned)((D + 63) / 64);
   if (BLN > 0 && N == NS && NS % V == 0) {
     const int64_t items = B * L * (2 * NS / V);
-    const unsigned nb_bc = (unsigned)((items + 255) / 256), nb_a = (unsigned)((D * N + 255) / 256),
-                   nb_d = (unsigned)((D + 255) / 256);
+    const unsigned nb_bc = (unsigned)((items + 255) / 256);
     hipLaunchKernelGGL((mamba_reduce_all<TIO>), dim3(nb_bc + nb_a + nb_d), dim3(256), 0, s, gBC_part, (TIO*)gBt,
-                       (TIO*)gCt, nT, B * L, NS, nb_bc, gA_part, gA, gDp_part, gDp, B, D * N, D, nb_a);
+                       (TIO*)gCt, nT, B * L, NS, nb_bc, gA_part, gA, gDp_part, gDp, rows, D * N, D, nb_a);
     return tsf_launch_status();
   }
   if (BLN > 0) {
@@ -911,9 +1153,8 @@ int launch_bwd(int64_t B, int64_t L, int64_t D, int64_t N, const void* draw, con
                        (TIO*)gBt, (TIO*)gCt, nT, B * L, (int)N, NS);
   }
   if (D > 0) {
-    hipLaunchKernelGGL(mamba_reduce_batch, dim3((unsigned)((D * N + 255) / 256)), dim3(256), 0, s, gA_part, gA, B,
-                       D * N);
-    hipLaunchKernelGGL(mamba_reduce_batch, dim3((unsigned)((D + 255) / 256)), dim3(256), 0, s, gDp_part, gDp, B, D);
+    hipLaunchKernelGGL(mamba_reduce_rows, dim3(nb_a + nb_d), dim3(256), 0, s, gA_part, gA, gDp_part, gDp, rows, D * N,
+                       D, nb_a);
   }
   return tsf_launch_status();
 }
@@ -937,14 +1178,14 @@ int launch_bwd(int64_t B, int64_t L, int64_t D, int64_t N, const void* draw, con
 template <int NS>
 int fwd_f32(int64_t B, int64_t L, int64_t D, int64_t N, const void* draw, const float* A, const void* Bt,
             const void* Ct, const void* u, const void* z, const float* Dp, const float* h0, void* out, float* h_last,
-            float* chk, hipStream_t s) {
-  return launch_fwd<float, NS>(B, L, D, N, draw, A, Bt, Ct, u, z, Dp, h0, out, h_last, chk, s);
+            float* chk, float* segs, hipStream_t s) {
+  return launch_fwd<float, NS>(B, L, D, N, draw, A, Bt, Ct, u, z, Dp, h0, out, h_last, chk, segs, s);
 }
 template <int NS>
 int fwd_bf16(int64_t B, int64_t L, int64_t D, int64_t N, const void* draw, const float* A, const void* Bt,
              const void* Ct, const void* u, const void* z, const float* Dp, const float* h0, void* out, float* h_last,
-             float* chk, hipStream_t s) {
-  return launch_fwd<bf16, NS>(B, L, D, N, draw, A, Bt, Ct, u, z, Dp, h0, out, h_last, chk, s);
+             float* chk, float* segs, hipStream_t s) {
+  return launch_fwd<bf16, NS>(B, L, D, N, draw, A, Bt, Ct, u, z, Dp, h0, out, h_last, chk, segs, s);
 }
 template <int NS>
 int bwd_f32(int64_t B, int64_t L, int64_t D, int64_t N, const void* draw, const float* A, const void* Bt,
@@ -1031,9 +1272,16 @@ int64_t tsfast_hip_mamba_workspace_bytes(int64_t B, int64_t L, int64_t D, int64_
   return workspace_bytes(ns, B, L, D, N);
 }
 
-int tsfast_hip_mamba_fwd(int64_t B, int64_t L, int64_t D, int64_t N, int io_dtype, const void* draw, const float* A,
-                         const void* Bt, const void* Ct, const void* u, const void* z, const float* Dp,
-                         const float* h0, void* out, float* h_last, float* chk, void* stream) {
+int64_t tsfast_hip_mamba_fwd_workspace_bytes(int64_t B, int64_t L, int64_t D, int64_t N) {
+  const int ns = ns_for(N);
+  if (ns == 0 || N < 1 || B < 0 || L < 0 || D < 0) return -1;
+  TSF_DISPATCH_NS(ns, fwd_workspace_bytes, B, L, D, N)
+}
+
+int tsfast_hip_mamba_fwd_ws(int64_t B, int64_t L, int64_t D, int64_t N, int io_dtype, const void* draw, const float* A,
+                            const void* Bt, const void* Ct, const void* u, const void* z, const float* Dp,
+                            const float* h0, void* out, float* h_last, float* chk, void* workspace,
+                            int64_t workspace_bytes, void* stream) {
   if (B < 0 || L < 0 || D < 0 || N < 1) return TSF_ERR_ARG;
   if ((D + 31) / 32 * B > INT32_MAX) return TSF_ERR_UNSUPPORTED;  // one-dimensional grid
   const int ns = ns_for(N);
@@ -1042,13 +1290,22 @@ int tsfast_hip_mamba_fwd(int64_t B, int64_t L, int64_t D, int64_t N, int io_dtyp
   if (!A || !Dp || !h_last) return TSF_ERR_ARG;
   if (L > 0 && (!draw || !Bt || !Ct || !u || !z || !out)) return TSF_ERR_ARG;
   if (!offsets_fit(L, D, N, chk_interval_for(ns))) return TSF_ERR_UNSUPPORTED;
+  if (workspace && workspace_bytes < tsfast_hip_mamba_fwd_workspace_bytes(B, L, D, N)) return TSF_ERR_WORKSPACE;
+  float* segs = static_cast<float*>(workspace);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (io_dtype == TSF_DTYPE_F32) {
-    TSF_DISPATCH_NS(ns, fwd_f32, B, L, D, N, draw, A, Bt, Ct, u, z, Dp, h0, out, h_last, chk, s)
+    TSF_DISPATCH_NS(ns, fwd_f32, B, L, D, N, draw, A, Bt, Ct, u, z, Dp, h0, out, h_last, chk, segs, s)
   } else if (io_dtype == TSF_DTYPE_BF16) {
-    TSF_DISPATCH_NS(ns, fwd_bf16, B, L, D, N, draw, A, Bt, Ct, u, z, Dp, h0, out, h_last, chk, s)
+    TSF_DISPATCH_NS(ns, fwd_bf16, B, L, D, N, draw, A, Bt, Ct, u, z, Dp, h0, out, h_last, chk, segs, s)
   }
   return TSF_ERR_ARG;
+}
+
+int tsfast_hip_mamba_fwd(int64_t B, int64_t L, int64_t D, int64_t N, int io_dtype, const void* draw, const float* A,
+                         const void* Bt, const void* Ct, const void* u, const void* z, const float* Dp,
+                         const float* h0, void* out, float* h_last, float* chk, void* stream) {
+  return tsfast_hip_mamba_fwd_ws(B, L, D, N, io_dtype, draw, A, Bt, Ct, u, z, Dp, h0, out, h_last, chk, nullptr, 0,
+                                 stream);
 }
 
 int tsfast_hip_mamba_bwd(int64_t B, int64_t L, int64_t D, int64_t N, int io_dtype, const void* draw, const float* A,

@@ -131,12 +131,14 @@ def _forward(draw, A, Bt, Ct, u, z, Dp, h0, store_chk: bool):
     chk = None
     if store_chk:
         chk = torch.empty(B, saved_floats(L, D, N, draw.dtype), device=draw.device, dtype=torch.float32)
+    nbytes = lib.tsfast_hip_mamba_fwd_workspace_bytes(B, L, D, N)  # 0 unless the rows are split in time
+    ws = _lib.workspace(nbytes, draw.device) if nbytes > 0 else None
     _lib.check(
-        lib.tsfast_hip_mamba_fwd(
-            B, L, D, N, _IO_DTYPES[draw.dtype], *map(_lib.ptr, (draw, A, Bt, Ct, u, z, Dp, h0, out, h_last, chk)),
-            _lib.stream_of(draw),
+        lib.tsfast_hip_mamba_fwd_ws(
+            B, L, D, N, _IO_DTYPES[draw.dtype], *map(_lib.ptr, (draw, A, Bt, Ct, u, z, Dp, h0, out, h_last, chk, ws)),
+            nbytes, _lib.stream_of(draw),
         ),
-        "tsfast_hip_mamba_fwd",
+        "tsfast_hip_mamba_fwd_ws",
     )
     return out, h_last, chk
 
