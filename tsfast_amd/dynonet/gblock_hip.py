@@ -162,6 +162,7 @@ def _(gy, g_xlast, u, b, a, u_tail, x0, saved):
 
 
 def _gblock_setup(ctx, inputs, output):
+    ctx.set_materialize_grads(False)  # no zero fill for outputs without a gradient (the saved state above all)
     u, b, a, u_tail, x0 = inputs
     _, _, saved = output
     ctx.has_tail, ctx.has_x0 = u_tail is not None, x0 is not None

@@ -258,6 +258,7 @@ def _(gout, ghlast, chk, draw, A, Bt, Ct, u, z, Dp, h0):
 
 
 def _scan_setup(ctx, inputs, output):
+    ctx.set_materialize_grads(False)  # no zero fill for outputs without a gradient (the saved state above all)
     draw, A, Bt, Ct, u, z, Dp, h0 = inputs
     ctx.save_for_backward(draw, A, Bt, Ct, u, z, Dp, h0, output[2])
 

@@ -212,6 +212,7 @@ def backward(gy, g_xlast, saved, u, W_re, W_im, lam, C_re, C_im, x0):
 
 
 def _scan_setup(ctx, inputs, output):
+    ctx.set_materialize_grads(False)  # no zero fill for outputs without a gradient (the saved state above all)
     u, W_re, W_im, lam, C_re, C_im, x0 = inputs
     ctx.save_for_backward(u, W_re, W_im, lam, C_re, C_im, x0, output[2])
 
@@ -363,12 +364,13 @@ def _(gy, g_xlast, x, u, W_re, W_im, lam, C_re, C_im, x0):
 
 
 def _wide_setup(ctx, inputs, output):
+    ctx.set_materialize_grads(False)  # no zero fill for outputs without a gradient (the saved state above all)
     u, W_re, W_im, lam, C_re, C_im, x0 = inputs
     ctx.save_for_backward(u, W_re, W_im, lam, C_re, C_im, x0, output[2])
 
 
 def _wide_backward_rule(ctx, gy, g_xlast, g_x):
-    # g_x is autograd's zero fill for the states output, which run() keeps for the backward only
+    # g_x belongs to the states output, which run() keeps for the backward only
     u, W_re, W_im, lam, C_re, C_im, x0, x = ctx.saved_tensors
     if gy is None:
         gy = u.new_zeros(u.shape[0], u.shape[1], C_re.shape[0])
