@@ -21,6 +21,7 @@ __all__ = [
 
 import contextvars
 import importlib
+import sys
 import warnings
 from contextlib import contextmanager
 from types import ModuleType
@@ -87,7 +88,7 @@ def resolve(
             continue
         if isinstance(target, str):
             try:
-                mod = importlib.import_module(target)
+                mod = sys.modules.get(target) or importlib.import_module(target)
             except Exception as e:
                 warn_fallback(
                     f"{op}.{name}",

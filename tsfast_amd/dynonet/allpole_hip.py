@@ -19,6 +19,7 @@ __all__ = ["supports", "run"]
 import torch
 
 from .. import _lib
+from ..ops import custom_op
 
 _MAX_NA = 16
 _LB_NA = 4  # highest order on the single-pass look-back path (allpole_core.h kLbNA)
@@ -50,7 +51,7 @@ def supports(a: torch.Tensor, w: torch.Tensor, y0: torch.Tensor | None) -> str |
     return None
 
 
-@torch.library.custom_op("tsfast_hip::dynonet_allpole", mutates_args=())
+@custom_op("tsfast_hip::dynonet_allpole")
 def _allpole_op(a: torch.Tensor, w: torch.Tensor, y0: torch.Tensor | None) -> torch.Tensor:
     lib = _lib.load()
     _lib.sync_deterministic()
@@ -79,7 +80,7 @@ def _(a, w, y0):
     return torch.empty_like(w)
 
 
-@torch.library.custom_op("tsfast_hip::dynonet_allpole_bwd", mutates_args=())
+@custom_op("tsfast_hip::dynonet_allpole_bwd")
 def _allpole_bwd_op(
     g: torch.Tensor, a: torch.Tensor, y: torch.Tensor, y0: torch.Tensor | None
 ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:

@@ -26,6 +26,7 @@ import torch.nn.functional as F
 
 from .. import blocked_scan
 from ..dispatch import resolve
+from ..ops import custom_op
 from . import allpole_hip, gblock_hip, linrec_hip
 
 _ALLPOLE_BACKENDS = {"hip": allpole_hip}
@@ -33,7 +34,7 @@ _GBLOCK_BACKENDS = {"hip": gblock_hip}
 _LINREC_BACKENDS = {"hip": linrec_hip}
 
 
-@torch.library.custom_op("tsfast_hip::linear_recurrence", mutates_args=())
+@custom_op("tsfast_hip::linear_recurrence")
 def _linear_recurrence_op(A: torch.Tensor, v: torch.Tensor, x0: torch.Tensor | None) -> torch.Tensor:
     return blocked_scan.scan_matrix(A, v, x0)
 
@@ -43,7 +44,7 @@ def _(A, v, x0):
     return torch.empty_like(v)
 
 
-@torch.library.custom_op("tsfast_hip::linear_recurrence_bwd", mutates_args=())
+@custom_op("tsfast_hip::linear_recurrence_bwd")
 def _linear_recurrence_bwd_op(
     g: torch.Tensor, A: torch.Tensor, out: torch.Tensor, x0: torch.Tensor | None
 ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:

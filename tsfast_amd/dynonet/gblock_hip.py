@@ -27,6 +27,7 @@ __all__ = ["supports", "run"]
 import torch
 
 from .. import _lib
+from ..ops import custom_op
 
 _MAX_NA = 4  # orders of the fused kernels
 _MAX_NB = 8  # taps the operator fuses (the kernels take up to 16; 9..16 ran 1.5x slower than staged)
@@ -84,7 +85,7 @@ def _screen(u, b, a, u_tail, x0):
         _lib.require(t, name, (torch.float32,), dev)
 
 
-@torch.library.custom_op("tsfast_hip::dynonet_gblock", mutates_args=())
+@custom_op("tsfast_hip::dynonet_gblock")
 def _gblock_op(
     u: torch.Tensor, b: torch.Tensor, a: torch.Tensor, u_tail: torch.Tensor | None, x0: torch.Tensor | None
 ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -122,7 +123,7 @@ def _(u, b, a, u_tail, x0):
     return u.new_empty(B, L, O), u.new_empty(B, I * O, na), u.new_empty(max(n_saved, 1), dtype=torch.float64)
 
 
-@torch.library.custom_op("tsfast_hip::dynonet_gblock_bwd", mutates_args=())
+@custom_op("tsfast_hip::dynonet_gblock_bwd")
 def _gblock_bwd_op(
     gy: torch.Tensor, g_xlast: torch.Tensor | None, u: torch.Tensor, b: torch.Tensor, a: torch.Tensor,
     u_tail: torch.Tensor | None, x0: torch.Tensor | None, saved: torch.Tensor,
@@ -194,7 +195,7 @@ def _fused(na: int, nb: int) -> bool:
 
 
 # ------------------------------------------------------------------------------ staged path
-@torch.library.custom_op("tsfast_hip::dynonet_fir", mutates_args=())
+@custom_op("tsfast_hip::dynonet_fir")
 def _fir_op(u: torch.Tensor, b: torch.Tensor, u_tail: torch.Tensor | None) -> torch.Tensor:
     lib = _lib.load()
     u, b = u.contiguous(), b.contiguous()
@@ -218,7 +219,7 @@ def _(u, b, u_tail):
     return u.new_empty(B, I * b.shape[0], L)
 
 
-@torch.library.custom_op("tsfast_hip::dynonet_fir_bwd", mutates_args=())
+@custom_op("tsfast_hip::dynonet_fir_bwd")
 def _fir_bwd_op(
     gw: torch.Tensor, u: torch.Tensor, b: torch.Tensor, u_tail: torch.Tensor | None
 ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:

@@ -23,6 +23,7 @@ import math
 import torch
 
 from .. import _lib
+from ..ops import custom_op
 
 _MAX_N = 16
 _MAX_WIDE_L = 65535 * 256  # two-pass path (n > 4): chunks of 256 steps, one grid row each
@@ -58,7 +59,7 @@ def _workspace(lib, lanes, L, n, device):
     return _lib.workspace(nbytes, device), nbytes
 
 
-@torch.library.custom_op("tsfast_hip::linear_recurrence_hip", mutates_args=())
+@custom_op("tsfast_hip::linear_recurrence_hip")
 def _linrec_op(A: torch.Tensor, v: torch.Tensor, x0: torch.Tensor | None) -> torch.Tensor:
     lib = _lib.load()
     _lib.sync_deterministic()
@@ -85,7 +86,7 @@ def _(A, v, x0):
     return torch.empty_like(v)
 
 
-@torch.library.custom_op("tsfast_hip::linear_recurrence_hip_bwd", mutates_args=())
+@custom_op("tsfast_hip::linear_recurrence_hip_bwd")
 def _linrec_bwd_op(
     g: torch.Tensor, A: torch.Tensor, out: torch.Tensor, x0: torch.Tensor | None
 ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:

@@ -20,6 +20,7 @@ __all__ = ["supports", "run"]
 import torch
 
 from .. import _lib
+from ..ops import custom_op
 
 _IO_DTYPES = {torch.float32: _lib.TSF_DTYPE_F32, torch.bfloat16: _lib.TSF_DTYPE_BF16}
 _PARAM_DTYPES = (torch.float32, torch.bfloat16)
@@ -81,7 +82,7 @@ def _screen(x, tail, weight, bias):
     _lib.require(bias, "bias", (torch.float32,), dev)
 
 
-@torch.library.custom_op("tsfast_hip::mamba_conv_silu", mutates_args=())
+@custom_op("tsfast_hip::mamba_conv_silu")
 def _conv_silu_op(x: torch.Tensor, tail: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
     lib = _lib.load()
     tail, weight = tail.contiguous(), weight.contiguous()
@@ -105,7 +106,7 @@ def _(x, tail, weight, bias):
     return torch.empty(x.shape, device=x.device, dtype=x.dtype)
 
 
-@torch.library.custom_op("tsfast_hip::mamba_conv_silu_bwd", mutates_args=())
+@custom_op("tsfast_hip::mamba_conv_silu_bwd")
 def _conv_silu_bwd_op(
     gy: torch.Tensor, x: torch.Tensor, tail: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None
 ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:

@@ -23,6 +23,7 @@ __all__ = ["supports", "run", "chk_interval", "saved_floats"]
 import torch
 
 from .. import _lib
+from ..ops import custom_op
 
 _IO_DTYPES = {torch.float32: _lib.TSF_DTYPE_F32, torch.bfloat16: _lib.TSF_DTYPE_BF16}
 _MAX_N = 64
@@ -143,7 +144,7 @@ def _forward(draw, A, Bt, Ct, u, z, Dp, h0, store_chk: bool):
     return out, h_last, chk
 
 
-@torch.library.custom_op("tsfast_hip::mamba_scan", mutates_args=())
+@custom_op("tsfast_hip::mamba_scan")
 def _scan_op(
     draw: torch.Tensor,
     A: torch.Tensor,
@@ -159,7 +160,7 @@ def _scan_op(
     return out, h_last
 
 
-@torch.library.custom_op("tsfast_hip::mamba_scan_train", mutates_args=())
+@custom_op("tsfast_hip::mamba_scan_train")
 def _scan_train_op(
     draw: torch.Tensor,
     A: torch.Tensor,
@@ -195,7 +196,7 @@ def _(draw, A, Bt, Ct, u, z, Dp, h0):
     return _fake_outs(draw, A, with_chk=True)
 
 
-@torch.library.custom_op("tsfast_hip::mamba_scan_bwd", mutates_args=())
+@custom_op("tsfast_hip::mamba_scan_bwd")
 def _scan_bwd_op(
     gout: torch.Tensor,
     ghlast: torch.Tensor | None,

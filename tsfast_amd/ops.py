@@ -1,0 +1,101 @@
+"""Custom ops that cost a plain eager call no dispatcher round trip.
+
+``custom_op`` registers an op as ``torch.library.custom_op`` does. A call that nothing but the
+kernels would see (dense GPU tensors; no trace, transform, mode, forward-mode level or profiler)
+runs the op's function directly, under an ``autograd.Function`` with the op's own rules when a
+gradient is wanted. Every other call goes through the registered op. The dispatcher's Python layers
+bound small passes: a truncated-BPTT chunk (8 x 4096 x 128, forward and backward) took 263 us
+through them and takes 192 us without, a Mamba window (64 x 512 x 128) 239 and 201 us, a forward
+call without gradients 49 and 44 us.
+"""
+
+from __future__ import annotations
+
+__all__ = ["custom_op"]
+
+import torch
+from torch.autograd import forward_ad
+
+_C = torch._C
+# dispatch keys of a plain dense GPU tensor (made in and outside inference mode); any other key
+# (conjugate or negative views, subclasses, functional, sparse, nested, batched ..) needs the dispatcher
+_plain_keys: set[int] = set()
+
+
+def _plain(t: torch.Tensor) -> bool:
+    if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
+        return False
+    keys = _C._dispatch_keys(t).raw_repr()
+    if keys in _plain_keys:
+        return True
+    if not _plain_keys and t.is_cuda:
+        _plain_keys.add(_C._dispatch_keys(torch.empty(0, device=t.device)).raw_repr())
+        with torch.inference_mode():
+            _plain_keys.add(_C._dispatch_keys(torch.empty(0, device=t.device)).raw_repr())
+        return keys in _plain_keys
+    return False
+
+
+def _unobserved() -> bool:
+    """No trace, transform, mode or profiler would see an op called now."""
+    return (
+        _C._len_torch_dispatch_stack() == 0
+        and not _C._is_torch_function_mode_enabled()
+        and _C._functorch.peek_interpreter_stack() is None
+        and _C._get_tracing_state() is None
+        and forward_ad._current_level < 0
+        and not _C._autograd._profiler_enabled()
+    )
+
+
+class _Op:
+    """A registered custom op and its direct form; see ``custom_op``."""
+
+    def __init__(self, name: str, fn):
+        self._fn = fn
+        self._def = torch.library.custom_op(name, fn, mutates_args=())
+        ns, op = name.split("::")
+        self._op = getattr(getattr(torch.ops, ns), op).default
+        self._function = None
+        self.__doc__ = fn.__doc__
+
+    def register_fake(self, fn):
+        return self._def.register_fake(fn)
+
+    def register_autograd(self, backward, *, setup_context):
+        self._def.register_autograd(backward, setup_context=setup_context)
+        impl = self._fn
+
+        class Direct(torch.autograd.Function):
+            @staticmethod
+            def forward(ctx, *args):
+                out = impl(*args)
+                setup_context(ctx, args, out)
+                return out
+
+            @staticmethod
+            def backward(ctx, *grads):
+                return backward(ctx, *grads)
+
+        Direct.__name__ = Direct.__qualname__ = f"Direct_{impl.__name__}"
+        self._function = Direct
+
+    def __call__(self, *args):
+        if torch.compiler.is_compiling() or not _unobserved():
+            return self._op(*args)
+        wants_grad = False
+        for t in args:
+            if isinstance(t, torch.Tensor):
+                if not _plain(t):
+                    return self._op(*args)
+                wants_grad = wants_grad or t.requires_grad
+        if wants_grad and torch.is_grad_enabled():
+            # an op without rules (a backward's) says so itself when it is differentiated
+            return self._op(*args) if self._function is None else self._function.apply(*args)
+        return self._fn(*args)
+
+
+def custom_op(name: str):
+    """Decorator: register ``fn`` as the custom op ``name`` (no argument mutated) and return it in
+    the form described above, with ``register_fake`` and ``register_autograd``."""
+    return lambda fn: _Op(name, fn)

@@ -24,6 +24,7 @@ import torch
 import torch.nn.functional as F
 
 from .. import _lib
+from ..ops import custom_op
 from . import diagonal_hip
 
 _MAX_H, _MAX_N, _MAX_O = 32, 256, 32
@@ -108,7 +109,7 @@ def _dense(*ts):
     return [t.contiguous() if t is not None else None for t in ts]
 
 
-@torch.library.custom_op("tsfast_hip::projected_scan", mutates_args=())
+@custom_op("tsfast_hip::projected_scan")
 def _scan_op(
     u: torch.Tensor, W_re: torch.Tensor, W_im: torch.Tensor, lam: torch.Tensor, C_re: torch.Tensor,
     C_im: torch.Tensor, x0: torch.Tensor | None,
@@ -117,7 +118,7 @@ def _scan_op(
     return y, x_last
 
 
-@torch.library.custom_op("tsfast_hip::projected_scan_train", mutates_args=())
+@custom_op("tsfast_hip::projected_scan_train")
 def _scan_train_op(
     u: torch.Tensor, W_re: torch.Tensor, W_im: torch.Tensor, lam: torch.Tensor, C_re: torch.Tensor,
     C_im: torch.Tensor, x0: torch.Tensor | None,
@@ -156,7 +157,7 @@ def _deterministic_bwd(gy, g_xlast, u, W_re, W_im, lam, C_re, C_im, x0):
     return _wide_backward(gy, g_xlast, _wide_states(u, W_re, W_im, lam, x0), u, W_re, W_im, lam, C_re, C_im, x0)
 
 
-@torch.library.custom_op("tsfast_hip::projected_scan_bwd", mutates_args=())
+@custom_op("tsfast_hip::projected_scan_bwd")
 def _scan_bwd_op(
     gy: torch.Tensor, g_xlast: torch.Tensor | None, saved: torch.Tensor, u: torch.Tensor, W_re: torch.Tensor,
     W_im: torch.Tensor, lam: torch.Tensor, C_re: torch.Tensor, C_im: torch.Tensor, x0: torch.Tensor | None,
@@ -319,7 +320,7 @@ def _wide_backward(gy, g_xlast, x, u, W_re, W_im, lam, C_re, C_im, x0):
             g_x0 if x0 is not None else lam.new_empty(0))
 
 
-@torch.library.custom_op("tsfast_hip::projected_scan_wide", mutates_args=())
+@custom_op("tsfast_hip::projected_scan_wide")
 def _wide_op(
     u: torch.Tensor, W_re: torch.Tensor, W_im: torch.Tensor, lam: torch.Tensor, C_re: torch.Tensor,
     C_im: torch.Tensor, x0: torch.Tensor | None,
@@ -328,7 +329,7 @@ def _wide_op(
     return y, x_last
 
 
-@torch.library.custom_op("tsfast_hip::projected_scan_wide_train", mutates_args=())
+@custom_op("tsfast_hip::projected_scan_wide_train")
 def _wide_train_op(
     u: torch.Tensor, W_re: torch.Tensor, W_im: torch.Tensor, lam: torch.Tensor, C_re: torch.Tensor,
     C_im: torch.Tensor, x0: torch.Tensor | None,
@@ -336,7 +337,7 @@ def _wide_train_op(
     return _wide_forward(*_dense(u, W_re, W_im, lam, C_re, C_im, x0))
 
 
-@torch.library.custom_op("tsfast_hip::projected_scan_wide_bwd", mutates_args=())
+@custom_op("tsfast_hip::projected_scan_wide_bwd")
 def _wide_bwd_op(
     gy: torch.Tensor, g_xlast: torch.Tensor | None, x: torch.Tensor, u: torch.Tensor, W_re: torch.Tensor,
     W_im: torch.Tensor, lam: torch.Tensor, C_re: torch.Tensor, C_im: torch.Tensor, x0: torch.Tensor | None,
