@@ -191,3 +191,20 @@ def test_linrec_wide_misaligned_rows(gpu, n):
     gA, gv, gx0 = O.linrec_backward(_np(gx), _np(A), want, _np(x0))
     assert O.rel_err(_np(ts[0].grad), gA) < TOL and O.rel_err(_np(ts[1].grad), gv) < TOL
     assert O.rel_err(_np(ts[2].grad), gx0) < TOL
+
+
+@pytest.mark.parametrize("n", [5, 6, 7, 8])
+@pytest.mark.parametrize("L", [524, 525, 526, 2560])
+def test_linrec_wide_row_stores(gpu, n, L):
+    """The re-runs' float4 row stores (rows of a multiple of four floats) and the per-float ones, with
+    a partial last sub-block, a partial wave of lanes, and ten chunks of carry (two prefetch groups)."""
+    M = 45
+    A, v, x0, gx = _make(M, L, n, seed=n + L)
+    ts = [A.to(gpu).requires_grad_(), v.to(gpu).requires_grad_(), x0.to(gpu).requires_grad_()]
+    x = linrec_hip.run(*ts)
+    x.backward(gx.to(gpu))
+    want = O.linrec_forward(_np(A), _np(v), _np(x0))
+    gA, gv, gx0 = O.linrec_backward(_np(gx), _np(A), want, _np(x0))
+    assert O.rel_err(_np(x), want) < TOL
+    for t, w in zip(ts, (gA, gv, gx0)):
+        assert O.rel_err(_np(t.grad), w) < TOL

@@ -563,6 +563,10 @@ int bwd_impl(int64_t lanes, int64_t L, const float* g, const float* A, const flo
 //             chunk re-run backwards, writing grad_v and its grad_A partial; linrec_finish adds the
 //             partials up in chunk order.
 // A stays fp32 in registers (exact in fp64 on use); state, carries and partials are fp64.
+// Chunks are long: the powers of a matrix far from normal grow before they decay (companion matrices
+// of clustered poles by 1e8 and more), and composing chunks that end inside the growth loses those
+// digits of the carried state (order 8, poles in 0.7 .. 0.97, against long double: 9e-6 with 256
+// steps a chunk, 8e-4 with 64).
 constexpr int kWideT = 256;
 constexpr int kWidePf = 4;  // steps fetched ahead by the chunk kernels
 constexpr int kWideThreads = 256;
@@ -587,40 +591,6 @@ TSF_DEV void ld_step(float (&d)[NS], const float* __restrict__ p) {
 #pragma unroll
     for (int i = 0; i < NS; ++i) d[i] = p[i];
   }
-}
-
-// M = P^e per lane, P = A or A^T, one thread per (lane, column c): column c is P applied e times
-// to the unit vector e_c in fp64 (step-by-step, as linrec_transfer, for the same accuracy reason).
-template <int NS>
-__global__ void __launch_bounds__(64) lw_power(const float* __restrict__ A, double* __restrict__ M, int64_t lanes,
-                                                int e, int transpose) {
-  const int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (idx >= lanes * NS) return;
-  const int64_t lane = idx / NS;
-  const int col = (int)(idx - lane * NS);
-  double P[NS][NS], x[NS];
-  const float* a = A + lane * NS * NS;
-#pragma unroll
-  for (int r = 0; r < NS; ++r) {
-    x[r] = r == col ? 1.0 : 0.0;
-#pragma unroll
-    for (int c = 0; c < NS; ++c) P[r][c] = (double)(transpose ? a[c * NS + r] : a[r * NS + c]);
-  }
-#pragma unroll 8
-  for (int step = 0; step < e; ++step) {
-    double y[NS];
-#pragma unroll
-    for (int r = 0; r < NS; ++r) {
-      double acc = 0.0;
-#pragma unroll
-      for (int c = 0; c < NS; ++c) acc = fma(P[r][c], x[c], acc);
-      y[r] = acc;
-    }
-#pragma unroll
-    for (int r = 0; r < NS; ++r) x[r] = y[r];
-  }
-#pragma unroll
-  for (int r = 0; r < NS; ++r) M[lane * NS * NS + r * NS + col] = x[r];
 }
 
 // The chunk kernels run two threads per lane (adjacent threads): thread h = threadIdx.x & 1 owns
@@ -708,7 +678,7 @@ struct HalfIdx {
   int64_t lane, c, t0, t1;
   bool live;
 };
-TSF_DEV HalfIdx half_idx(int64_t lanes, int64_t L, int NH) {
+TSF_DEV HalfIdx half_idx(int64_t lanes, int64_t L, int NH, unsigned row0 = 0) {
   HalfIdx q;
   q.h = threadIdx.x & 1;
   q.ll = threadIdx.x >> 1;
@@ -716,18 +686,57 @@ TSF_DEV HalfIdx half_idx(int64_t lanes, int64_t L, int NH) {
   q.par0 = (1 - q.h) * NH;
   q.lane = blockIdx.x * (int64_t)kWideLanes + q.ll;
   q.live = q.lane < lanes;
-  q.c = blockIdx.y;
+  q.c = blockIdx.y - row0;
   q.t0 = q.c * kWideT;
   q.t1 = (q.t0 + kWideT < L) ? q.t0 + kWideT : L;
   return q;
 }
 
-// Forward chunk ends from a zero state: e [nchunks][lanes][NS]
+// Column `col` of M = P^kWideT per lane (P = A or A^T, M [lanes][NS][NS] fp64), a pair of threads per
+// lane: P applied kWideT times to the unit vector, step by step as linrec_transfer and for the same
+// accuracy reason. The sum kernels run it in their first NS grid rows, beside the chunks: as a launch
+// of its own ahead of them (one thread per column) it took 37 us at 4096 lanes, n 8.
+template <int NS, bool TR>
+TSF_DEV void half_power(const float* __restrict__ A, double* __restrict__ M, int64_t lanes, int col) {
+  constexpr int NH = half_rows(NS);
+  const int h = threadIdx.x & 1;
+  const int64_t lane = blockIdx.x * (int64_t)kWideLanes + (threadIdx.x >> 1);
+  if (lane >= lanes) return;
+  float mo[NH][NH], mp[NH][NH];
+  half_matrix<NS, TR>(mo, mp, A + lane * NS * NS, h * NH, (1 - h) * NH);
+  double s[NH];
+  float zero[NH];
+#pragma unroll
+  for (int i = 0; i < NH; ++i) {
+    s[i] = h * NH + i == col ? 1.0 : 0.0;
+    zero[i] = 0.0f;
+  }
+#pragma unroll 2
+  for (int t = 0; t < kWideT; ++t) {
+    // keeps the matrix in fp32 registers: hoisted, its fp64 form takes twice as many
+#pragma unroll
+    for (int i = 0; i < NH; ++i)
+#pragma unroll
+      for (int j = 0; j < NH; ++j) asm volatile("" : "+v"(mo[i][j]), "+v"(mp[i][j]));
+    half_step<NH>(mo, mp, s, zero);
+  }
+#pragma unroll
+  for (int i = 0; i < NH; ++i)
+    if (h * NH + i < NS) M[(lane * NS + h * NH + i) * NS + col] = s[i];
+}
+
+// Forward chunk ends from a zero state: e [nchunks][lanes][NS]; the first `power_rows` grid
+// rows form M (half_power), the others take a chunk each
 template <int NS, int VEC>
 __global__ void __launch_bounds__(kWideThreads) lw_sum_fwd(const float* __restrict__ A, const float* __restrict__ v,
-                                                           double* __restrict__ e, int64_t lanes, int64_t L) {
+                                                           double* __restrict__ e, double* __restrict__ M,
+                                                           int64_t lanes, int64_t L, unsigned power_rows) {
   constexpr int NH = half_rows(NS), VH = half_vec<NS, VEC>();
-  const HalfIdx q = half_idx(lanes, L, NH);
+  if (blockIdx.y < power_rows) {
+    half_power<NS, false>(A, M, lanes, (int)blockIdx.y);
+    return;
+  }
+  const HalfIdx q = half_idx(lanes, L, NH, power_rows);
   if (!q.live) return;  // both threads of a pair
   float mo[NH][NH], mp[NH][NH];
   half_matrix<NS, false>(mo, mp, A + q.lane * NS * NS, q.own0, q.par0);
@@ -768,24 +777,49 @@ constexpr int wide_out_sb() {
 // A re-run's outputs of sub-block tb (cnt steps) leave through LDS: each thread left its rows of
 // every step in its lane's LDS row, and each wave now writes its 32 lanes' row segments with
 // whole-segment (coalesced) stores, one lane at a time, so HBM sees full lines.
-template <int NS, int SB>
-TSF_DEV void half_write_segments(float* __restrict__ dst, const float (*s_o)[SB * NS + 1], int64_t lanes, int64_t L,
-                                 int64_t tb, int cnt) {
+// VEC floats a thread, so 64 / (SB * NS / VEC) lanes a store: with one float a thread the stores' own
+// instructions cost as much as the steps' arithmetic (n 8 at 100 lanes x 4000 steps: forward re-run
+// 93 -> 53 us, adjoint 126 -> 87 us with float4).
+template <int NS, int SB, int VEC>
+TSF_DEV void half_write_vec(float* __restrict__ dst, const float (*s_o)[SB * NS + 1], int64_t lanes, int64_t L,
+                            int64_t tb, int cnt) {
+  constexpr int TPL = SB * NS / VEC, LPI = 64 / TPL;  // threads per lane, lanes per store
+  static_assert(SB * NS % VEC == 0, "a sub-block is whole vectors");
   const int wl = threadIdx.x & 63, wlane0 = (threadIdx.x & ~63) >> 1;
   const int64_t l0 = blockIdx.x * (int64_t)kWideLanes;
-  const int wseg = cnt * NS;
+  const int sub = LPI == 1 ? 0 : wl / TPL, off = (LPI == 1 ? wl : wl % TPL) * VEC;
+  const bool on = sub < LPI && off < cnt * NS;
 #pragma unroll 8
-  for (int l = 0; l < 32; ++l) {
+  for (int lb = 0; lb < 32; lb += LPI) {
+    const int l = lb + sub;
     const int64_t ln = l0 + wlane0 + l;
-    if (ln < lanes && wl < wseg) dst[(ln * L + tb) * NS + wl] = s_o[wlane0 + l][wl];
+    if (on && l < 32 && ln < lanes) {
+      float* p = dst + (ln * L + tb) * NS + off;
+      const float* q = &s_o[wlane0 + l][off];
+      if constexpr (VEC == 4)
+        *reinterpret_cast<float4*>(p) = make_float4(q[0], q[1], q[2], q[3]);
+      else
+        *p = *q;
+    }
   }
+}
+// float4 stores for a whole sub-block when every lane's row allows them (ov == 4, from the host:
+// sub-blocks start whole vectors into a row, so only the rows' own starts count), else by floats.
+template <int NS, int SB>
+TSF_DEV void half_write_segments(float* __restrict__ dst, const float (*s_o)[SB * NS + 1], int64_t lanes, int64_t L,
+                                 int64_t tb, int cnt, int ov) {
+  static_assert(SB * NS % 4 == 0 && kWideT * NS % 4 == 0, "sub-blocks and chunks are whole float4s");
+  if (cnt == SB && ov == 4)
+    half_write_vec<NS, SB, 4>(dst, s_o, lanes, L, tb, cnt);
+  else
+    half_write_vec<NS, SB, 1>(dst, s_o, lanes, L, tb, cnt);
 }
 
 // Every chunk re-run from its entering state, writing x.
 template <int NS, int VEC>
 __global__ void __launch_bounds__(kWideThreads) lw_apply_fwd(const float* __restrict__ A, const float* __restrict__ v,
                                                              const double* __restrict__ carry, float* __restrict__ x,
-                                                             int64_t lanes, int64_t L) {
+                                                             int64_t lanes, int64_t L, int ov) {
   constexpr int NH = half_rows(NS), VH = half_vec<NS, VEC>();
   constexpr int SB = wide_out_sb<NS>();
   __shared__ float s_o[kWideLanes][SB * NS + 1];
@@ -836,17 +870,22 @@ __global__ void __launch_bounds__(kWideThreads) lw_apply_fwd(const float* __rest
       }
     }
     __syncthreads();
-    half_write_segments<NS, SB>(x, s_o, lanes, L, tb, cnt);
+    half_write_segments<NS, SB>(x, s_o, lanes, L, tb, cnt, ov);
     __syncthreads();
   }
 }
 
-// Adjoint chunk starts from a zero right-end state: f [nchunks][lanes][NS]
+// Adjoint chunk starts from a zero right-end state: f [nchunks][lanes][NS]; grid rows as lw_sum_fwd
 template <int NS, int VEC>
 __global__ void __launch_bounds__(kWideThreads) lw_sum_bwd(const float* __restrict__ A, const float* __restrict__ g,
-                                                           double* __restrict__ f, int64_t lanes, int64_t L) {
+                                                           double* __restrict__ f, double* __restrict__ M,
+                                                           int64_t lanes, int64_t L, unsigned power_rows) {
   constexpr int NH = half_rows(NS), VH = half_vec<NS, VEC>();
-  const HalfIdx q = half_idx(lanes, L, NH);
+  if (blockIdx.y < power_rows) {
+    half_power<NS, true>(A, M, lanes, (int)blockIdx.y);
+    return;
+  }
+  const HalfIdx q = half_idx(lanes, L, NH, power_rows);
   if (!q.live) return;  // both threads of a pair
   float mo[NH][NH], mp[NH][NH];
   half_matrix<NS, true>(mo, mp, A + q.lane * NS * NS, q.own0, q.par0);
@@ -877,60 +916,84 @@ __global__ void __launch_bounds__(kWideThreads) lw_sum_bwd(const float* __restri
     if (q.own0 + i < NS) f[(q.c * lanes + q.lane) * NS + q.own0 + i] = G[i];
 }
 
-// Entering state of every chunk: carry[c] = M carry[c-1] + e[c-1], carry[0] = x0 (or 0)
-template <int NS>
-__global__ void __launch_bounds__(64) lw_carry_fwd(const double* __restrict__ M, const float* __restrict__ x0,
-                                                    const double* __restrict__ e, double* __restrict__ carry,
-                                                    int64_t lanes, int64_t nchunks) {
-  const int64_t lane = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (lane >= lanes) return;
-  double m[NS][NS], s[NS];
-  for (int r = 0; r < NS; ++r) {
-    for (int c = 0; c < NS; ++c) m[r][c] = M[lane * NS * NS + r * NS + c];
-    s[r] = x0 ? (double)x0[lane * NS + r] : 0.0;
-  }
-  for (int64_t c = 0; c < nchunks; ++c) {
-    double t[NS];
-    for (int r = 0; r < NS; ++r) {
-      carry[(c * lanes + lane) * NS + r] = s[r];
-      double acc = e[(c * lanes + lane) * NS + r];
-      for (int j = 0; j < NS; ++j) acc = fma(m[r][j], s[j], acc);
-      t[r] = acc;
+// Entering state of every chunk, a pair of threads per lane (each half the rows, as the chunk
+// kernels). Forward: carry[c] = M carry[c-1] + e[c-1], carry[0] = x0 (or 0). ADJ: the adjoint
+// entering every chunk from the right, carry[c] = G at the first step of chunk c + 1 (zero for the
+// last chunk), carry[c-1] = e[c] + M carry[c]; then grad_x0 = A^T G_0 with G_0 = e[0] + M carry[0].
+// The chain is one small product per chunk; the chunk ends are loaded kCarryPf chunks ahead (one
+// thread per lane with each chunk's load on the chain took 0.67 us a chunk, now 0.2).
+constexpr int kCarryPf = 8;
+template <int NS, bool ADJ>
+__global__ void __launch_bounds__(64) lw_carry(const float* __restrict__ A, const double* __restrict__ M,
+                                               const float* __restrict__ x0, const double* __restrict__ e,
+                                               double* __restrict__ carry, float* __restrict__ gx0, int64_t lanes,
+                                               int64_t nchunks) {
+  constexpr int NH = half_rows(NS);
+  const int h = threadIdx.x & 1, own0 = h * NH, par0 = (1 - h) * NH;
+  const int64_t lane = blockIdx.x * (int64_t)32 + (threadIdx.x >> 1);
+  if (lane >= lanes) return;  // both threads of a pair
+  double mo[NH][NH], mp[NH][NH], s[NH];
+  const double* m = M + lane * NS * NS;
+#pragma unroll
+  for (int j = 0; j < NH; ++j) {
+    const bool row = own0 + j < NS;
+#pragma unroll
+    for (int i = 0; i < NH; ++i) {
+      mo[j][i] = (row && own0 + i < NS) ? m[(own0 + j) * NS + own0 + i] : 0.0;
+      mp[j][i] = (row && par0 + i < NS) ? m[(own0 + j) * NS + par0 + i] : 0.0;
     }
-    for (int r = 0; r < NS; ++r) s[r] = t[r];
+    s[j] = (!ADJ && x0 && row) ? (double)x0[lane * NS + own0 + j] : 0.0;
   }
-}
-
-
-// Adjoint entering every chunk from the right: rc[c] = G at the first step of chunk c + 1 (zero
-// for the last chunk), rc[c-1] = f[c] + M rc[c]; then grad_x0 = A^T G_0 with G_0 = f[0] + M rc[0].
-template <int NS>
-__global__ void __launch_bounds__(64) lw_carry_bwd(const float* __restrict__ A, const double* __restrict__ M,
-                                                    const double* __restrict__ f, double* __restrict__ rc,
-                                                    float* __restrict__ gx0, int64_t lanes, int64_t nchunks) {
-  const int64_t lane = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (lane >= lanes) return;
-  double m[NS][NS], R[NS];
-  for (int r = 0; r < NS; ++r) {
-    for (int c = 0; c < NS; ++c) m[r][c] = M[lane * NS * NS + r * NS + c];
-    R[r] = 0.0;
-  }
-  for (int64_t c = nchunks - 1; c >= 0; --c) {
-    double t[NS];
-    for (int r = 0; r < NS; ++r) {
-      rc[(c * lanes + lane) * NS + r] = R[r];
-      double acc = f[(c * lanes + lane) * NS + r];
-      for (int j = 0; j < NS; ++j) acc = fma(m[r][j], R[j], acc);
-      t[r] = acc;
+  auto at = [&](int64_t c) { return ((ADJ ? nchunks - 1 - c : c) * lanes + lane) * NS + own0; };
+  double d[kCarryPf][NH];
+  auto fetch = [&](int k, int64_t c) __attribute__((always_inline)) {
+    const double* p = e + at(c < nchunks ? c : nchunks - 1);
+#pragma unroll
+    for (int j = 0; j < NH; ++j) d[k][j] = p[own0 + j < NS ? j : 0];
+  };
+  auto step = [&](int k, int64_t c) __attribute__((always_inline)) {
+    double sp[NH], t[NH];
+    half_swap<NH>(sp, s);
+#pragma unroll
+    for (int j = 0; j < NH; ++j) {
+      if (own0 + j < NS) carry[at(c) + j] = s[j];
+      double acc = own0 + j < NS ? d[k][j] : 0.0;
+#pragma unroll
+      for (int i = 0; i < NH; ++i) acc = fma(mo[j][i], s[i], acc);
+#pragma unroll
+      for (int i = 0; i < NH; ++i) acc = fma(mp[j][i], sp[i], acc);
+      t[j] = acc;
     }
-    for (int r = 0; r < NS; ++r) R[r] = t[r];
+#pragma unroll
+    for (int j = 0; j < NH; ++j) s[j] = t[j];
+  };
+#pragma unroll
+  for (int k = 0; k < kCarryPf; ++k) fetch(k, k);
+  int64_t c = 0;
+  for (; c + kCarryPf <= nchunks; c += kCarryPf) {
+#pragma unroll
+    for (int k = 0; k < kCarryPf; ++k) {
+      step(k, c + k);
+      fetch(k, c + k + kCarryPf);
+    }
   }
-  if (gx0) {  // R now holds G_0; grad_x0 = A^T G_0
+#pragma unroll
+  for (int k = 0; k < kCarryPf - 1; ++k)
+    if (c + k < nchunks) step(k, c + k);
+  if (ADJ && gx0) {  // s now holds G_0; grad_x0 = A^T G_0
+    double sp[NH];
+    half_swap<NH>(sp, s);
     const float* a = A + lane * NS * NS;
-    for (int r = 0; r < NS; ++r) {
+#pragma unroll
+    for (int j = 0; j < NH; ++j) {
+      if (own0 + j >= NS) break;
       double acc = 0.0;
-      for (int j = 0; j < NS; ++j) acc = fma((double)a[j * NS + r], R[j], acc);
-      gx0[lane * NS + r] = (float)acc;
+#pragma unroll
+      for (int i = 0; i < NH; ++i) {
+        if (own0 + i < NS) acc = fma((double)a[(own0 + i) * NS + own0 + j], s[i], acc);
+        if (par0 + i < NS) acc = fma((double)a[(par0 + i) * NS + own0 + j], sp[i], acc);
+      }
+      gx0[lane * NS + own0 + j] = (float)acc;
     }
   }
 }
@@ -943,10 +1006,11 @@ template <int NS, int VEC>
 __global__ void __launch_bounds__(kWideThreads) lw_apply_bwd(const float* __restrict__ A, const float* __restrict__ g,
                                                              const float* __restrict__ out, const float* __restrict__ x0,
                                                              const double* __restrict__ rc, float* __restrict__ gv,
-                                                             double* __restrict__ part, int64_t lanes, int64_t L) {
+                                                             double* __restrict__ part, int64_t lanes, int64_t L,
+                                                             int ov) {
   constexpr int NH = half_rows(NS), VH = half_vec<NS, VEC>();
   constexpr int SB = wide_out_sb<NS>();
-  constexpr int kPfB = 2;  // steps fetched ahead; SB is a multiple of it (4 and 8 measured no faster)
+  constexpr int kPfB = 2;  // steps fetched ahead; SB is a multiple of it (4, 8 and a whole sub-block measured no faster)
   constexpr bool kMaskPad = NS == 7;  // ld_half's load form (measured, see there)
   static_assert(SB % kPfB == 0, "sub-blocks hold whole prefetch pairs");
   __shared__ float s_o[kWideLanes][SB * NS + 1];
@@ -977,9 +1041,9 @@ __global__ void __launch_bounds__(kWideThreads) lw_apply_bwd(const float* __rest
   if (q.live) {
     half_matrix<NS, true>(mo, mp, A + q.lane * NS * NS, q.own0, q.par0);
 #pragma unroll
-    for (int i = 0; i < kPfB; ++i) {
-      const int64_t t = t1 - 1 - i;
-      if (t >= t0) fetch((int)((t - t0) % kPfB), t);
+    for (int k = 0; k < kPfB; ++k) {  // slot k: the last step t of the chunk with (t - t0) % kPfB == k
+      const int64_t t = t1 - 1 - (t1 - 1 - t0 + kPfB - k) % kPfB;
+      if (t >= t0) fetch(k, t);
     }
   }
   const int64_t nsb = (t1 - t0 + SB - 1) / SB;
@@ -1038,7 +1102,7 @@ __global__ void __launch_bounds__(kWideThreads) lw_apply_bwd(const float* __rest
       }
     }
     __syncthreads();
-    half_write_segments<NS, SB>(gv, s_o, lanes, L, tb, cnt);
+    half_write_segments<NS, SB>(gv, s_o, lanes, L, tb, cnt, ov);
     __syncthreads();
   }
   if (q.live) {
@@ -1075,8 +1139,25 @@ LwPlan lw_plan(int64_t lanes, int64_t L, int64_t ns) {
 }
 
 inline bool lw_grid_fits(int64_t lanes, int64_t L) {
-  // one grid row per chunk; two threads per lane, at most 2^32 - 1 threads per grid row
+  // one grid row per chunk (and one for M); two threads per lane, at most 2^32 - 1 threads per grid row
   return (L + kWideT - 1) / kWideT <= 65535 && (lanes + kWideLanes - 1) / kWideLanes <= UINT32_MAX / kWideThreads;
+}
+
+// Floats per store that every lane's output row allows (rows start `row` floats apart).
+int wide_out_vec(const float* p, int64_t row) {
+  const uintptr_t a = reinterpret_cast<uintptr_t>(p);
+  return (a % 16 == 0 && row % 4 == 0) ? 4 : 1;
+}
+
+// A sum kernel's grid: NS rows for M, then a row per chunk; two launches where that is more than a
+// grid's 65535 rows.
+template <int NS, typename F>
+void sum_launch(F kernel, unsigned gx, int64_t nchunks, hipStream_t s, const float* A, const float* in, double* out,
+                double* M, int64_t lanes, int64_t L) {
+  const bool one = nchunks + NS <= 65535;
+  if (!one) hipLaunchKernelGGL(kernel, dim3(gx, NS), dim3(kWideThreads), 0, s, A, in, out, M, lanes, L, (unsigned)NS);
+  hipLaunchKernelGGL(kernel, dim3(gx, (unsigned)nchunks + (one ? NS : 0)), dim3(kWideThreads), 0, s, A, in, out, M,
+                     lanes, L, one ? (unsigned)NS : 0u);
 }
 
 template <int NS, int VEC>
@@ -1086,13 +1167,12 @@ int wide_fwd_impl(int64_t lanes, int64_t L, const float* A, const float* v, cons
   double* e = reinterpret_cast<double*>(ws + p.off_e);
   double* carry = reinterpret_cast<double*>(ws + p.off_carry);
   double* M = reinterpret_cast<double*>(ws + p.off_M);
-  const dim3 grid((unsigned)((lanes + kWideLanes - 1) / kWideLanes), (unsigned)p.nchunks);
-  const unsigned lb = (unsigned)((lanes + 63) / 64);
-  hipLaunchKernelGGL((lw_power<NS>), dim3((unsigned)((lanes * NS + 63) / 64)), dim3(64), 0, s, A, M, lanes, kWideT, 0);
-  hipLaunchKernelGGL((lw_sum_fwd<NS, VEC>), grid, dim3(kWideThreads), 0, s, A, v, e, lanes, L);
-  hipLaunchKernelGGL((lw_carry_fwd<NS>), dim3(lb), dim3(64), 0, s, (const double*)M, x0, (const double*)e, carry,
-                     lanes, p.nchunks);
-  hipLaunchKernelGGL((lw_apply_fwd<NS, VEC>), grid, dim3(kWideThreads), 0, s, A, v, (const double*)carry, x, lanes, L);
+  const unsigned gx = (unsigned)((lanes + kWideLanes - 1) / kWideLanes);
+  sum_launch<NS>(lw_sum_fwd<NS, VEC>, gx, p.nchunks, s, A, v, e, M, lanes, L);
+  hipLaunchKernelGGL((lw_carry<NS, false>), dim3((unsigned)((lanes + 31) / 32)), dim3(64), 0, s, A, (const double*)M, x0,
+                     (const double*)e, carry, (float*)nullptr, lanes, p.nchunks);
+  hipLaunchKernelGGL((lw_apply_fwd<NS, VEC>), dim3(gx, (unsigned)p.nchunks), dim3(kWideThreads), 0, s, A, v,
+                     (const double*)carry, x, lanes, L, wide_out_vec(x, L * NS));
   return tsf_launch_status();
 }
 
@@ -1109,14 +1189,12 @@ int wide_bwd_impl(int64_t lanes, int64_t L, const float* g, const float* A, cons
   double* rc = reinterpret_cast<double*>(ws + p.off_carry);
   double* M = reinterpret_cast<double*>(ws + p.off_M);
   double* part = reinterpret_cast<double*>(ws + p.off_part);
-  const dim3 grid((unsigned)((lanes + kWideLanes - 1) / kWideLanes), (unsigned)p.nchunks);
-  const unsigned lb = (unsigned)((lanes + 63) / 64);
-  hipLaunchKernelGGL((lw_power<NS>), dim3((unsigned)((lanes * NS + 63) / 64)), dim3(64), 0, s, A, M, lanes, kWideT, 1);
-  hipLaunchKernelGGL((lw_sum_bwd<NS, VEC>), grid, dim3(kWideThreads), 0, s, A, g, f, lanes, L);
-  hipLaunchKernelGGL((lw_carry_bwd<NS>), dim3(lb), dim3(64), 0, s, A, (const double*)M, (const double*)f, rc, gx0,
-                     lanes, p.nchunks);
-  hipLaunchKernelGGL((lw_apply_bwd<NS, VEC>), grid, dim3(kWideThreads), 0, s, A, g, out, x0, (const double*)rc, gv, part,
-                     lanes, L);
+  const unsigned gx = (unsigned)((lanes + kWideLanes - 1) / kWideLanes);
+  sum_launch<NS>(lw_sum_bwd<NS, VEC>, gx, p.nchunks, s, A, g, f, M, lanes, L);
+  hipLaunchKernelGGL((lw_carry<NS, true>), dim3((unsigned)((lanes + 31) / 32)), dim3(64), 0, s, A, (const double*)M,
+                     (const float*)nullptr, (const double*)f, rc, gx0, lanes, p.nchunks);
+  hipLaunchKernelGGL((lw_apply_bwd<NS, VEC>), dim3(gx, (unsigned)p.nchunks), dim3(kWideThreads), 0, s, A, g, out, x0,
+                     (const double*)rc, gv, part, lanes, L, wide_out_vec(gv, L * NS));
   hipLaunchKernelGGL(linrec_finish, dim3((unsigned)((lanes * NS * NS + 63) / 64)), dim3(1024), 0, s,
                      (const double*)part, gA, lanes * NS * NS, p.nchunks);
   return tsf_launch_status();
@@ -1198,7 +1276,7 @@ TSF_DEV void spread_row(double (&p)[kSpread], const float* __restrict__ A, int64
 }
 
 // M = P^e per lane, fp64 [lanes][n][n]: a workgroup per lane, group c runs column c (P applied e
-// times to the unit vector e_c, step by step as lw_power).
+// times to the unit vector e_c, step by step as half_power).
 __global__ void __launch_bounds__(256) lsp_power(const float* __restrict__ A, double* __restrict__ M, int64_t lanes,
                                                  int n, int e, int transpose) {
   const int64_t lane = blockIdx.x;
