@@ -193,3 +193,24 @@ def test_gblock_supports_reasons(gpu):
     b2, a2 = torch.randn(2, 3, 4, device=gpu), torch.randn(2, 3, 17, device=gpu)
     assert "order" in gblock_hip.supports(u[..., :2], b2[:, :2], a2[:, :2], None, None)
     assert "GPU-only" in gblock_hip.supports(u.cpu(), b.cpu(), a.cpu(), None, None)
+
+
+@pytest.mark.parametrize(
+    "B,L,I,O_,nb,na",
+    [(1, 2900, 1, 1, 3, 3),  # one lane group of one pair, 12 tiles of 8 chunks, a ragged last one
+     (3, 256, 2, 2, 2, 2),  # one whole tile
+     (3, 257, 2, 2, 5, 4),  # and one step of a second
+     (17, 2305, 8, 8, 4, 2)],  # 17 groups: the middle anchor spacing
+)
+def test_gblock_few_groups(gpu, B, L, I, O_, nb, na):
+    """Few lane groups: whole 8-chunk tiles and anchors several tiles apart, against the oracle."""
+    ins = _make(B, L, I, O_, nb, na, seed=L + O_)
+    u, b, a, ut, x0, gy, gxl = ins
+    leaves = [t.to(gpu).requires_grad_() for t in (u, b, a, ut, x0)]
+    y, x_last = gblock_hip.run(*leaves)
+    torch.autograd.backward([y, x_last], [gy.to(gpu), gxl.to(gpu)])
+    want_y, want_x, _ = O.gblock_forward(*map(_np, (u, b, a, ut, x0)))
+    gu, gut, gb, ga, gx0 = O.gblock_backward(*map(_np, (gy, gxl, u, b, a, ut, x0)))
+    assert O.rel_err(_np(y), want_y) < TOL and O.rel_err(_np(x_last), want_x) < TOL
+    for t, w in zip(leaves, (gu, gb, ga, gut, gx0)):
+        assert O.rel_err(_np(t.grad), w) < TOL

@@ -393,15 +393,13 @@ TSF_DEV void regs_to_chunk(const float (&xb)[kTileT], float* __restrict__ dst, i
   __builtin_amdgcn_wave_barrier();
 }
 
-// Tile plan of the single-pass path: K (chunks per tile) starts at kLbWaves and halves down to 2
-// while there are fewer than kApTileTarget tiles. Workspace: the tile counter, agg and inc
+// Tile plan of the single-pass path: kLbWaves chunks per tile (all of a shorter sequence's). Halving
+// them to reach one tile per CU, as few lanes once did, lengthens the chain of look-backs by more than
+// the extra workgroups shorten the tiles, at every size measured: all-pole order 3, 64 lanes x 16000
+// steps, forward / backward 222 / 233 us at 2 chunks a tile, 39 / 47 at 8; G-block 8 rows x 16000, one
+// pair, 371 / 483 and 46 / 77 us (with the anchors below). Workspace: the tile counter, agg and inc
 // [nsuper][lanes][NA] (reset before each scan), the grad_a partials [nsuper][lanes][NA], and
 // the transfer matrices Mc, Ms [lanes][NA][NA].
-#ifndef TSF_AP_TILE_TARGET
-#define TSF_AP_TILE_TARGET 256
-#endif
-constexpr int64_t kApTileTarget = TSF_AP_TILE_TARGET;
-
 struct LbPlan {
   int64_t groups = 0, nsuper = 0;
   int K = 1;
@@ -412,11 +410,8 @@ LbPlan lb_plan(int64_t lanes, int64_t L, int64_t na) {
   LbPlan p;
   p.groups = (lanes + kTile - 1) / kTile;
   if (L > 0) {
-    p.K = kLbWaves;
-    auto tiles = [&](int K) { return p.groups * ((L + (int64_t)kTileT * K - 1) / ((int64_t)kTileT * K)); };
-    while (p.K > 2 && tiles(p.K) < kApTileTarget) p.K /= 2;
     const int64_t chunks = (L + kTileT - 1) / kTileT;
-    if (p.K > chunks) p.K = (int)chunks;
+    p.K = chunks < kLbWaves ? (int)chunks : kLbWaves;
     p.nsuper = (L + (int64_t)kTileT * p.K - 1) / ((int64_t)kTileT * p.K);
   }
   const size_t f = 8, vecs = f * p.nsuper * lanes * na;

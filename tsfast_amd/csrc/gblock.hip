@@ -38,9 +38,15 @@ namespace {
 
 #include "allpole_core.h"
 
-// Deterministic-mode anchor spacing: every tile an anchor (a chained look-back), measured the
-// cheapest at config 4's channels (4.5% over the default mode, against 12% at spacing K).
-constexpr int kGbAnchorSpacing = 1;
+// Deterministic-mode anchor spacing by lane groups. With 64 groups side by side each group's chain of
+// tiles is short and every tile an anchor is cheapest (64 rows of 8 x 8 channels x 16384 steps:
+// backward 401 us, 456 at spacing 8). Few groups wait for their chains: 4 groups of 64 tiles took
+// 118 / 182 us forward / backward at spacing 1, 54 / 89 at 4 and 42 / 73 at 8; 24 groups 151 / 290,
+// 84 / 212 and 82 / 212; 40 groups 150 / 303, 114 / 303 and 117 / 307.
+inline int gb_anchor_spacing(int64_t groups, int K, bool backward) {
+  const int s = groups < 16 ? 8 : groups < (backward ? 40 : 64) ? 4 : 1;
+  return s < K ? s : K;  // the look-back window holds K tiles
+}
 
 constexpr int kGbMaxNB = 16;
 
@@ -781,7 +787,7 @@ void fwd_impl(const GbPlan& p, int64_t B, int64_t L, int I, int O, int nb, const
                      bcoef, acoef, u_tail, x0, y, x_last, saved, (const double*)Mc, (const double*)Ms,
                      reinterpret_cast<double*>(ws + p.off_agg), reinterpret_cast<double*>(ws + p.off_inc),
                      reinterpret_cast<unsigned*>(ws), B, L, I, O, p.pp, nb, p.lb.groups, p.lb.K, p.lb.nsuper,
-                     lb_spacing_for(kGbAnchorSpacing));
+                     lb_spacing_for(gb_anchor_spacing(p.lb.groups, p.lb.K, false)));
 }
 
 template <int NA, int NBT>
@@ -804,7 +810,7 @@ void bwd_impl(const GbPlan& p, int64_t B, int64_t L, int I, int O, int nb, const
                        gy, g_xlast, u, bcoef, acoef, u_tail, x0, saved, (const double*)Mc, (const double*)Ms,
                        reinterpret_cast<double*>(ws + p.off_agg), reinterpret_cast<double*>(ws + p.off_inc),
                        reinterpret_cast<unsigned*>(ws), gu, gu_tail, pa, pb, gh, B, L, I, O, p.pp, nb, p.lb.groups,
-                       p.lb.K, p.lb.nsuper, lb_spacing_for(kGbAnchorSpacing));
+                       p.lb.K, p.lb.nsuper, lb_spacing_for(gb_anchor_spacing(p.lb.groups, p.lb.K, true)));
   } else if (gu_tail && nb > 1) {
     const int64_t nt = B * (nb - 1) * I;
     hipLaunchKernelGGL(gblock_zero, grid_for(nt), dim3(256), 0, s, gu_tail, nt);

@@ -473,8 +473,8 @@ __global__ void __launch_bounds__(256) linrec_zero(float* __restrict__ p, int64_
   if (i < n) p[i] = 0.0f;
 }
 
-// Plan: K (chunks per tile) starts at kLbWaves and halves down to 2 while there are fewer than
-// kApTileTarget tiles. Workspace: the tile counter, agg and inc [nsuper][lanes][n] (reset
+// Plan: kLbWaves chunks per tile as lb_plan (32 lanes x 1000 steps, n 4: forward / backward 76 / 83 us
+// at 2 chunks a tile, 22 / 31 at 8). Workspace: the tile counter, agg and inc [nsuper][lanes][n] (reset
 // before each scan), the grad_A partials [nsuper][lanes][n][n], and Mc, Ms [lanes][n][n].
 struct LrPlan {
   int64_t groups = 0, nsuper = 0;
@@ -486,12 +486,9 @@ LrPlan lr_plan(int64_t lanes, int64_t L, int64_t ns) {
   LrPlan p;
   const int64_t S = kTileT / ns;
   p.groups = (lanes + kTile - 1) / kTile;
+  const int64_t chunks = L > 0 ? (L + S - 1) / S : 0;
   if (L > 0) {
-    p.K = kLbWaves;
-    auto tiles = [&](int K) { return p.groups * ((L + S * K - 1) / (S * K)); };
-    while (p.K > 2 && tiles(p.K) < kApTileTarget) p.K /= 2;
-    const int64_t chunks = (L + S - 1) / S;
-    if (p.K > chunks) p.K = (int)chunks;
+    p.K = chunks < kLbWaves ? (int)chunks : kLbWaves;
     p.nsuper = (L + S * p.K - 1) / (S * p.K);
   }
   const size_t f = 8, vecs = f * p.nsuper * lanes * ns;
@@ -500,7 +497,12 @@ LrPlan lr_plan(int64_t lanes, int64_t L, int64_t ns) {
   p.off_part = p.off_inc + vecs;
   p.off_Mc = p.off_part + vecs * ns;
   p.off_Ms = p.off_Mc + f * lanes * ns * ns;
-  p.bytes = p.off_Ms + f * lanes * ns * ns;
+  // The size query keeps the bound of shorter tiles on few lanes (K halved down to 2 below 256 tiles),
+  // which this plan stays within: callers have sized buffers by it.
+  int64_t K = kLbWaves, rows = 0;
+  while (K > 2 && p.groups * ((chunks + K - 1) / K) < 256) K /= 2;
+  if (chunks > 0) rows = K < chunks ? (chunks + K - 1) / K : 1;
+  p.bytes = p.off_agg + f * (rows * lanes * ns * (2 + ns) + 2 * lanes * ns * ns);
   return p;
 }
 
