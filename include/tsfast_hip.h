@@ -298,6 +298,17 @@ int tsfast_hip_projscan_bwd(int64_t B, int64_t L, int64_t H, int64_t N, int64_t 
                             float* g_w_re, float* g_w_im, void* g_lam, float* g_c_re, float* g_c_im, void* g_x0,
                             void* workspace, int64_t workspace_bytes, void* stream);
 
+/* Weight layouts and gradient sums of the projected scan beyond the fused kernel's widths (GEMMs around
+ * the diagonal scan). pack: w [2N, H] rows 2s, 2s + 1 = W_re[s], W_im[s]; c [O, 2N] columns 2s, 2s + 1 =
+ * C_re[:, s], -C_im[:, s]; lam_rows [B, N] = lam per batch row. unpack: the gradients of W, C and lam from
+ * gw [parts_w, 2N, H], gc [parts_c, O, 2N] and glam_rows [B, N], each summed in a fixed order. */
+int tsfast_hip_wide_pack(int64_t B, int64_t H, int64_t N, int64_t O, const float* W_re, const float* W_im,
+                         const void* lam, const float* C_re, const float* C_im, float* w, float* c, void* lam_rows,
+                         void* stream);
+int tsfast_hip_wide_unpack(int64_t B, int64_t H, int64_t N, int64_t O, int64_t parts_w, int64_t parts_c,
+                           const float* gw, const float* gc, const void* glam_rows, float* gW_re, float* gW_im,
+                           void* glam, float* gC_re, float* gC_im, void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * Chunked adjoint of a time-varying matrix recurrence (the sequence-parallel part of a
  * NeuralStateSpace backward). Replaces the pair ssm_bwd_summary + ssm_bwd_scan

@@ -203,3 +203,20 @@ def test_projscan_tbptt_chunks_equal_one_call(gpu):
     torch.cuda.synchronize()
     assert O.rel_err(_np(torch.cat(ys, 1)), _np(y_full)) < TOL
     assert O.rel_err(_np(state), _np(xl_full)) < TOL
+
+
+@pytest.mark.parametrize("B,H,N,O,parts", [(1, 1, 1, 1, 1), (3, 33, 17, 40, 2), (40, 128, 70, 5, 17), (2, 70, 256, 129, 16)])
+def test_wide_pack_and_unpack(gpu, B, H, N, O, parts):
+    """The wide route's weight layouts and gradient sums in one launch each, against torch: the layouts
+    bit for bit, the sums against float64 (partials are added in float64, so only the final rounding)."""
+    g = torch.Generator().manual_seed(N + H)
+    r = lambda *s: torch.randn(*s, generator=g).to(gpu)  # noqa: E731
+    W_re, W_im, C_re, C_im, lam = r(N, H), r(N, H), r(O, N), r(O, N), torch.complex(r(N), r(N))
+    w, c, rows = projected_hip._pack(B, W_re, W_im, lam, C_re, C_im)
+    assert torch.equal(w, projected_hip._w_cat(W_re, W_im)) and torch.equal(c, projected_hip._c_cat(C_re, C_im))
+    assert torch.equal(rows, lam.expand(B, N))
+    g_w, g_c, g_rows = r(parts, 2 * N, H), r(parts, O, 2 * N), torch.complex(r(B, N), r(B, N))
+    gw, gc = g_w.double().sum(0), g_c.double().sum(0)
+    want = (gw[0::2], gw[1::2], g_rows.to(torch.complex128).sum(0), gc[:, 0::2], -gc[:, 1::2])
+    for got, ref in zip(projected_hip._unpack(g_w, g_c, g_rows), want):
+        assert got.is_contiguous() and (got - ref).abs().max() <= 1e-7 * max(1.0, ref.abs().max().item())

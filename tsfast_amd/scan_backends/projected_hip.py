@@ -154,7 +154,9 @@ def _deterministic_bwd(gy, g_xlast, u, W_re, W_im, lam, C_re, C_im, x0):
     the tiles the workgroup takes from a counter, and which tiles those are depends on timing,
     while every step here gives the same bits on every run (the diagonal scan's look-back is
     anchored in this mode)."""
-    return _wide_backward(gy, g_xlast, _wide_states(u, W_re, W_im, lam, x0), u, W_re, W_im, lam, C_re, C_im, x0)
+    packed = _pack(u.shape[0], W_re, W_im, lam, C_re, C_im)
+    x = _wide_states(u, packed[0], packed[2], x0)
+    return _wide_backward(gy, g_xlast, x, u, W_re, W_im, lam, C_re, C_im, x0, packed)
 
 
 @custom_op("tsfast_hip::projected_scan_bwd")
@@ -242,16 +244,19 @@ def _gram(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     gradients of the projections. One GEMM with K in the hundreds of thousands keeps few output
     tiles busy (24-73 TFLOP/s measured at M, N = 512..1024, 32..128); cut into 16 batched products
     over consecutive row blocks and summed in a fixed order, the same product runs at 110-134."""
+    return _gram_parts(a, b).sum(0)
+
+
+def _gram_parts(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+    """``_gram``'s partial products ``[parts, M, N]``, one over each block of rows."""
     K, M = a.shape
     parts = min(_SPLITK_PARTS, K // _SPLITK_ROWS)
     if parts < 2:
-        return a.t() @ b
+        return (a.t() @ b).unsqueeze(0)
     rows = K // parts
     main = parts * rows
-    out = torch.bmm(a[:main].view(parts, rows, M).transpose(1, 2), b[:main].view(parts, rows, b.shape[1])).sum(0)
-    if main < K:
-        out += a[main:].t() @ b[main:]
-    return out
+    out = torch.bmm(a[:main].view(parts, rows, M).transpose(1, 2), b[:main].view(parts, rows, b.shape[1]))
+    return out if main == K else torch.cat((out, (a[main:].t() @ b[main:]).unsqueeze(0)))
 
 
 def _w_cat(W_re, W_im):
@@ -268,18 +273,58 @@ def _c_cat(C_re, C_im):
     return torch.stack((C_re, -C_im), -1).view(O, 2 * N)
 
 
+def _pack(B, W_re, W_im, lam, C_re, C_im):
+    """``(w, c, lam_rows)``: ``_w_cat``, ``_c_cat`` and lam once per batch row ``[B, N]``, in one
+    launch on the GPU."""
+    N, H = W_re.shape
+    O = C_re.shape[0]
+    if not W_re.is_cuda:
+        return _w_cat(W_re, W_im), _c_cat(C_re, C_im), lam.expand(B, N).contiguous()
+    lib = _lib.load()
+    for name, t in (("W_re", W_re), ("W_im", W_im), ("C_re", C_re), ("C_im", C_im)):
+        _lib.require(t, name, (torch.float32,), W_re.device)
+    _lib.require(lam, "lam", (torch.complex64,), W_re.device)
+    w, c, rows = W_re.new_empty(2 * N, H), C_re.new_empty(O, 2 * N), lam.new_empty(B, N)
+    _lib.check(
+        lib.tsfast_hip_wide_pack(B, H, N, O, *map(_lib.ptr, (W_re, W_im, lam, C_re, C_im, w, c, rows)), _lib.stream_of(W_re)),
+        "tsfast_hip_wide_pack",
+    )
+    return w, c, rows
+
+
+def _unpack(g_w, g_c, g_lam_rows):
+    """``(g_W_re, g_W_im, g_lam, g_C_re, g_C_im)`` from the partial products ``g_w [parts, 2N, H]`` and
+    ``g_c [parts, O, 2N]`` in the packed layouts and ``g_lam_rows [B, N]``, each summed in order; one
+    launch on the GPU."""
+    if not g_w.is_cuda:
+        gw, gc = g_w.sum(0), g_c.sum(0)
+        return _fresh(gw[0::2]), _fresh(gw[1::2]), g_lam_rows.sum(0), _fresh(gc[:, 0::2]), -gc[:, 1::2]
+    lib = _lib.load()
+    g_w, g_c, g_lam_rows = _dense(g_w, g_c, g_lam_rows)
+    for name, t, dt in (("g_w", g_w, torch.float32), ("g_c", g_c, torch.float32), ("g_lam", g_lam_rows, torch.complex64)):
+        _lib.require(t, name, (dt,), g_w.device)
+    (parts_w, N2, H), (parts_c, O, _), (B, N) = g_w.shape, g_c.shape, g_lam_rows.shape
+    out = (g_w.new_empty(N, H), g_w.new_empty(N, H), g_lam_rows.new_empty(N), g_c.new_empty(O, N), g_c.new_empty(O, N))
+    _lib.check(
+        lib.tsfast_hip_wide_unpack(
+            B, H, N, O, parts_w, parts_c, *map(_lib.ptr, (g_w, g_c, g_lam_rows, *out)), _lib.stream_of(g_w)
+        ),
+        "tsfast_hip_wide_unpack",
+    )
+    return out
+
+
 def _fresh(t):
     """A contiguous copy: a custom op's outputs may not alias each other (a slice that is already
     contiguous, as at B = 1 or N = 1, would come back from ``contiguous()`` as a view)."""
     return t.clone(memory_format=torch.contiguous_format)
 
 
-def _wide_states(u, W_re, W_im, lam, x0):
+def _wide_states(u, w, lam_rows, x0):
     """The states x [B, L, N] (B L > 0): v by one GEMM, then the diagonal scan kernels."""
     B, L, _ = u.shape
-    N = lam.shape[0]
-    v = torch.view_as_complex(F.linear(u, _w_cat(W_re, W_im)).view(B, L, N, 2))
-    return diagonal_hip.forward(lam.expand(B, N).contiguous(), v, x0)
+    v = torch.view_as_complex(F.linear(u, w).view(B, L, lam_rows.shape[1], 2))
+    return diagonal_hip.forward(lam_rows, v, x0)
 
 
 def _wide_forward(u, W_re, W_im, lam, C_re, C_im, x0):
@@ -289,15 +334,17 @@ def _wide_forward(u, W_re, W_im, lam, C_re, C_im, x0):
     if B * L == 0:
         x_last = x0.clone() if x0 is not None else lam.new_zeros(B, N)
         return u.new_zeros(B, L, O), x_last, lam.new_empty(B, L, N)
-    x = _wide_states(u, W_re, W_im, lam, x0)
-    y = F.linear(torch.view_as_real(x).view(B, L, 2 * N), _c_cat(C_re, C_im))
+    w, c, lam_rows = _pack(B, W_re, W_im, lam, C_re, C_im)
+    x = _wide_states(u, w, lam_rows, x0)
+    y = F.linear(torch.view_as_real(x).view(B, L, 2 * N), c)
     return y, _fresh(x[:, -1]), x
 
 
-def _wide_backward(gy, g_xlast, x, u, W_re, W_im, lam, C_re, C_im, x0):
+def _wide_backward(gy, g_xlast, x, u, W_re, W_im, lam, C_re, C_im, x0, packed=None):
     """Every gradient of the wide route, written out: g_x = gy C (one GEMM, plus the returned
     state's gradient at the last step), the adjoint scan kernels (grad v, grad lam per row, grad
-    x0), g_u = grad v W (one GEMM), and the weight gradients by ``_gram``."""
+    x0), g_u = grad v W (one GEMM), and the weight gradients by ``_gram_parts``. ``packed`` is
+    ``_pack``'s result where the caller has it."""
     B, L, H = u.shape
     N, O = lam.shape[0], C_re.shape[0]
     g_x0 = lam.new_empty(0)
@@ -306,18 +353,17 @@ def _wide_backward(gy, g_xlast, x, u, W_re, W_im, lam, C_re, C_im, x0):
             g_x0 = g_xlast.clone() if g_xlast is not None else torch.zeros_like(x0)
         zeros = [torch.zeros_like(t) for t in (u, W_re, W_im, lam, C_re, C_im)]
         return (*zeros, g_x0)
-    w, c = _w_cat(W_re, W_im), _c_cat(C_re, C_im)
+    w, c, lam_rows = packed if packed is not None else _pack(B, W_re, W_im, lam, C_re, C_im)
     g_x = torch.view_as_complex((gy.view(B * L, O) @ c).view(B, L, N, 2))
     if g_xlast is not None:
         g_x[:, -1] += g_xlast
-    g_lam_rows, g_v, g_x0 = diagonal_hip.backward(g_x, lam.expand(B, N).contiguous(), x, x0)
+    g_lam_rows, g_v, g_x0 = diagonal_hip.backward(g_x, lam_rows, x, x0)
     del g_x
     g_vr = torch.view_as_real(g_v).view(B * L, 2 * N)
     g_u = (g_vr @ w).view(B, L, H)
-    g_w = _gram(g_vr, u.view(B * L, H))
-    g_c = _gram(gy.view(B * L, O), torch.view_as_real(x).view(B * L, 2 * N))
-    return (g_u, _fresh(g_w[0::2]), _fresh(g_w[1::2]), g_lam_rows.sum(0), _fresh(g_c[:, 0::2]), -g_c[:, 1::2],
-            g_x0 if x0 is not None else lam.new_empty(0))
+    g_w = _gram_parts(g_vr, u.view(B * L, H))
+    g_c = _gram_parts(gy.view(B * L, O), torch.view_as_real(x).view(B * L, 2 * N))
+    return (g_u, *_unpack(g_w, g_c, g_lam_rows), g_x0 if x0 is not None else lam.new_empty(0))
 
 
 @custom_op("tsfast_hip::projected_scan_wide")
