@@ -220,3 +220,12 @@ def test_wide_pack_and_unpack(gpu, B, H, N, O, parts):
     want = (gw[0::2], gw[1::2], g_rows.to(torch.complex128).sum(0), gc[:, 0::2], -gc[:, 1::2])
     for got, ref in zip(projected_hip._unpack(g_w, g_c, g_rows), want):
         assert got.is_contiguous() and (got - ref).abs().max() <= 1e-7 * max(1.0, ref.abs().max().item())
+
+
+@pytest.mark.parametrize("shape", [(1, 545, 5, 20, 3), (30, 300, 4, 70, 4), (64, 161, 4, 96, 4)])
+def test_projscan_anchor_spacings(gpu, shape):
+    """One case per anchor spacing (8, 4 and 2 chunks apart), with a partial last chunk and a chain
+    longer than one span."""
+    u, W_re, W_im, lam, C_re, C_im, x0, gy, g_xl = _make(*shape, seed=sum(shape))
+    y, xl, grads = _run(gpu, u, W_re, W_im, lam, C_re, C_im, x0, gy, g_xl)
+    _check(y, xl, grads, u, W_re, W_im, lam, C_re, C_im, x0, gy, g_xl)

@@ -324,3 +324,18 @@ def test_forced_give_up_raises_without_debug_mode(gpu):
     torch.cuda.synchronize()
     _lib.raise_if_lookback_gave_up("clean")
     assert O.rel_err(_np(out2), O.diag_forward(_np(lam[:2]), _np(small_v))) < TOL
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.complex64])
+@pytest.mark.parametrize("M,L,N", [(1, 4097, 5), (2, 4400, 70), (1, 8449, 33)])
+def test_diag_few_lanes_keep_whole_tiles(gpu, dtype, M, L, N):
+    """Sequences past the whole-sequence tiles on a lane group or three: 16-chunk look-back tiles with
+    a ragged last one, and a chain longer than one anchor span."""
+    lam, v, x0, g = _make_diag((M, L, N), (N,), dtype, seed=L)
+    lam, v, x0, g = (t.to(gpu) for t in (lam.expand(M, N).contiguous(), v, x0.expand(M, N).contiguous(), g))
+    out = diagonal_hip.forward(lam, v, x0)
+    glam, gv, gx0 = diagonal_hip.backward(g, lam, out, x0)
+    want = O.diag_forward(_np(lam), _np(v), _np(x0))
+    wl, wv, w0 = O.diag_backward(_np(g), _np(lam), want, _np(x0))
+    for got, ref in ((out, want), (glam, wl), (gv, wv), (gx0, w0)):
+        assert O.rel_err(_np(got), ref) < TOL

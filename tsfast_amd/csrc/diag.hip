@@ -859,18 +859,17 @@ inline dim3 grid_for(int64_t threads) { return dim3((unsigned)((threads + 255) /
 // the 128 VGPRs a 1024-thread workgroup allows). Every
 // thread issues all TC loads of its chunk at once, so the bytes in flight do not depend on TC;
 // the wave count (lanes / 64 x L / TC) does, and TC drops to 16 when 32 would leave fewer than
-// kDiagWaveTarget waves. K (chunks per tile) starts at TSF_DIAG_KMAX and halves down to 4 while
-// there are fewer than kDiagTileTarget tiles.
-#ifndef TSF_DIAG_TILE_TARGET
-#define TSF_DIAG_TILE_TARGET 256
-#endif
+// kDiagWaveTarget waves. K (chunks per tile) is TSF_DIAG_KMAX, or the chunks of a shorter sequence:
+// halving it to reach a tile per CU, as few lanes once did, lengthens the chain of look-backs by more
+// than the extra workgroups shorten the tiles (4 rows x 8192 steps x 32 lanes, forward / backward:
+// complex 58 / 64 us at 4 chunks a tile, 21 / 27 at 16; real 46 / 48 and 15 / 19; no size measured was
+// slower at 16).
 #ifndef TSF_DIAG_WAVE_TARGET
 #define TSF_DIAG_WAVE_TARGET 4096
 #endif
 #ifndef TSF_DIAG_KMAX
 #define TSF_DIAG_KMAX 16
 #endif
-constexpr int64_t kDiagTileTarget = TSF_DIAG_TILE_TARGET;
 constexpr int64_t kDiagWaveTarget = TSF_DIAG_WAVE_TARGET;
 static_assert(TSF_DIAG_KMAX >= 4 && TSF_DIAG_KMAX <= kMaxWaves, "K range");
 
@@ -887,8 +886,6 @@ DiagTile diag_tile(int64_t lanes, int64_t L, int tc_max) {
   t.TC = (t.groups * ((L + 31) / 32) < kDiagWaveTarget) ? 16 : 32;
   if (t.TC > tc_max) t.TC = tc_max;
   t.K = TSF_DIAG_KMAX;
-  auto tiles = [&](int K) { return t.groups * ((L + (int64_t)t.TC * K - 1) / ((int64_t)t.TC * K)); };
-  while (t.K > 4 && tiles(t.K) < kDiagTileTarget) t.K /= 2;
   const int64_t chunks = (L + t.TC - 1) / t.TC;
   if (t.K > chunks) t.K = (int)chunks;  // no waves past the end of a short sequence
   t.SL = (int64_t)t.TC * t.K;

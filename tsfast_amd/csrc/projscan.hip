@@ -50,7 +50,15 @@ constexpr int kRho = 2 * kWaveStates;     // interleaved real rows (re, im) of a
 constexpr int kMaxWaves = 8;              // N <= 256
 constexpr int kXtStride = kRho + 4;       // floats per row of a wave's transposed block in LDS
 constexpr uint32_t kOob = 0xFFFFFFF0u;    // buffer offset past every resource: loads return 0
-constexpr int kProjAnchorSpacing = 2;     // deterministic-mode anchor spacing (measured: 1-2 cost nothing, 8 cost 10%)
+// Deterministic-mode anchor spacing, by the waves that run side by side in one chunk of every row. Many
+// keep the chip busy while a chain waits, and an anchor every other chunk is cheapest (64 rows, N 256,
+// 4096 steps: forward 350 us at 2, 387 at 4); few wait for their chains, one round trip per anchor (8 rows,
+// N 64, 4000 steps: forward / backward 122 / 210 us at 2, 85 / 141 at 4, 71 / 112 at 8; 16 rows, N 256 154 / 289
+// at 2, 142 / 277 at 4, 153 / 294 at 8; 64 rows, N 32 171 / 288, 156 / 215 and 160 / 215).
+inline int proj_anchor_spacing(int64_t B, int64_t N) {
+  const int64_t waves = B * ((N + 31) / 32);
+  return waves >= 192 ? 2 : waves >= 56 ? 4 : 8;
+}
 
 TSF_DEV f4 mfma(float a, float b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 TSF_DEV f4 f4_zero() { return f4{0.0f, 0.0f, 0.0f, 0.0f}; }
@@ -917,7 +925,7 @@ int fwd_launch(const PsPlan& p, int64_t B, int64_t L, int64_t H, int64_t N, int6
   hipLaunchKernelGGL((projscan_fwd<KS, OB>), dim3((unsigned)(p.tiles < cap ? p.tiles : cap)), dim3(threads), lds, s, u,
                      w_re, w_im, lam, c_re, c_im, x0, y, x_last, saved, reinterpret_cast<double2*>(ws + p.off_agg),
                      reinterpret_cast<double2*>(ws + p.off_inc), reinterpret_cast<unsigned*>(ws), (int)B, (int)L,
-                     (int)H, (int)N, (int)O, (int)p.nchunks, (int)p.nsub, lb_spacing_for(kProjAnchorSpacing));
+                     (int)H, (int)N, (int)O, (int)p.nchunks, (int)p.nsub, lb_spacing_for(proj_anchor_spacing(B, N)));
   return TSF_OK;
 }
 
@@ -938,7 +946,7 @@ int bwd_launch(const PbPlan& p, int64_t B, int64_t L, int64_t H, int64_t N, int6
   hipLaunchKernelGGL((projscan_bwd<KS, OB>), dim3((unsigned)grid), dim3(threads), lds, s, gy, g_xlast, saved, u, w_re,
                      w_im, lam, c_re, c_im, g_u, g_x0, part, p.part_stride,
                      reinterpret_cast<double2*>(ws + p.off_agg), reinterpret_cast<double2*>(ws + p.off_inc),
-                     reinterpret_cast<unsigned*>(ws), (int)B, (int)L, (int)H, (int)N, (int)O, (int)p.nsub, lb_spacing_for(kProjAnchorSpacing));
+                     reinterpret_cast<unsigned*>(ws), (int)B, (int)L, (int)H, (int)N, (int)O, (int)p.nsub, lb_spacing_for(proj_anchor_spacing(B, N)));
   const int64_t outs = 2 * N * H + 2 * O * N + 2 * N;
   hipLaunchKernelGGL(projscan_bwd_reduce, dim3((unsigned)((outs + 63) / 64)), dim3(256), 0, s, part, p.part_stride,
                      grid, (int)N, p.nw * kWaveStates, (int)H, KS == 8 ? 32 : 16, (int)O, 16 * OB, g_w_re, g_w_im, g_c_re,
