@@ -93,6 +93,14 @@ int tsfast_hip_diag_fwd(int64_t M, int64_t L, int64_t N, int is_complex, const v
 int tsfast_hip_diag_bwd(int64_t M, int64_t L, int64_t N, int is_complex, const void* g, const void* lam,
                         const void* out, const void* x0, void* gv, void* glam, void* gx0, void* workspace,
                         int64_t workspace_bytes, void* stream);
+/* The same scan with one coefficient row for every batch row: lam and glam are [N] (glam summed over the
+ * rows), everything else as above. */
+int64_t tsfast_hip_diag_shared_workspace_bytes(int64_t M, int64_t L, int64_t N, int is_complex);
+int tsfast_hip_diag_shared_fwd(int64_t M, int64_t L, int64_t N, int is_complex, const void* lam, const void* v,
+                               const void* x0, void* out, void* workspace, int64_t workspace_bytes, void* stream);
+int tsfast_hip_diag_shared_bwd(int64_t M, int64_t L, int64_t N, int is_complex, const void* g, const void* lam,
+                               const void* out, const void* x0, void* gv, void* glam, void* gx0, void* workspace,
+                               int64_t workspace_bytes, void* stream);
 
 /* No-allocation variant of tsfast_hip_diag_fwd. It has no counterpart in the reference: it is for
  * callers that cannot allocate device memory (code under HIP graph capture, tight serving loops,

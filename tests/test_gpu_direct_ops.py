@@ -37,7 +37,7 @@ def test_direct_equals_dispatched_and_modes_see_the_ops(gpu):
     direct = _pass(*_inputs(gpu))
     with _Names() as mode:
         dispatched = _pass(*_inputs(gpu))
-    assert any("scan_diagonal." in n for n in mode.names) and any("scan_diagonal_bwd" in n for n in mode.names)
+    assert any("scan_diagonal_shared." in n for n in mode.names) and any("shared_bwd" in n for n in mode.names)
     for a, b in zip(direct, dispatched):
         assert torch.equal(a, b)
 

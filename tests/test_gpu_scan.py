@@ -339,3 +339,22 @@ def test_diag_few_lanes_keep_whole_tiles(gpu, dtype, M, L, N):
     wl, wv, w0 = O.diag_backward(_np(g), _np(lam), want, _np(x0))
     for got, ref in ((out, want), (glam, wl), (gv, wv), (gx0, w0)):
         assert O.rel_err(_np(got), ref) < TOL
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.complex64])
+@pytest.mark.parametrize("M,L,N", [(1, 40, 5), (7, 200, 33), (300, 64, 70), (5, 1300, 130), (130, 1100, 140), (3, 9000, 17), (2, 0, 4), (0, 5, 4)])
+def test_diag_shared_coefficients(gpu, dtype, M, L, N):
+    """One coefficient row for every batch row (whole-sequence and look-back tiles, one and many row
+    blocks, empty sequences and batches): the states, grad v and grad x0 of the expanded call bit for
+    bit, grad lam against the float64 sum of the rows' gradients."""
+    lam, v, x0, g = _make_diag((M, L, N), (N,), dtype, seed=M + L)
+    lam, v, x0, g = (t.to(gpu) for t in (lam, v, x0, g))
+    rows = lam.expand(M, N).contiguous()
+    out = diagonal_hip.forward(lam, v, x0)
+    assert torch.equal(out, diagonal_hip.forward(rows, v, x0))
+    glam, gv, gx0 = diagonal_hip.backward(g, lam, out, x0)
+    wl, wv, w0 = diagonal_hip.backward(g, rows, out, x0)
+    assert torch.equal(gv, wv) and torch.equal(gx0, w0) and glam.shape == (N,)
+    ref = wl.to(torch.complex128 if dtype.is_complex else torch.float64).sum(0)
+    scale = wl.abs().double().sum(0).clamp_min(1e-30)  # each row's gradient carries one fp32 rounding
+    assert ((glam - ref).abs() <= 3e-7 * scale).all()

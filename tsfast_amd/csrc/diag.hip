@@ -175,7 +175,7 @@ __global__ void __launch_bounds__(1024) diag_fwd(const T* __restrict__ lam, cons
                                                  Map<typename Wide<T>::type>* __restrict__ agg,
                                                  typename Wide<T>::type* __restrict__ inc, unsigned* __restrict__ counter,
                                                  int64_t lanes, int64_t L, int64_t N, int64_t groups, int K,
-                                                 int64_t nsuper, LbCfg lb_spacing) {
+                                                 int64_t nsuper, LbCfg lb_spacing, bool shared) {
   using W = typename Wide<T>::type;
   __shared__ W s_e[kMaxWaves][64];
   // the look-back window, then (once the look-back is done) the state entering each chunk
@@ -202,8 +202,8 @@ __global__ void __launch_bounds__(1024) diag_fwd(const T* __restrict__ lam, cons
     T vb[TC];
     int64_t base = 0;
     if (live) {
-      a = Wide<T>::up(lam[lane]);
       const int64_t m = lane / N, n = lane - m * N;
+      a = Wide<T>::up(lam[shared ? n : lane]);
       base = (m * L + t0) * N + n;
       const T* vp = v + base;
       if (len == TC) {
@@ -276,7 +276,8 @@ __global__ void __launch_bounds__(1024) diag_bwd(const T* __restrict__ lam, cons
                                                  typename Wide<T>::type* __restrict__ inc, unsigned* __restrict__ counter,
                                                  T* __restrict__ gv, typename Wide<T>::type* __restrict__ part,
                                                  T* __restrict__ glam, T* __restrict__ gx0, int64_t lanes, int64_t L,
-                                                 int64_t N, int64_t groups, int K, int64_t nsuper, LbCfg lb_spacing) {
+                                                 int64_t N, int64_t groups, int K, int64_t nsuper, LbCfg lb_spacing,
+                                                 bool shared) {
   using W = typename Wide<T>::type;
   __shared__ W s_f[kMaxWaves][64];
   // the look-back window, then G entering each chunk from the right (s_start) and the glam
@@ -310,8 +311,8 @@ __global__ void __launch_bounds__(1024) diag_bwd(const T* __restrict__ lam, cons
     T gb[TC];  // g_t of the chunk's steps
     int64_t base = 0;
     if (live) {
-      ac = Num<W>::conj(Wide<T>::up(lam[lane]));
       const int64_t m = lane / N, n = lane - m * N;
+      ac = Num<W>::conj(Wide<T>::up(lam[shared ? n : lane]));
       base = (m * L + t0) * N + n;
       const T* gp = g + base;
       const T* xp = out + base;
@@ -400,7 +401,7 @@ __global__ void __launch_bounds__(1024) diag_bwd(const T* __restrict__ lam, cons
     if (k == 0 && live) {
       W s = s_acc[0][lid];
       for (int j = 1; j < K; ++j) s = Num<W>::add(s, s_acc[j][lid]);
-      if (nsuper == 1)
+      if (nsuper == 1 && !shared)
         glam[lane] = Wide<T>::down(s);
       else
         part[sc * lanes + lane] = s;
@@ -428,7 +429,7 @@ template <typename T, int TC, int LG, int KMAX>
 __global__ void __launch_bounds__(LG * KMAX) diag_whole_fwd(const T* __restrict__ lam, const T* __restrict__ v,
                                                                  const T* __restrict__ x0, T* __restrict__ out,
                                                                  unsigned* __restrict__ ws_head, int64_t lanes,
-                                                                 int64_t L, int64_t N) {
+                                                                 int64_t L, int64_t N, bool shared) {
   using W = typename Wide<T>::type;
   __shared__ W s_e[KMAX][LG];
   const int lid = threadIdx.x % LG, k = threadIdx.x / LG;
@@ -441,8 +442,8 @@ __global__ void __launch_bounds__(LG * KMAX) diag_whole_fwd(const T* __restrict_
   T vb[TC];
   int64_t base = 0;
   if (live) {
-    a = Wide<T>::up(lam[lane]);
     const int64_t m = lane / N, n = lane - m * N;
+    a = Wide<T>::up(lam[shared ? n : lane]);
     base = (m * L + t0) * N + n;
     const T* vp = v + base;
     if (len == TC) {
@@ -494,7 +495,7 @@ __global__ void __launch_bounds__(LG * KMAX) diag_whole_bwd(const T* __restrict_
                                                                  const T* __restrict__ out, const T* __restrict__ x0,
                                                                  T* __restrict__ gv, T* __restrict__ glam,
                                                                  T* __restrict__ gx0, unsigned* __restrict__ ws_head,
-                                                                 int64_t lanes, int64_t L, int64_t N) {
+                                                                 int64_t lanes, int64_t L, int64_t N, bool shared) {
   using W = typename Wide<T>::type;
   constexpr int H2 = TC / 2;
   constexpr bool kKeep = LG * KMAX <= 256;
@@ -511,8 +512,8 @@ __global__ void __launch_bounds__(LG * KMAX) diag_whole_bwd(const T* __restrict_
   T gb[TC];
   T xb[kKeep ? TC : 1];  // narrow groups: x_{t-1} of the whole chunk, loaded with g
   if (live) {
-    ac = Num<W>::conj(Wide<T>::up(lam[lane]));
     const int64_t m = lane / N, n = lane - m * N;
+    ac = Num<W>::conj(Wide<T>::up(lam[shared ? n : lane]));
     base = (m * L + t0) * N + n;
     const T* gp = g + base;
     if (kKeep) {
@@ -604,7 +605,10 @@ __global__ void __launch_bounds__(LG * KMAX) diag_whole_bwd(const T* __restrict_
   if (k == 0 && live) {
     W sum = s_acc[0][lid];
     for (int j = 1; j < K; ++j) sum = Num<W>::add(sum, s_acc[j][lid]);
-    glam[lane] = Wide<T>::down(sum);
+    if (shared)  // this lane's term, after the header (summed over the rows by diag_sum_shared)
+      reinterpret_cast<W*>(reinterpret_cast<char*>(ws_head) + kCounterBytes)[lane] = sum;
+    else
+      glam[lane] = Wide<T>::down(sum);
   }
 }
 
@@ -853,6 +857,31 @@ __global__ void __launch_bounds__(1024) sel_bwd(const float* __restrict__ a, con
 
 inline dim3 grid_for(int64_t threads) { return dim3((unsigned)((threads + 255) / 256)); }
 
+// grad of coefficients shared by every batch row: the sum of the partials [rows][N] (a row per
+// super-chunk and batch row) over the rows, in a fixed order: 16 columns a workgroup, thread (s, j) the
+// rows s, s + 64, .. of column j with eight loads in flight, then the 64 sums in order. As torch's sum of
+// the per-row gradients it was another pass and launch after diag_sum_parts.
+template <typename T>
+__global__ void __launch_bounds__(1024) diag_sum_shared(const typename Wide<T>::type* __restrict__ part,
+                                                        T* __restrict__ dst, int64_t N, int64_t rows) {
+  using W = typename Wide<T>::type;
+  __shared__ W s_p[64][16];
+  const int j = threadIdx.x & 15, s = threadIdx.x >> 4;
+  const int64_t n = blockIdx.x * (int64_t)16 + j;
+  W acc = Num<W>::zero();
+  if (n < N) {
+#pragma unroll 8
+    for (int64_t r = s; r < rows; r += 64) acc = Num<W>::add(acc, part[r * N + n]);
+  }
+  s_p[s][j] = acc;
+  __syncthreads();
+  if (s == 0 && n < N) {
+    W t = s_p[0][j];
+    for (int q = 1; q < 64; ++q) t = Num<W>::add(t, s_p[q][j]);
+    dst[n] = Wide<T>::down(t);
+  }
+}
+
 // Tile shape for one call. TC (steps per chunk) is a template parameter, at most tc_max: 32 for
 // real lanes, 16 for complex ones and for the time-varying backward (a thread keeps its chunk's
 // inputs in registers across the look-back: TC complex values, or three TC-step arrays, within
@@ -944,11 +973,12 @@ inline bool whole_both(int64_t lanes, int64_t L, bool cplx) {
 
 template <typename T, int TC>
 void whole_fwd_launch(const WholeTile& w, int64_t lanes, int64_t L, int64_t N, const T* lam, const T* v, const T* x0,
-                      T* out, unsigned* ws, hipStream_t s) {
+                      T* out, unsigned* ws, hipStream_t s, bool shared) {
   const dim3 grid((unsigned)((lanes + w.lg - 1) / w.lg)), block((unsigned)(w.lg * ((L + TC - 1) / TC)));
 #define TSF_WHOLE_FWD(LG, KMAX) \
   if (w.lg == LG && w.kmax == KMAX) { \
-    hipLaunchKernelGGL((diag_whole_fwd<T, TC, LG, KMAX>), grid, block, 0, s, lam, v, x0, out, ws, lanes, L, N); \
+    hipLaunchKernelGGL((diag_whole_fwd<T, TC, LG, KMAX>), grid, block, 0, s, lam, v, x0, out, ws, lanes, L, N, \
+                       shared); \
     return; \
   }
   TSF_WHOLE_FWD(64, 16) TSF_WHOLE_FWD(16, 16) TSF_WHOLE_FWD(8, 16) TSF_WHOLE_FWD(16, 64) TSF_WHOLE_FWD(8, 64)
@@ -957,12 +987,16 @@ void whole_fwd_launch(const WholeTile& w, int64_t lanes, int64_t L, int64_t N, c
 
 template <typename T, int TC>
 void whole_bwd_launch(const WholeTile& w, int64_t lanes, int64_t L, int64_t N, const T* lam, const T* g, const T* out,
-                      const T* x0, T* gv, T* glam, T* gx0, unsigned* ws, hipStream_t s) {
+                      const T* x0, T* gv, T* glam, T* gx0, unsigned* ws, hipStream_t s, bool shared) {
   const dim3 grid((unsigned)((lanes + w.lg - 1) / w.lg)), block((unsigned)(w.lg * ((L + TC - 1) / TC)));
 #define TSF_WHOLE_BWD(LG, KMAX) \
   if (w.lg == LG && w.kmax == KMAX) { \
     hipLaunchKernelGGL((diag_whole_bwd<T, TC, LG, KMAX>), grid, block, 0, s, lam, g, out, x0, gv, glam, gx0, ws, \
-                       lanes, L, N); \
+                       lanes, L, N, shared); \
+    if (shared) \
+      hipLaunchKernelGGL(diag_sum_shared<T>, dim3((unsigned)((N + 15) / 16)), dim3(1024), 0, s, \
+                         reinterpret_cast<const typename Wide<T>::type*>(reinterpret_cast<char*>(ws) + kCounterBytes), \
+                         glam, N, lanes / N); \
     return; \
   }
   TSF_WHOLE_BWD(64, 16) TSF_WHOLE_BWD(16, 16)
@@ -971,19 +1005,20 @@ void whole_bwd_launch(const WholeTile& w, int64_t lanes, int64_t L, int64_t N, c
 
 template <typename T, int TC>
 void diag_fwd_launch(const DiagTile& t, const T* lam, const T* v, const T* x0, T* out, char* ws, int64_t L, int64_t N,
-                     hipStream_t s) {
+                     hipStream_t s, bool shared) {
   using W = typename Wide<T>::type;
   static int occ[kMaxWaves + 1];
   auto* agg = reinterpret_cast<Map<W>*>(ws + kCounterBytes);
   auto* inc = reinterpret_cast<W*>(agg + t.nsuper * t.lanes);
   lookback_reset_launch(ws, lookback_bytes(t, sizeof(W)) / 8, s);
   hipLaunchKernelGGL((diag_fwd<T, TC>), dim3(persistent_grid(t, diag_fwd<T, TC>, occ)), dim3(64 * t.K), 0, s, lam, v,
-                     x0, out, agg, inc, reinterpret_cast<unsigned*>(ws), t.lanes, L, N, t.groups, t.K, t.nsuper, lb_spacing_for(anchor_spacing_for_groups(t.groups)));
+                     x0, out, agg, inc, reinterpret_cast<unsigned*>(ws), t.lanes, L, N, t.groups, t.K, t.nsuper,
+                     lb_spacing_for(anchor_spacing_for_groups(t.groups)), shared);
 }
 
 template <typename T, int TC>
 void diag_bwd_launch(const DiagTile& t, const T* g, const T* lam, const T* out, const T* x0, T* gv, T* glam, T* gx0,
-                     char* ws, int64_t L, int64_t N, hipStream_t s) {
+                     char* ws, int64_t L, int64_t N, hipStream_t s, bool shared) {
   using W = typename Wide<T>::type;
   static int occ[kMaxWaves + 1];
   auto* agg = reinterpret_cast<Map<W>*>(ws + kCounterBytes);
@@ -992,8 +1027,11 @@ void diag_bwd_launch(const DiagTile& t, const T* g, const T* lam, const T* out, 
   lookback_reset_launch(ws, lookback_bytes(t, sizeof(W)) / 8, s);
   hipLaunchKernelGGL((diag_bwd<T, TC>), dim3(persistent_grid(t, diag_bwd<T, TC>, occ)), dim3(64 * t.K), 0, s, lam, g,
                      out, x0, agg, inc, reinterpret_cast<unsigned*>(ws), gv, part, glam, gx0, t.lanes, L, N, t.groups,
-                     t.K, t.nsuper, lb_spacing_for(anchor_spacing_for_groups(t.groups)));
-  if (t.nsuper > 1)
+                     t.K, t.nsuper, lb_spacing_for(anchor_spacing_for_groups(t.groups)), shared);
+  if (shared)
+    hipLaunchKernelGGL(diag_sum_shared<T>, dim3((unsigned)((N + 15) / 16)), dim3(1024), 0, s, (const W*)part, glam, N,
+                       t.nsuper * (t.lanes / N));
+  else if (t.nsuper > 1)
     hipLaunchKernelGGL(diag_sum_parts<T>, dim3((unsigned)t.groups), dim3(64 * kMaxWaves), 0, s, (const W*)part, glam,
                        t.lanes, t.nsuper);
 }
@@ -1085,8 +1123,9 @@ int64_t tsfast_hip_diag_workspace_bytes(int64_t M, int64_t L, int64_t N, int is_
   return kCounterBytes + 4 * (f.nsuper > b.nsuper ? f.nsuper : b.nsuper) * M * N * (is_complex ? 16 : 8);
 }
 
-int tsfast_hip_diag_fwd(int64_t M, int64_t L, int64_t N, int is_complex, const void* lam, const void* v,
-                        const void* x0, void* out, void* workspace, int64_t workspace_bytes, void* stream) {
+static int diag_fwd_impl(int64_t M, int64_t L, int64_t N, int is_complex, const void* lam, const void* v,
+                         const void* x0, void* out, void* workspace, int64_t workspace_bytes, void* stream,
+                         bool shared) {
   if (M < 0 || L < 0 || N < 0) return TSF_ERR_ARG;
   if (M == 0 || L == 0 || N == 0) return TSF_OK;
   if (!lam || !v || !out) return TSF_ERR_ARG;
@@ -1097,52 +1136,78 @@ int tsfast_hip_diag_fwd(int64_t M, int64_t L, int64_t N, int is_complex, const v
     if ((M * N + 15) / 16 > INT32_MAX) return TSF_ERR_UNSUPPORTED;
     if (is_complex)
       whole_fwd_launch<float2, whole_tc(true, false)>(wf, M * N, L, N, (const float2*)lam, (const float2*)v,
-                                                      (const float2*)x0, (float2*)out, (unsigned*)workspace, s);
+                                                      (const float2*)x0, (float2*)out, (unsigned*)workspace, s, shared);
     else
       whole_fwd_launch<float, whole_tc(false, false)>(wf, M * N, L, N, (const float*)lam, (const float*)v,
-                                                      (const float*)x0, (float*)out, (unsigned*)workspace, s);
+                                                      (const float*)x0, (float*)out, (unsigned*)workspace, s, shared);
     return tsf_launch_status();
   }
   const DiagTile t = const_tile(M * N, L, is_complex != 0, false);
   if (!grid_fits(t)) return TSF_ERR_UNSUPPORTED;
   char* ws = static_cast<char*>(workspace);
   if (is_complex)
-    diag_fwd_launch<float2, 16>(t, (const float2*)lam, (const float2*)v, (const float2*)x0, (float2*)out, ws, L, N, s);
+    diag_fwd_launch<float2, 16>(t, (const float2*)lam, (const float2*)v, (const float2*)x0, (float2*)out, ws, L, N, s,
+                                shared);
   else if (t.TC == 32)
-    diag_fwd_launch<float, 32>(t, (const float*)lam, (const float*)v, (const float*)x0, (float*)out, ws, L, N, s);
+    diag_fwd_launch<float, 32>(t, (const float*)lam, (const float*)v, (const float*)x0, (float*)out, ws, L, N, s, shared);
   else
-    diag_fwd_launch<float, 16>(t, (const float*)lam, (const float*)v, (const float*)x0, (float*)out, ws, L, N, s);
+    diag_fwd_launch<float, 16>(t, (const float*)lam, (const float*)v, (const float*)x0, (float*)out, ws, L, N, s, shared);
   return tsf_launch_status();
 }
 
-int tsfast_hip_diag_bwd(int64_t M, int64_t L, int64_t N, int is_complex, const void* g, const void* lam,
-                        const void* out, const void* x0, void* gv, void* glam, void* gx0, void* workspace,
-                        int64_t workspace_bytes, void* stream) {
+int tsfast_hip_diag_fwd(int64_t M, int64_t L, int64_t N, int is_complex, const void* lam, const void* v,
+                        const void* x0, void* out, void* workspace, int64_t workspace_bytes, void* stream) {
+  return diag_fwd_impl(M, L, N, is_complex, lam, v, x0, out, workspace, workspace_bytes, stream, false);
+}
+
+int64_t tsfast_hip_diag_shared_workspace_bytes(int64_t M, int64_t L, int64_t N, int is_complex) {
+  // whole-sequence tiles keep a term per lane after the header; the look-back's partials are in its words
+  const int64_t base = tsfast_hip_diag_workspace_bytes(M, L, N, is_complex);
+  const int64_t terms = kCounterBytes + M * N * (is_complex ? 16 : 8);
+  return base > terms ? base : terms;
+}
+
+int tsfast_hip_diag_shared_fwd(int64_t M, int64_t L, int64_t N, int is_complex, const void* lam, const void* v,
+                               const void* x0, void* out, void* workspace, int64_t workspace_bytes, void* stream) {
+  return diag_fwd_impl(M, L, N, is_complex, lam, v, x0, out, workspace, workspace_bytes, stream, true);
+}
+
+static int diag_bwd_impl(int64_t M, int64_t L, int64_t N, int is_complex, const void* g, const void* lam,
+                         const void* out, const void* x0, void* gv, void* glam, void* gx0, void* workspace,
+                         int64_t workspace_bytes, void* stream, bool shared) {
   if (M < 0 || L < 0 || N < 0) return TSF_ERR_ARG;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t lanes = M * N;
+  if (shared && lanes == 0 && N > 0) {  // no rows: the shared coefficients' gradient is zero
+    if (!glam) return TSF_ERR_ARG;
+    const int64_t nf = N * (is_complex ? 2 : 1);
+    hipLaunchKernelGGL(zero_fill, grid_for(nf), dim3(256), 0, s, (float*)glam, nf);
+    return tsf_launch_status();
+  }
   if (lanes == 0) return TSF_OK;
   if (!lam || !glam || (x0 && !gx0)) return TSF_ERR_ARG;
   if (L == 0) {
     // empty sequence: every gradient is zero
-    const int64_t nf = lanes * (is_complex ? 2 : 1);
-    hipLaunchKernelGGL(zero_fill, grid_for(nf), dim3(256), 0, s, (float*)glam, nf);
+    const int64_t nf = lanes * (is_complex ? 2 : 1), nl = (shared ? N : lanes) * (is_complex ? 2 : 1);
+    hipLaunchKernelGGL(zero_fill, grid_for(nl), dim3(256), 0, s, (float*)glam, nl);
     if (gx0) hipLaunchKernelGGL(zero_fill, grid_for(nf), dim3(256), 0, s, (float*)gx0, nf);
     return tsf_launch_status();
   }
   if (!g || !out || !gv) return TSF_ERR_ARG;
-  if (workspace_bytes < tsfast_hip_diag_workspace_bytes(M, L, N, is_complex) || !workspace) return TSF_ERR_WORKSPACE;
+  const int64_t need = shared ? tsfast_hip_diag_shared_workspace_bytes(M, L, N, is_complex)
+                              : tsfast_hip_diag_workspace_bytes(M, L, N, is_complex);
+  if (workspace_bytes < need || !workspace) return TSF_ERR_WORKSPACE;
   const WholeTile wb = whole_tile(lanes, L, whole_tc(is_complex != 0, true), true);
   if (wb.kmax > 0) {
     if ((lanes + 15) / 16 > INT32_MAX) return TSF_ERR_UNSUPPORTED;
     if (is_complex)
       whole_bwd_launch<float2, whole_tc(true, true)>(wb, lanes, L, N, (const float2*)lam, (const float2*)g,
                                                      (const float2*)out, (const float2*)x0, (float2*)gv,
-                                                     (float2*)glam, (float2*)gx0, (unsigned*)workspace, s);
+                                                     (float2*)glam, (float2*)gx0, (unsigned*)workspace, s, shared);
     else
       whole_bwd_launch<float, whole_tc(false, true)>(wb, lanes, L, N, (const float*)lam, (const float*)g,
                                                      (const float*)out, (const float*)x0, (float*)gv, (float*)glam,
-                                                     (float*)gx0, (unsigned*)workspace, s);
+                                                     (float*)gx0, (unsigned*)workspace, s, shared);
     return tsf_launch_status();
   }
   const DiagTile t = const_tile(lanes, L, is_complex != 0, true);
@@ -1150,14 +1215,26 @@ int tsfast_hip_diag_bwd(int64_t M, int64_t L, int64_t N, int is_complex, const v
   char* ws = static_cast<char*>(workspace);
   if (is_complex)
     diag_bwd_launch<float2, 16>(t, (const float2*)g, (const float2*)lam, (const float2*)out, (const float2*)x0,
-                                (float2*)gv, (float2*)glam, (float2*)gx0, ws, L, N, s);
+                                (float2*)gv, (float2*)glam, (float2*)gx0, ws, L, N, s, shared);
   else if (t.TC == 32)
     diag_bwd_launch<float, 32>(t, (const float*)g, (const float*)lam, (const float*)out, (const float*)x0, (float*)gv,
-                               (float*)glam, (float*)gx0, ws, L, N, s);
+                               (float*)glam, (float*)gx0, ws, L, N, s, shared);
   else
     diag_bwd_launch<float, 16>(t, (const float*)g, (const float*)lam, (const float*)out, (const float*)x0, (float*)gv,
-                               (float*)glam, (float*)gx0, ws, L, N, s);
+                               (float*)glam, (float*)gx0, ws, L, N, s, shared);
   return tsf_launch_status();
+}
+
+int tsfast_hip_diag_bwd(int64_t M, int64_t L, int64_t N, int is_complex, const void* g, const void* lam,
+                        const void* out, const void* x0, void* gv, void* glam, void* gx0, void* workspace,
+                        int64_t workspace_bytes, void* stream) {
+  return diag_bwd_impl(M, L, N, is_complex, g, lam, out, x0, gv, glam, gx0, workspace, workspace_bytes, stream, false);
+}
+
+int tsfast_hip_diag_shared_bwd(int64_t M, int64_t L, int64_t N, int is_complex, const void* g, const void* lam,
+                               const void* out, const void* x0, void* gv, void* glam, void* gx0, void* workspace,
+                               int64_t workspace_bytes, void* stream) {
+  return diag_bwd_impl(M, L, N, is_complex, g, lam, out, x0, gv, glam, gx0, workspace, workspace_bytes, stream, true);
 }
 
 int64_t tsfast_hip_diag_noalloc_max_bytes(void) { return kNoAllocScratchBytes; }

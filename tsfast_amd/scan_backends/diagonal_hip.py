@@ -28,11 +28,11 @@ def supports(lam: torch.Tensor, v: torch.Tensor, x0: torch.Tensor | None) -> str
         return f"lam dtype {lam.dtype} != v dtype {v.dtype}"
     if x0 is not None and x0.dtype != v.dtype:
         return f"x0 dtype {x0.dtype} != v dtype {v.dtype}"
-    if v.dim() != 3 or lam.dim() != 2:
-        return "expects the lane layout lam [M, N], v [M, L, N]"
-    if tuple(lam.shape) != (v.shape[0], v.shape[2]):
+    if v.dim() != 3 or lam.dim() not in (1, 2):
+        return "expects the lane layout lam [M, N] (or one row [N]), v [M, L, N]"
+    if tuple(lam.shape) not in ((v.shape[0], v.shape[2]), (v.shape[2],)):
         return f"lam {tuple(lam.shape)} does not match v {tuple(v.shape)}"
-    if x0 is not None and tuple(x0.shape) != tuple(lam.shape):
+    if x0 is not None and tuple(x0.shape) != (v.shape[0], v.shape[2]):
         return f"x0 {tuple(x0.shape)} does not match lam {tuple(lam.shape)}"
     if any(t.device != v.device for t in (lam, x0) if t is not None):
         return "inputs on different devices"
@@ -41,19 +41,24 @@ def supports(lam: torch.Tensor, v: torch.Tensor, x0: torch.Tensor | None) -> str
     return None
 
 
+def _entry(name: str, shared: bool):
+    return getattr(_lib.load(), f"tsfast_hip_diag_{'shared_' if shared else ''}{name}")
+
+
 def forward(lam: torch.Tensor, v: torch.Tensor, x0: torch.Tensor | None) -> torch.Tensor:
-    """Forward recurrence on the lane layout; returns the states ``[M, L, N]``."""
-    lib = _lib.load()
+    """Forward recurrence on the lane layout; returns the states ``[M, L, N]``. A one-dimensional
+    ``lam [N]`` is one coefficient row for every batch row."""
     _lib.sync_deterministic()
     M, L, N = v.shape
+    shared = lam.dim() == 1
     for name, t in (("lam", lam), ("v", v), ("x0", x0)):
         _lib.require(t, name, (v.dtype,), v.device)
     cplx = int(v.is_complex())
     out = torch.empty_like(v)
-    nbytes = lib.tsfast_hip_diag_workspace_bytes(M, L, N, cplx)
+    nbytes = _entry("workspace_bytes", shared)(M, L, N, cplx)
     ws = _lib.workspace(nbytes, v.device)
     _lib.check(
-        lib.tsfast_hip_diag_fwd(
+        _entry("fwd", shared)(
             M, L, N, cplx, _lib.ptr(lam), _lib.ptr(v), _lib.ptr(x0), _lib.ptr(out), _lib.ptr(ws), nbytes,
             _lib.stream_of(v),
         ),
@@ -66,20 +71,21 @@ def forward(lam: torch.Tensor, v: torch.Tensor, x0: torch.Tensor | None) -> torc
 def backward(
     g: torch.Tensor, lam: torch.Tensor, out: torch.Tensor, x0: torch.Tensor | None
 ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    """Adjoint sweep, returning ``(glam, gv, gx0)`` (gx0 empty when x0 is None)."""
-    lib = _lib.load()
+    """Adjoint sweep, returning ``(glam, gv, gx0)`` (gx0 empty when x0 is None; glam summed over the
+    batch rows for a one-dimensional ``lam``)."""
     _lib.sync_deterministic()
     M, L, N = out.shape
+    shared = lam.dim() == 1
     for name, t in (("g", g), ("lam", lam), ("out", out), ("x0", x0)):
         _lib.require(t, name, (out.dtype,), out.device)
     cplx = int(out.is_complex())
     gv = torch.empty_like(out)
     glam = torch.empty_like(lam)
-    gx0 = torch.empty_like(lam) if x0 is not None else None
-    nbytes = lib.tsfast_hip_diag_workspace_bytes(M, L, N, cplx)
+    gx0 = lam.new_empty(M, N) if x0 is not None else None
+    nbytes = _entry("workspace_bytes", shared)(M, L, N, cplx)
     ws = _lib.workspace(nbytes, out.device)
     _lib.check(
-        lib.tsfast_hip_diag_bwd(
+        _entry("bwd", shared)(
             M, L, N, cplx, _lib.ptr(g), _lib.ptr(lam), _lib.ptr(out), _lib.ptr(x0), _lib.ptr(gv), _lib.ptr(glam),
             _lib.ptr(gx0), _lib.ptr(ws), nbytes, _lib.stream_of(out),
         ),
