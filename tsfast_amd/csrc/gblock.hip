@@ -652,12 +652,26 @@ __global__ void __launch_bounds__(1024) gblock_finish_lane(
   const int64_t rl = lane / Pp * P + p;  // the caller's [B, P, na] row
   const int64_t seg = (n + 15) / 16;
   const int64_t r0 = k * seg, r1 = (r0 + seg < n) ? r0 + seg : n;
+  // every value of a super-chunk in one pass over them: all its loads in flight together (a pass per
+  // value, each load waiting on the one before, took 6 us longer: 403 -> 397 us for the backward of 64 rows
+  // of 8 x 8 channels x 16384 steps)
+  double acc[NA + NBT];
+#pragma unroll
+  for (int q = 0; q < NA + NBT; ++q) acc[q] = 0.0;
+  if (live) {
+#pragma unroll 2
+    for (int64_t r = r0; r < r1; ++r) {
+      const double* pa = part_ga + (r * lanes + lane) * NA;
+      const double* pb = part_gb + (r * lanes + lane) * NBT;
+#pragma unroll
+      for (int q = 0; q < NA; ++q) acc[q] += pa[q];
+#pragma unroll
+      for (int q = 0; q < NBT; ++q) acc[NA + q] += pb[q];
+    }
+  }
+#pragma unroll
   for (int q = 0; q < NA + NBT; ++q) {
-    double acc = 0.0;
-    if (live)
-      for (int64_t r = r0; r < r1; ++r)
-        acc += q < NA ? part_ga[(r * lanes + lane) * NA + q] : part_gb[(r * lanes + lane) * NBT + (q - NA)];
-    s_p[k][lid] = acc;
+    s_p[k][lid] = acc[q];
     __syncthreads();
     if (k == 0) {
       double t = s_p[0][lid];

@@ -136,16 +136,18 @@ def _gblock_bwd_op(
     _lib.require(g_xlast, "g_xlast", (torch.float32,), u.device)
     B, L, I, O, nb, na = _dims(u, b, a)
     gu = torch.empty_like(u)
-    gu_tail = torch.zeros(B, nb - 1, I, device=u.device, dtype=torch.float32)
     gb = torch.empty_like(b)
     ga = torch.empty_like(a)
-    gx0 = torch.empty(B, I * O, na, device=u.device, dtype=torch.float32)
+    # absent initial conditions have no gradient: an empty tensor, and NULL to the kernels
+    gu_tail = torch.zeros_like(u_tail) if u_tail is not None else u.new_empty(0)
+    gx0 = torch.empty_like(x0) if x0 is not None else u.new_empty(0)
     ws, nbytes = _workspace(lib, u, b, a)
     _lib.check(
         lib.tsfast_hip_gblock_bwd(
             B, L, I, O, nb, na, _lib.ptr(gy), _lib.ptr(g_xlast), _lib.ptr(u), _lib.ptr(b), _lib.ptr(a),
-            _lib.ptr(u_tail), _lib.ptr(x0), _lib.ptr(saved), _lib.ptr(gu), _lib.ptr(gu_tail), _lib.ptr(gb),
-            _lib.ptr(ga), _lib.ptr(gx0), _lib.ptr(ws), nbytes, _lib.stream_of(u),
+            _lib.ptr(u_tail), _lib.ptr(x0), _lib.ptr(saved), _lib.ptr(gu),
+            _lib.ptr(gu_tail if u_tail is not None else None), _lib.ptr(gb), _lib.ptr(ga),
+            _lib.ptr(gx0 if x0 is not None else None), _lib.ptr(ws), nbytes, _lib.stream_of(u),
         ),
         "tsfast_hip_gblock_bwd",
     )
@@ -155,11 +157,8 @@ def _gblock_bwd_op(
 
 @_gblock_bwd_op.register_fake
 def _(gy, g_xlast, u, b, a, u_tail, x0, saved):
-    B, _, I = u.shape
-    O, _, nb = b.shape
-    na = a.shape[-1]
-    return (torch.empty_like(u), u.new_empty(B, nb - 1, I), torch.empty_like(b), torch.empty_like(a),
-            u.new_empty(B, I * O, na))
+    return (torch.empty_like(u), u.new_empty(0) if u_tail is None else torch.empty_like(u_tail), torch.empty_like(b),
+            torch.empty_like(a), u.new_empty(0) if x0 is None else torch.empty_like(x0))
 
 
 def _gblock_setup(ctx, inputs, output):
