@@ -132,3 +132,28 @@ def test_conv_supports_reasons(gpu):
     assert "kernel width" in conv_hip.supports(x, torch.randn(2, 8, 8, device=gpu), torch.randn(8, 1, 9, device=gpu), None)
     assert "tail.shape" in conv_hip.supports(x, torch.randn(2, 8, 2, device=gpu), w, None)
     assert "GPU-only" in conv_hip.supports(x.cpu(), tail.cpu(), w.cpu(), None)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("K", [2, 4, 5])
+@pytest.mark.parametrize("D", [3, 4, 5, 7, 8, 9, 17, 254, 255, 257, 263, 509])
+def test_conv_rows_of_any_alignment(gpu, D, K, dtype):
+    """16-byte pieces at any alignment (channel stride 1) against the element path (any other channel
+    stride): the same arithmetic in the same order, so the same bits. The view ends where its storage
+    ends, and its rows start at every alignment; widths from under one piece to several blocks."""
+    B, L, off = 2, 131, 1
+    g = torch.Generator().manual_seed(D * 10 + K)
+    wide = torch.randn(B, L, off + D, generator=g).to(gpu, dtype)
+    rows = wide[..., off:]
+    columns = rows.transpose(1, 2).contiguous().transpose(1, 2)
+    tail = torch.randn(B, D, K - 1, generator=g).to(gpu, dtype)
+    weight, bias = (torch.randn(D, 1, K, generator=g) * 0.5).to(gpu), torch.randn(D, generator=g).to(gpu)
+    gy = torch.randn(B, L, D, generator=g).to(gpu, dtype)
+    results = []
+    for x in (rows, columns):
+        assert x.stride(2) == 1 or x is columns
+        leaves = [t.detach().requires_grad_() for t in (x, tail, weight, bias)]
+        y = conv_hip.run(*leaves)
+        results.append((y, *torch.autograd.grad(y, leaves, gy)))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)

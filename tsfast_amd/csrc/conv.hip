@@ -13,8 +13,8 @@
 //    the whole run plus its K-1 step halo in registers, loaded before the arithmetic.
 //  * bf16: a 16-byte vector holds 8 channels, too many for register tiles, so a workgroup owns
 //    256 consecutive channels (one per thread) of one batch row over a segment of kSeg steps.
-//    Row tiles are moved into LDS with 16-byte vector loads (element loads for layouts without
-//    aligned rows), and the next tile's loads are in flight while the current tile is computed.
+//    Row tiles are moved into LDS with 16-byte vector loads at any alignment (element loads for
+//    channel strides other than 1), and the next tile's loads are in flight while the current tile is computed.
 //    Each thread walks its channel's column with K-step rolling windows in registers (tile rows
 //    are a multiple of K, so ring slots are compile-time), so its registers hold only the windows,
 //    taps and partial sums and many waves stay resident.
@@ -68,10 +68,40 @@ struct alignas(16) Piece {
   TIO v[VE];
 };
 
+// 16 bytes at element offset o of a row base (32-bit byte offsets from a workgroup-uniform base),
+// aligned to its elements only: a global access of this target needs no more, whatever its width.
+template <typename TIO>
+struct Raw16;
+template <>
+struct Raw16<float> {
+  typedef uint32_t T __attribute__((ext_vector_type(4), aligned(4), may_alias));
+};
+template <>
+struct Raw16<bf16> {
+  typedef uint32_t T __attribute__((ext_vector_type(4), aligned(2), may_alias));
+};
+template <typename P, typename TIO>
+TSF_DEV P ld16(const TIO* base, uint32_t o) {
+  using T = typename Raw16<TIO>::T;
+  const char* p = reinterpret_cast<const char*>(base) + o * (uint32_t)sizeof(TIO);
+  return __builtin_bit_cast(P, *reinterpret_cast<const T*>(p));
+}
+template <typename P, typename TIO>
+TSF_DEV void st16(TIO* base, uint32_t o, const P& v) {
+  using T = typename Raw16<TIO>::T;
+  *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + o * (uint32_t)sizeof(TIO)) = __builtin_bit_cast(T, v);
+}
+
 // A tile of TR rows x kCh channels of one tensor, staged through registers: thread t handles
-// pieces e = t + q * kCh (row e / PPR, piece e % PPR). Rows outside [0, L) and channels past D
-// read as zero. VECL: rows are 16-byte aligned runs (channel stride 1, D a multiple of VE), so a
-// piece is one vector load; otherwise its elements are loaded one by one.
+// pieces e = t + q * kCh (row e / PPR, piece e % PPR). Rows outside [0, L) read as zero; what a tile
+// holds in channels past D is never used. How the rows lie decides how a piece moves:
+//  kAligned: whole 16-byte aligned pieces, one vector access each.
+//  kRuns: runs (channel stride 1) of at least one piece, at any alignment: one unaligned vector access
+//    each. These went by elements before: at 16 x 4096 steps, bf16, K 4, forward and forward + backward
+//    took 142 and 478 us at D 1531, now 111 and 292. Aligned rows taken this way would run at 91 and
+//    251 us, against 85 and 228 at D 1536.
+//  kElements: any strides, element by element.
+enum Rows { kAligned, kRuns, kElements };
 template <typename TIO, int TR>
 struct TileRegs2 {
   static constexpr int VE = Piece<TIO>::VE;
@@ -82,7 +112,7 @@ struct TileRegs2 {
 
 // Issue the loads of stream rows [s0, s0 + TR) (sequence rows; row s at base + s * sl + c * sc for
 // channel c) into the staging registers.
-template <typename TIO, int TR, bool VECL>
+template <typename TIO, int TR, Rows ROWS>
 TSF_DEV void tile_issue(TileRegs2<TIO, TR>& rg, const TIO* __restrict__ base, int64_t s0, int64_t L, int64_t c0,
                         int64_t D, int64_t sl, int64_t sc) {
   using R = TileRegs2<TIO, TR>;
@@ -92,13 +122,21 @@ TSF_DEV void tile_issue(TileRegs2<TIO, TR>& rg, const TIO* __restrict__ base, in
     const int row = e / R::PPR, pc = e % R::PPR;
     const int64_t srow = s0 + row, c = c0 + (int64_t)pc * R::VE;
     const bool rok = e < TR * R::PPR && srow >= 0 && srow < L;
-    if (VECL) {
+    if (ROWS == kAligned) {
       if (rok && c < D) {
         rg.r[q] = ld32(reinterpret_cast<const Piece<TIO>*>(base), (uint32_t)((srow * sl + c) / R::VE));
       } else {
 #pragma unroll
         for (int v = 0; v < R::VE; ++v) rg.r[q].v[v] = zero_io<TIO>();
       }
+    } else if (ROWS == kRuns) {
+      const int back = c + R::VE > D ? (int)(c + R::VE - D) : 0;  // a row's last piece ends at D ...
+      unsigned __int128 v = 0;
+      if (rok && c < D) {
+        v = ld16<unsigned __int128>(base, (uint32_t)(srow * sl + c - back));
+        if (back) v >>= back * 8 * (int)sizeof(TIO);  // ... and gives up what belongs to the one before
+      }
+      rg.r[q] = __builtin_bit_cast(Piece<TIO>, v);
     } else {
 #pragma unroll
       for (int v = 0; v < R::VE; ++v)
@@ -119,7 +157,7 @@ TSF_DEV void tile_commit(const TileRegs2<TIO, TR>& rg, TIO (*tile)[kCh]) {
 
 // Store tile rows r (r0 <= r < r1) as sequence rows s0 + r of a contiguous [*, L, D] row source
 // (dst = its batch row), channels past D skipped; the same piece mapping as tile_issue.
-template <typename TIO, int TR, bool VECL>
+template <typename TIO, int TR, Rows ROWS>
 TSF_DEV void tile_store(TIO (*tile)[kCh], TIO* __restrict__ dst, int64_t s0, int r0, int r1, int64_t c0, int64_t D) {
   using R = TileRegs2<TIO, TR>;
 #pragma unroll
@@ -130,8 +168,10 @@ TSF_DEV void tile_store(TIO (*tile)[kCh], TIO* __restrict__ dst, int64_t s0, int
     if (e < TR * R::PPR && row >= r0 && row < r1) {
       const Piece<TIO> v = *reinterpret_cast<const Piece<TIO>*>(&tile[row][pc * R::VE]);
       const int64_t o = (s0 + row) * D + c;
-      if (VECL) {
+      if (ROWS == kAligned) {
         if (c < D) st32(reinterpret_cast<Piece<TIO>*>(dst), (uint32_t)(o / R::VE), v);
+      } else if (ROWS == kRuns && c + R::VE <= D) {
+        st16(dst, (uint32_t)o, v);
       } else {
 #pragma unroll
         for (int u = 0; u < R::VE; ++u)
@@ -164,7 +204,7 @@ TSF_DEV Wg3 wg3(uint32_t nx, uint32_t ny) {
 }
 
 // ------------------------------------------------------------------------------------ forward
-template <typename TIO, int K, bool VECL>
+template <typename TIO, int K, Rows ROWS>
 __global__ void __launch_bounds__(kCh) conv_silu_fwd_kernel(const TIO* __restrict__ x, const TIO* __restrict__ tail,
                                                             const float* __restrict__ w,
                                                             const float* __restrict__ bias, TIO* __restrict__ out,
@@ -192,14 +232,31 @@ __global__ void __launch_bounds__(kCh) conv_silu_fwd_kernel(const TIO* __restric
     if (live) xr[k] = xbuf_at<TIO, K>(xrow, tail, b, t0 - K + k, d, L, D, sxl, sxd);
   TIO* orow = out + b * L * D;
   TileRegs2<TIO, TR> rg;
-  tile_issue<TIO, TR, VECL>(rg, xrow, t0, L, c0, D, sxl, sxd);
+  tile_issue<TIO, TR, ROWS>(rg, xrow, t0, L, c0, D, sxl, sxd);
   const bool all_live = c0 + kCh <= D;  // uniform over the workgroup
   for (int64_t jb = 0; jb < nrow; jb += TR) {
     __syncthreads();
     tile_commit<TIO, TR>(rg, s_x);
     __syncthreads();
-    if (jb + TR < nrow) tile_issue<TIO, TR, VECL>(rg, xrow, t0 + jb + TR, L, c0, D, sxl, sxd);
-    if (all_live && jb + TR <= nrow) {
+    if (jb + TR < nrow) tile_issue<TIO, TR, ROWS>(rg, xrow, t0 + jb + TR, L, c0, D, sxl, sxd);
+    if (ROWS == kRuns) {
+      // rows that start anywhere: a wave's 128-byte store would straddle two lines, so outputs take their
+      // inputs' places in the tile and leave by pieces (111 us against 127 stored by lane, D 1531; aligned
+      // rows are faster stored by lane, below)
+#pragma unroll 1
+      for (int i0 = 0; i0 < TR; i0 += K) {
+#pragma unroll
+        for (int r = 0; r < K; ++r) {
+          xr[r] = to_f32(s_x[i0 + r][tid]);
+          float p = bv;
+#pragma unroll
+          for (int k = 0; k < K; ++k) p = fmaf(wk[k], xr[(r + 1 + k) % K], p);
+          s_x[i0 + r][tid] = from_f32<TIO>(silu_f(p));
+        }
+      }
+      __syncthreads();
+      tile_store<TIO, TR, ROWS>(s_x, orow, t0 + jb, 0, nrow - jb < TR ? (int)(nrow - jb) : TR, c0, D);
+    } else if (all_live && jb + TR <= nrow) {
       // a whole tile of a fully live workgroup: no per-step exit or store mask. Groups of K steps
       // (TR is a multiple of K, so a step's ring slot is its place in the group) in a loop that is
       // not unrolled: unrolled over the whole tile, the compiler hoisted the later steps' reads
@@ -236,7 +293,7 @@ __global__ void __launch_bounds__(kCh) conv_silu_fwd_kernel(const TIO* __restric
 // A segment streams rows t0 .. t0+kSeg+K-2 (the last K-1 give the gpre that its own last gx
 // rows need); gx of row j - (K-1) is formed once gpre_j is known. One partial row per (batch,
 // segment): part [B, nseg, D, K+1] (K taps, then the bias term).
-template <typename TIO, int K, bool VECL>
+template <typename TIO, int K, Rows ROWS>
 __global__ void __launch_bounds__(kCh) conv_silu_bwd_kernel(
     const TIO* __restrict__ x, const TIO* __restrict__ tail, const float* __restrict__ w,
     const float* __restrict__ bias, const TIO* __restrict__ gy, TIO* __restrict__ gx, TIO* __restrict__ gtail,
@@ -270,16 +327,16 @@ __global__ void __launch_bounds__(kCh) conv_silu_bwd_kernel(
   for (int k = 1; k < K; ++k)
     if (live) xr[k] = xbuf_at<TIO, K>(xrow, tail, b, t0 - K + k, d, L, D, sxl, sxd);
   TileRegs2<TIO, TR> rx, rgy;
-  tile_issue<TIO, TR, VECL>(rx, xrow, t0, L, c0, D, sxl, sxd);
-  tile_issue<TIO, TR, VECL>(rgy, gyrow, t0, L, c0, D, D, 1);
+  tile_issue<TIO, TR, ROWS>(rx, xrow, t0, L, c0, D, sxl, sxd);
+  tile_issue<TIO, TR, ROWS>(rgy, gyrow, t0, L, c0, D, D, 1);
   for (int64_t jb = 0; jb < nrow; jb += TR) {
     __syncthreads();
     tile_commit<TIO, TR>(rx, s_x);
     tile_commit<TIO, TR>(rgy, s_g);
     __syncthreads();
     if (jb + TR < nrow) {
-      tile_issue<TIO, TR, VECL>(rx, xrow, t0 + jb + TR, L, c0, D, sxl, sxd);
-      tile_issue<TIO, TR, VECL>(rgy, gyrow, t0 + jb + TR, L, c0, D, D, 1);
+      tile_issue<TIO, TR, ROWS>(rx, xrow, t0 + jb + TR, L, c0, D, sxl, sxd);
+      tile_issue<TIO, TR, ROWS>(rgy, gyrow, t0 + jb + TR, L, c0, D, D, 1);
     }
 #pragma unroll
     for (int i = 0; i < TR; ++i) {
@@ -320,7 +377,7 @@ __global__ void __launch_bounds__(kCh) conv_silu_bwd_kernel(
     {
       const int64_t lo = (K - 1) - jb, hi = own + (K - 1) - jb;
       const int r0 = lo > 0 ? (int)lo : 0, r1 = hi < TR ? (int)(hi > 0 ? hi : 0) : TR;
-      tile_store<TIO, TR, VECL>(s_g, gxrow, t0 + jb - (K - 1), r0, r1, c0, D);
+      tile_store<TIO, TR, ROWS>(s_g, gxrow, t0 + jb - (K - 1), r0, r1, c0, D);
     }
   }
   if (live) {
@@ -339,18 +396,13 @@ constexpr int kRun = 16;   // forward steps per thread
 constexpr int kCgWg = 64;  // channel groups per workgroup (one wave wide)
 constexpr int kRunsWg = 4; // runs per workgroup (one per wave)
 
-// VEC consecutive channels of one row: one vector access when the row is contiguous.
-template <typename TIO, int VEC>
-struct alignas(sizeof(TIO) * VEC) Vec {
-  TIO v[VEC];
-};
-
 // VEC channels at element offset o of a row base (32-bit byte offsets from a workgroup-uniform
 // base: the SGPR-base + VGPR-offset address form, no 64-bit arithmetic per access).
 template <typename TIO, int VEC>
 TSF_DEV void load_vec(float (&dst)[VEC], const TIO* base, uint32_t o) {
   if (VEC > 1) {
-    const Vec<TIO, VEC> r = ld32(reinterpret_cast<const Vec<TIO, VEC>*>(base), o / VEC);
+    static_assert(VEC == 1 || VEC * sizeof(TIO) == 16);
+    const Piece<TIO> r = ld16<Piece<TIO>>(base, o);
 #pragma unroll
     for (int c = 0; c < VEC; ++c) dst[c] = to_f32(r.v[c]);
   } else {
@@ -361,17 +413,25 @@ TSF_DEV void load_vec(float (&dst)[VEC], const TIO* base, uint32_t o) {
 template <typename TIO, int VEC>
 TSF_DEV void store_vec(TIO* base, uint32_t o, const float (&src)[VEC]) {
   if (VEC > 1) {
-    Vec<TIO, VEC> r;
+    Piece<TIO> r;
 #pragma unroll
     for (int c = 0; c < VEC; ++c) r.v[c] = from_f32<TIO>(src[c]);
-    st32(reinterpret_cast<Vec<TIO, VEC>*>(base), o / VEC, r);
+    st16(base, o, r);
   } else {
     st32(base, o, from_f32<TIO>(src[0]));
   }
 }
 
 
-// Thread coordinates: channel group cg (VEC channels from d0 = cg * VEC), run r, batch row b.
+// First channel of group cg: VEC channels each, the last group moved back to end at D (the channels it
+// shares with the group before are formed twice, alike, instead of by elements behind guards; D >= VEC).
+template <int VEC>
+TSF_DEV int64_t first_channel(int64_t cg, int64_t D) {
+  const int64_t d0 = cg * VEC;
+  return VEC == 1 || d0 + VEC <= D ? d0 : D - VEC;
+}
+
+// Thread coordinates: channel group cg (VEC channels from d0), run r, batch row b.
 struct Coord {
   int64_t b, run, d0;
   bool live;
@@ -385,7 +445,7 @@ TSF_DEV Coord coord(int64_t D, int64_t runs, uint32_t nx, uint32_t ny) {
   Coord c;
   c.b = wg.z;
   c.run = run;
-  c.d0 = cg * VEC;
+  c.d0 = first_channel<VEC>(cg, D);
   c.live = cg < cgs && run < runs;
   return c;
 }
@@ -467,7 +527,7 @@ __global__ void __launch_bounds__(kCgWg* kRunsWg) conv_silu_bwd_reg(
   const Wg3 wg = wg3(nx, ny);
   const int64_t cg = wg.x * kCgWg + ln;
   const int64_t b = wg.z;
-  const int64_t d0 = cg * VEC;
+  const int64_t d0 = first_channel<VEC>(cg, D);
   const int64_t run0 = (wg.y * kRunsWg + wv) * kRpt;
   const TIO* xrow = x + b * sxb;
   const TIO* gyrow = gy + b * L * D;
@@ -553,13 +613,14 @@ __global__ void __launch_bounds__(kCgWg* kRunsWg) conv_silu_bwd_reg(
     for (int ch = 0; ch < VEC; ++ch) s_part[wv][k][ln * VEC + ch] = acc[k][ch];
   __syncthreads();
   const int64_t groups = ny;
+  const int64_t rest = D % VEC;  // channels of a last group that was moved back: they are its last ones
   for (int idx = threadIdx.x; idx < KP * kCgWg * VEC; idx += kCgWg * kRunsWg) {
     const int k = idx / (kCgWg * VEC), dd = idx % (kCgWg * VEC);
     const int64_t d = wg.x * kCgWg * VEC + dd;
     if (d < D) {
       float s = 0.0f;
 #pragma unroll
-      for (int r = 0; r < kRunsWg; ++r) s += s_part[r][k][dd];
+      for (int r = 0; r < kRunsWg; ++r) s += s_part[r][k][d < D - rest ? dd : dd + VEC - (int)rest];
       part[(wg.z * groups + wg.y) * D * KP + d * KP + k] = s;
     }
   }
@@ -613,43 +674,40 @@ ConvPlan conv_plan(int64_t L, int64_t D) {
   return p;
 }
 
-// Whole 16-byte pieces per tile row: channel stride 1, D and the row strides multiples of the
-// piece, 16-byte aligned bases (y, z: the contiguous [B, L, D] tensors read or written the same
-// way, or NULL).
+// y, z: the contiguous [B, L, D] tensors read or written the same way, or NULL.
 template <typename TIO>
-bool vec_rows(const void* x, int64_t D, int64_t sxb, int64_t sxl, int64_t sxd, const void* y, const void* z) {
+Rows rows_of(const void* x, int64_t D, int64_t sxb, int64_t sxl, int64_t sxd, const void* y, const void* z) {
   constexpr int64_t VE = 16 / sizeof(TIO);
   const uintptr_t a = (uintptr_t)x | (uintptr_t)y | (uintptr_t)z;
-  return sxd == 1 && D % VE == 0 && sxl % VE == 0 && sxb % VE == 0 && a % 16 == 0;
+  if (sxd != 1 || D < VE) return kElements;
+  return D % VE == 0 && sxl % VE == 0 && sxb % VE == 0 && a % 16 == 0 ? kAligned : kRuns;
 }
 
 template <typename TIO, int K>
-void fwd_k(bool vec, int64_t B, int64_t L, int64_t D, const void* x, int64_t sxb, int64_t sxl, int64_t sxd,
+void fwd_k(Rows rows, int64_t B, int64_t L, int64_t D, const void* x, int64_t sxb, int64_t sxl, int64_t sxd,
            const void* tail, const float* w, const float* bias, void* out, hipStream_t s) {
   const ConvPlan p = conv_plan(L, D);
   const dim3 grid((unsigned)(p.cblocks * p.nseg * B));
   const uint32_t nx = (uint32_t)p.cblocks, ny = (uint32_t)p.nseg;
-  if (vec)
-    hipLaunchKernelGGL((conv_silu_fwd_kernel<TIO, K, true>), grid, dim3(kCh), 0, s, (const TIO*)x, (const TIO*)tail, w,
-                       bias, (TIO*)out, L, D, sxb, sxl, sxd, nx, ny);
-  else
-    hipLaunchKernelGGL((conv_silu_fwd_kernel<TIO, K, false>), grid, dim3(kCh), 0, s, (const TIO*)x, (const TIO*)tail,
-                       w, bias, (TIO*)out, L, D, sxb, sxl, sxd, nx, ny);
+  auto* const kernel = rows == kAligned ? conv_silu_fwd_kernel<TIO, K, kAligned>
+                       : rows == kRuns  ? conv_silu_fwd_kernel<TIO, K, kRuns>
+                                        : conv_silu_fwd_kernel<TIO, K, kElements>;
+  hipLaunchKernelGGL(kernel, grid, dim3(kCh), 0, s, (const TIO*)x, (const TIO*)tail, w, bias, (TIO*)out, L, D, sxb,
+                     sxl, sxd, nx, ny);
 }
 
 template <typename TIO, int K>
-void bwd_k(bool vec, int64_t B, int64_t L, int64_t D, const void* x, int64_t sxb, int64_t sxl, int64_t sxd,
+void bwd_k(Rows rows, int64_t B, int64_t L, int64_t D, const void* x, int64_t sxb, int64_t sxl, int64_t sxd,
            const void* tail, const float* w, const float* bias, const void* gy, void* gx, void* gtail, float* gw,
            float* gb, float* part, hipStream_t s) {
   const ConvPlan p = conv_plan(L, D);
   const dim3 grid((unsigned)(p.cblocks * p.nseg * B));
   const uint32_t nx = (uint32_t)p.cblocks, ny = (uint32_t)p.nseg;
-  if (vec)
-    hipLaunchKernelGGL((conv_silu_bwd_kernel<TIO, K, true>), grid, dim3(kCh), 0, s, (const TIO*)x, (const TIO*)tail, w,
-                       bias, (const TIO*)gy, (TIO*)gx, (TIO*)gtail, part, L, D, sxb, sxl, sxd, nx, ny);
-  else
-    hipLaunchKernelGGL((conv_silu_bwd_kernel<TIO, K, false>), grid, dim3(kCh), 0, s, (const TIO*)x, (const TIO*)tail,
-                       w, bias, (const TIO*)gy, (TIO*)gx, (TIO*)gtail, part, L, D, sxb, sxl, sxd, nx, ny);
+  auto* const kernel = rows == kAligned ? conv_silu_bwd_kernel<TIO, K, kAligned>
+                       : rows == kRuns  ? conv_silu_bwd_kernel<TIO, K, kRuns>
+                                        : conv_silu_bwd_kernel<TIO, K, kElements>;
+  hipLaunchKernelGGL(kernel, grid, dim3(kCh), 0, s, (const TIO*)x, (const TIO*)tail, w, bias, (const TIO*)gy, (TIO*)gx,
+                     (TIO*)gtail, part, L, D, sxb, sxl, sxd, nx, ny);
   const int64_t n = D * (K + 1);
   hipLaunchKernelGGL(conv_reduce_params, dim3((unsigned)((n + 63) / 64)), dim3(64 * kRedWaves), 0, s,
                      (const float*)part, gw, gb, B * p.nseg, D, K);
@@ -668,13 +726,18 @@ RegPlan reg_plan(int64_t L, int64_t D, int vec, int run_len, int runs_per_group)
   return p;
 }
 
-// Vector width 4 (both passes) when every row of x and of the contiguous outputs is a 16-byte-aligned run of
-// whole channel groups; the tail, weights and bias are read per channel either way.
-template <typename TIO>
-int vec_for(const void* x, int64_t D, int64_t sxb, int64_t sxl, int64_t sxd, const void* y) {
-  const uintptr_t a = (uintptr_t)x | (uintptr_t)y;
-  const bool ok = sxd == 1 && D % 4 == 0 && sxl % 4 == 0 && sxb % 4 == 0 && a % (4 * sizeof(TIO)) == 0;
-  return ok ? 4 : 1;
+// Vector width 4 (both passes) when rows of x are runs of at least one channel group. Rows that are not
+// whole aligned groups went one channel a thread before: at 16 x 4096 steps, D 1531, K 4, forward and
+// forward + backward took 233 and 568 us, now 185 and 480 (157 and 407 at D 1536). They still do where the
+// wider groups would leave more than a third of the lanes without a channel: 170 us against 192 at 50 x
+// 2000 steps, D 303 (320 lanes of one channel, or 128 of four for 76 groups), K 3. The tail, weights and
+// bias are read per channel either way.
+int vec_for(const void* x, int64_t D, int64_t sxb, int64_t sxl, int64_t sxd, const void* y, const void* z) {
+  if (sxd != 1 || D < 4) return 1;
+  const uintptr_t a = (uintptr_t)x | (uintptr_t)y | (uintptr_t)z;
+  if (D % 4 == 0 && sxl % 4 == 0 && sxb % 4 == 0 && a % 16 == 0) return 4;
+  const int64_t lanes4 = (D + 4 * kCgWg - 1) / (4 * kCgWg) * 4 * kCgWg, lanes1 = (D + kCgWg - 1) / kCgWg * kCgWg;
+  return 2 * lanes4 <= 3 * lanes1 ? 4 : 1;
 }
 
 template <typename TIO, int K, int VEC>
@@ -778,13 +841,13 @@ int tsfast_hip_conv_silu_fwd(int64_t B, int64_t L, int64_t D, int64_t K, int io_
   if (const int st = conv_layout_status(L, D, sxl, sxd, io_dtype == TSF_DTYPE_BF16 ? 2 : 4)) return st;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (io_dtype == TSF_DTYPE_F32) {
-    const int vec = vec_for<float>(x, D, sxb, sxl, sxd, out);
+    const int vec = vec_for(x, D, sxb, sxl, sxd, out, nullptr);
 #define CALL(KK) fwd_reg<float, KK>(vec, B, L, D, x, sxb, sxl, sxd, tail, weight, bias, out, s)
     TSF_CONV_K_SWITCH(K, CALL)
 #undef CALL
   } else if (io_dtype == TSF_DTYPE_BF16) {
-    const bool vec = vec_rows<bf16>(x, D, sxb, sxl, sxd, out, nullptr);
-#define CALL(KK) fwd_k<bf16, KK>(vec, B, L, D, x, sxb, sxl, sxd, tail, weight, bias, out, s)
+    const Rows rows = rows_of<bf16>(x, D, sxb, sxl, sxd, out, nullptr);
+#define CALL(KK) fwd_k<bf16, KK>(rows, B, L, D, x, sxb, sxl, sxd, tail, weight, bias, out, s)
     TSF_CONV_K_SWITCH(K, CALL)
 #undef CALL
   } else {
@@ -814,18 +877,18 @@ int tsfast_hip_conv_silu_bwd(int64_t B, int64_t L, int64_t D, int64_t K, int io_
   if (const int st = conv_layout_status(L, D, sxl, sxd, io_dtype == TSF_DTYPE_BF16 ? 2 : 4)) return st;
   float* part = static_cast<float*>(workspace);
   if (io_dtype == TSF_DTYPE_F32 && K >= TSF_CONV_F32_TILED_K) {
-    const bool vec = vec_rows<float>(x, D, sxb, sxl, sxd, gy, gx);
-#define CALL(KK) bwd_k<float, KK>(vec, B, L, D, x, sxb, sxl, sxd, tail, weight, bias, gy, gx, gtail, gw, gb, part, s)
+    const Rows rows = rows_of<float>(x, D, sxb, sxl, sxd, gy, gx);
+#define CALL(KK) bwd_k<float, KK>(rows, B, L, D, x, sxb, sxl, sxd, tail, weight, bias, gy, gx, gtail, gw, gb, part, s)
     TSF_CONV_K_SWITCH(K, CALL)
 #undef CALL
   } else if (io_dtype == TSF_DTYPE_F32) {
-    const int vec = vec_for<float>(x, D, sxb, sxl, sxd, gy) == 4 && ((uintptr_t)gx % 16 == 0) ? 4 : 1;
+    const int vec = vec_for(x, D, sxb, sxl, sxd, gy, gx);
 #define CALL(KK) bwd_reg<float, KK>(vec, B, L, D, x, sxb, sxl, sxd, tail, weight, bias, gy, gx, gtail, gw, gb, part, s)
     TSF_CONV_K_SWITCH(K, CALL)
 #undef CALL
   } else if (io_dtype == TSF_DTYPE_BF16) {
-    const bool vec = vec_rows<bf16>(x, D, sxb, sxl, sxd, gy, gx);
-#define CALL(KK) bwd_k<bf16, KK>(vec, B, L, D, x, sxb, sxl, sxd, tail, weight, bias, gy, gx, gtail, gw, gb, part, s)
+    const Rows rows = rows_of<bf16>(x, D, sxb, sxl, sxd, gy, gx);
+#define CALL(KK) bwd_k<bf16, KK>(rows, B, L, D, x, sxb, sxl, sxd, tail, weight, bias, gy, gx, gtail, gw, gb, part, s)
     TSF_CONV_K_SWITCH(K, CALL)
 #undef CALL
   } else {
