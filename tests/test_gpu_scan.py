@@ -350,6 +350,8 @@ def test_diag_shared_coefficients(gpu, dtype, M, L, N):
     lam, v, x0, g = _make_diag((M, L, N), (N,), dtype, seed=M + L)
     lam, v, x0, g = (t.to(gpu) for t in (lam, v, x0, g))
     rows = lam.expand(M, N).contiguous()
+    assert diagonal_hip.supports_shared(lam, v, x0) is None and diagonal_hip.supports(rows, v, x0) is None
+    assert diagonal_hip.supports(lam, v, x0) and diagonal_hip.supports_shared(rows, v, x0)
     out = diagonal_hip.forward(lam, v, x0)
     assert torch.equal(out, diagonal_hip.forward(rows, v, x0))
     glam, gv, gx0 = diagonal_hip.backward(g, lam, out, x0)

@@ -20,6 +20,15 @@ _DTYPES = (torch.float32, torch.complex64)
 
 def supports(lam: torch.Tensor, v: torch.Tensor, x0: torch.Tensor | None) -> str | None:
     """Reason this backend cannot handle the inputs, or None when it can."""
+    return _reason(lam, v, x0, 2)
+
+
+def supports_shared(lam: torch.Tensor, v: torch.Tensor, x0: torch.Tensor | None) -> str | None:
+    """``supports`` for one coefficient row ``lam [N]`` that all batch rows share."""
+    return _reason(lam, v, x0, 1)
+
+
+def _reason(lam, v, x0, lam_dims: int) -> str | None:
     if v.device.type != "cuda":
         return f"input on {v.device.type}, hip backend is GPU-only"
     if v.dtype not in _DTYPES:
@@ -28,9 +37,9 @@ def supports(lam: torch.Tensor, v: torch.Tensor, x0: torch.Tensor | None) -> str
         return f"lam dtype {lam.dtype} != v dtype {v.dtype}"
     if x0 is not None and x0.dtype != v.dtype:
         return f"x0 dtype {x0.dtype} != v dtype {v.dtype}"
-    if v.dim() != 3 or lam.dim() not in (1, 2):
-        return "expects the lane layout lam [M, N] (or one row [N]), v [M, L, N]"
-    if tuple(lam.shape) not in ((v.shape[0], v.shape[2]), (v.shape[2],)):
+    if v.dim() != 3 or lam.dim() != lam_dims:
+        return "expects the lane layout lam [M, N], v [M, L, N]"
+    if tuple(lam.shape) != (v.shape[0], v.shape[2])[2 - lam_dims :]:
         return f"lam {tuple(lam.shape)} does not match v {tuple(v.shape)}"
     if x0 is not None and tuple(x0.shape) != (v.shape[0], v.shape[2]):
         return f"x0 {tuple(x0.shape)} does not match lam {tuple(lam.shape)}"
