@@ -8,7 +8,9 @@ sections through the HIP ops with Inductor.
 """
 
 import numpy as np
+import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
 
 from tsfast_amd import scan
 from tsfast_amd.dynonet import core as dcore
@@ -84,3 +86,25 @@ def test_trace_dynonet_sections():
 
     _check(gblock, u, b, ad, tail, x0)
     _check(lambda u, b, ad: dcore.linear_dynamical_operator(u, b, ad), u, b, ad)
+
+
+@pytest.mark.parametrize("M,L", [(2, 0), (0, 4), (0, 0), (2, 4)])
+@pytest.mark.parametrize("with_x0", [True, False])
+@pytest.mark.parametrize("kind", ["diagonal", "shared", "selective"])
+def test_traced_scan_gradients_have_the_shapes_of_the_real_ones(kind, with_x0, M, L):
+    """Under fake tensors (what a compiled program's backward is traced with), also without a step
+    or a row: the shapes and types that the op gives on these sizes."""
+    N = 3
+    lam_shape = {"diagonal": (M, N), "shared": (N,), "selective": (M, L, N)}[kind]
+    fwd = {"diagonal": scan._scan_diagonal_op, "shared": scan._scan_shared_op, "selective": scan._scan_selective_op}[kind]
+    bwd = {"diagonal": scan._scan_diagonal_bwd_op, "shared": scan._scan_shared_bwd_op, "selective": scan._scan_selective_bwd_op}[kind]
+
+    def call():
+        lam, v, g = torch.rand(lam_shape), torch.rand(M, L, N), torch.rand(M, L, N)
+        x0 = torch.rand(M, N) if with_x0 else None
+        out = fwd(lam, v, x0)
+        return [(t.shape, t.dtype) for t in (out, *bwd(g, lam, out, x0))]
+
+    want = call()
+    with FakeTensorMode():
+        assert call() == want
