@@ -88,3 +88,16 @@ def test_transforms_take_the_registered_op(gpu, monkeypatch):
     with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
         scan.diagonal_recurrence(lam, v)
     assert any(e.key.startswith("tsfast_hip::scan_diagonal") for e in prof.key_averages())
+
+
+def test_a_first_call_in_inference_mode_leaves_later_calls_direct(gpu, monkeypatch):
+    lam, v, gy = _inputs(gpu)
+    monkeypatch.setattr(ops, "_plain_keys", set())
+    with torch.inference_mode():
+        scan.diagonal_recurrence(lam, v)
+    dispatched = []
+    monkeypatch.setattr(scan._scan_shared_op, "_op", lambda *a: dispatched.append(a))
+    _pass(lam, v, gy)
+    with torch.inference_mode():
+        scan.diagonal_recurrence(lam, v.clone())
+    assert not dispatched

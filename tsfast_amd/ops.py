@@ -1,7 +1,8 @@
 """Custom ops that cost a plain eager call no dispatcher round trip.
 
 ``custom_op`` registers an op as ``torch.library.custom_op`` does. A call that nothing but the
-kernels would see (dense GPU tensors; no trace, transform, mode, forward-mode level or profiler)
+kernels would see (dense GPU tensors; no trace, transform, forward-mode level or profiler, no mode:
+``torch.set_default_device`` is one)
 runs the op's function directly, under an ``autograd.Function`` with the op's own rules when a
 gradient is wanted. Every other call goes through the registered op. The dispatcher's Python layers
 bound small passes: a truncated-BPTT chunk (8 x 4096 x 128, forward and backward) took 263 us
@@ -22,18 +23,22 @@ _C = torch._C
 _plain_keys: set[int] = set()
 
 
+def _keys_of_plain(device: torch.device) -> set[int]:
+    """The keys of both, whatever mode the caller is in: a first call under inference mode (a model
+    validated before it is trained) must not leave ordinary tensors to the dispatcher for good."""
+    keys = set()
+    for mode in (False, True):
+        with torch.inference_mode(mode):
+            keys.add(_C._dispatch_keys(torch.empty(0, device=device)).raw_repr())
+    return keys
+
+
 def _plain(t: torch.Tensor) -> bool:
     if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
         return False
-    keys = _C._dispatch_keys(t).raw_repr()
-    if keys in _plain_keys:
-        return True
     if not _plain_keys and t.is_cuda:
-        _plain_keys.add(_C._dispatch_keys(torch.empty(0, device=t.device)).raw_repr())
-        with torch.inference_mode():
-            _plain_keys.add(_C._dispatch_keys(torch.empty(0, device=t.device)).raw_repr())
-        return keys in _plain_keys
-    return False
+        _plain_keys.update(_keys_of_plain(t.device))
+    return _C._dispatch_keys(t).raw_repr() in _plain_keys
 
 
 def _unobserved() -> bool:
