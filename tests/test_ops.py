@@ -1,5 +1,6 @@
 """Ops called without the dispatcher (tsfast_amd/ops.py), on the CPU: which calls may go directly."""
 
+import pytest
 import torch
 
 from tsfast_amd import ops
@@ -16,3 +17,44 @@ def test_plain_keys_do_not_depend_on_the_mode_of_the_first_call():
         first_in_inference = ops._keys_of_plain(torch.device("cpu"))
     assert _keys(ordinary) != _keys(inference)
     assert first_in_inference == ops._keys_of_plain(torch.device("cpu")) == {_keys(ordinary), _keys(inference)}
+
+
+@pytest.fixture(scope="module")
+def scaled():
+    """An op of the package's kind, ``x * 2 (+ y)``."""
+
+    @ops.custom_op("tsfast_hip_test::scaled")
+    def scaled(x: torch.Tensor, y: torch.Tensor | None) -> torch.Tensor:
+        return x * 2 if y is None else x * 2 + y
+
+    scaled.register_fake(lambda x, y: torch.empty_like(x))
+    return scaled
+
+
+@pytest.fixture
+def direct(monkeypatch):
+    """CPU tensors stand in for GPU tensors: plain ones are called directly."""
+    monkeypatch.setattr(ops, "_plain_keys", ops._keys_of_plain(torch.device("cpu")))
+
+
+def test_tensor_likes_and_keywords_reach_the_registered_op(scaled, direct):
+    x = torch.arange(3.0)
+
+    class Recorder:
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            return func
+
+    assert torch.equal(scaled(x, None), 2 * x)
+    assert scaled(x, Recorder()) is torch.ops.tsfast_hip_test.scaled.default
+    assert torch.equal(scaled(x, y=x), 3 * x)
+    with pytest.raises(RuntimeError):
+        scaled(x, "y")
+
+
+def test_ops_offer_what_a_custom_op_offers(scaled, direct):
+    scaled.register_vmap(lambda info, in_dims, x, y: (scaled(x, y), in_dims[0]))
+    x = torch.randn(4, 3)
+    assert torch.equal(torch.func.vmap(lambda t: scaled(t, None))(x), 2 * x)
+    with pytest.raises(AttributeError):
+        scaled.no_such_attribute

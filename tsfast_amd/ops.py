@@ -1,13 +1,13 @@
 """Custom ops that cost a plain eager call no dispatcher round trip.
 
 ``custom_op`` registers an op as ``torch.library.custom_op`` does. A call that nothing but the
-kernels would see (dense GPU tensors; no trace, transform, forward-mode level or profiler, no mode:
-``torch.set_default_device`` is one)
-runs the op's function directly, under an ``autograd.Function`` with the op's own rules when a
-gradient is wanted. Every other call goes through the registered op. The dispatcher's Python layers
-bound small passes: a truncated-BPTT chunk (8 x 4096 x 128, forward and backward) took 263 us
-through them and takes 192 us without, a Mamba window (64 x 512 x 128) 239 and 201 us, a forward
-call without gradients 49 and 44 us.
+kernels would see (dense GPU tensors, or None; no trace, transform, mode, forward-mode level or
+profiler) runs the op's function directly, under an ``autograd.Function`` with the op's own rules
+when a gradient is wanted. Every other call goes through the registered op, also under
+``torch.set_default_device``, which is a mode. The dispatcher's Python layers bound small passes: a
+truncated-BPTT chunk (8 x 4096 x 128, forward and backward) took 263 us through them and takes 192
+us without, a Mamba window (64 x 512 x 128) 239 and 201 us, a forward call without gradients 49 and
+44 us.
 """
 
 from __future__ import annotations
@@ -33,7 +33,7 @@ def _keys_of_plain(device: torch.device) -> set[int]:
     return keys
 
 
-def _plain(t: torch.Tensor) -> bool:
+def _plain(t) -> bool:
     if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
         return False
     if not _plain_keys and t.is_cuda:
@@ -64,8 +64,11 @@ class _Op:
         self._function = None
         self.__doc__ = fn.__doc__
 
-    def register_fake(self, fn):
-        return self._def.register_fake(fn)
+    def __getattr__(self, name):
+        """Everything else a custom op offers (``register_kernel``, ``register_vmap`` ..)."""
+        if name == "_def":  # not set yet
+            raise AttributeError(name)
+        return getattr(self._def, name)
 
     def register_autograd(self, backward, *, setup_context):
         self._def.register_autograd(backward, setup_context=setup_context)
@@ -85,15 +88,16 @@ class _Op:
         Direct.__name__ = Direct.__qualname__ = f"Direct_{impl.__name__}"
         self._function = Direct
 
-    def __call__(self, *args):
-        if torch.compiler.is_compiling() or not _unobserved():
-            return self._op(*args)
+    def __call__(self, *args, **kwargs):
+        if kwargs or torch.compiler.is_compiling() or not _unobserved():
+            return self._op(*args, **kwargs)
         wants_grad = False
         for t in args:
-            if isinstance(t, torch.Tensor):
-                if not _plain(t):
-                    return self._op(*args)
-                wants_grad = wants_grad or t.requires_grad
+            if t is None:
+                continue
+            if not _plain(t):  # also what is no tensor: the dispatcher takes or refuses it (a proxy of a trace ..)
+                return self._op(*args)
+            wants_grad = wants_grad or t.requires_grad
         if wants_grad and torch.is_grad_enabled():
             # an op without rules (a backward's) says so itself when it is differentiated
             return self._op(*args) if self._function is None else self._function.apply(*args)
