@@ -58,3 +58,33 @@ def test_ops_offer_what_a_custom_op_offers(scaled, direct):
     assert torch.equal(torch.func.vmap(lambda t: scaled(t, None))(x), 2 * x)
     with pytest.raises(AttributeError):
         scaled.no_such_attribute
+
+
+@pytest.mark.parametrize("how", ["kernel", "library", "autocast", "autograd"])
+def test_registrations_from_elsewhere_are_not_passed_by(direct, monkeypatch, how):
+    name = f"tsfast_hip_test::replaced_by_{how}"
+
+    @ops.custom_op(name)
+    def op(x: torch.Tensor) -> torch.Tensor:
+        return x * 2
+
+    op.register_autograd(lambda ctx, g: 2 * g, setup_context=lambda ctx, inputs, output: None)
+    dispatched = []
+    registered = op._op
+    monkeypatch.setattr(op, "_op", lambda *a: dispatched.append(1) or registered(*a))
+    x = torch.randn(3, requires_grad=True)
+    op(x).sum().backward()
+    assert not dispatched and torch.equal(x.grad, torch.full((3,), 2.0))
+    if how == "kernel":
+        torch.library.register_kernel(name, "cuda", lambda x: x * 3)
+    elif how == "library":
+        library = torch.library.Library("tsfast_hip_test", "IMPL")
+        library.impl(name.split("::")[1], lambda x: x * 3, "CUDA")
+    elif how == "autocast":
+        torch.library.register_autocast(name, "cuda", torch.float32)
+    else:
+        torch.library.register_autograd(name, lambda ctx, g: 5 * g)
+    x.grad = None
+    op(x).sum().backward()
+    assert dispatched
+    assert torch.equal(x.grad, torch.full((3,), 5.0 if how == "autograd" else 2.0))

@@ -4,7 +4,8 @@
 kernels would see (dense GPU tensors, or None; no trace, transform, mode, forward-mode level or
 profiler) runs the op's function directly, under an ``autograd.Function`` with the op's own rules
 when a gradient is wanted. Every other call goes through the registered op, also under
-``torch.set_default_device``, which is a mode. The dispatcher's Python layers bound small passes: a
+``torch.set_default_device``, which is a mode, and where a program has registered a kernel, cast or
+autograd rule of its own on the op (from Python). The dispatcher's Python layers bound small passes: a
 truncated-BPTT chunk (8 x 4096 x 128, forward and backward) took 263 us through them and takes 192
 us without, a Mamba window (64 x 512 x 128) 239 and 201 us, a forward call without gradients 49 and
 44 us.
@@ -61,7 +62,11 @@ class _Op:
         self._def = torch.library.custom_op(name, fn, mutates_args=())
         ns, op = name.split("::")
         self._op = getattr(getattr(torch.ops, ns), op).default
-        self._function = None
+        self._function = self._backward = None
+        # what a registration from elsewhere that a GPU call would meet is recorded under
+        self._overrides = frozenset(
+            f"{ns}/{op}{overload}/{key}" for overload in ("", ".default") for key in ("CUDA", "AutogradCUDA", "AutocastCUDA")
+        )
         self.__doc__ = fn.__doc__
 
     def __getattr__(self, name):
@@ -86,10 +91,13 @@ class _Op:
                 return backward(ctx, *grads)
 
         Direct.__name__ = Direct.__qualname__ = f"Direct_{impl.__name__}"
-        self._function = Direct
+        self._function, self._backward = Direct, self._def._backward_fn
+
+    def _overridden(self) -> bool:
+        return not self._overrides.isdisjoint(torch.library._impls) or self._def._backward_fn is not self._backward
 
     def __call__(self, *args, **kwargs):
-        if kwargs or torch.compiler.is_compiling() or not _unobserved():
+        if kwargs or torch.compiler.is_compiling() or not _unobserved() or self._overridden():
             return self._op(*args, **kwargs)
         wants_grad = False
         for t in args:
