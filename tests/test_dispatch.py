@@ -1,6 +1,7 @@
 """Dispatch semantics (mirrors the reference's tests/test_scan_dispatch.py:17-112) on the CPU."""
 
 import sys
+import threading
 import types
 import warnings
 
@@ -132,3 +133,36 @@ def test_lookback_give_up_check(monkeypatch):
         _lib.check_lookback(ws, "scan")
     monkeypatch.setattr(_lib, "_CHECK_LOOKBACK", False)
     _lib.check_lookback(ws, "scan")  # debug mode off: never reads the flag
+
+
+def test_a_module_another_thread_is_importing_is_waited_for(tmp_path, monkeypatch):
+    """A dotted backend is in ``sys.modules`` from the start of its import on, complete only at its end."""
+    started, go = threading.Event(), threading.Event()
+    monkeypatch.setattr(threading, "backend_started", started, raising=False)
+    monkeypatch.setattr(threading, "backend_go", go, raising=False)
+    (tmp_path / "slow_backend_module.py").write_text(
+        "import threading\n"
+        "threading.backend_started.set()\n"
+        "assert threading.backend_go.wait(30)\n"
+        "def supports(*args):\n    return None\n"
+    )
+    monkeypatch.syspath_prepend(str(tmp_path))
+    monkeypatch.delitem(sys.modules, "slow_backend_module", raising=False)
+    registry = {"hip": "slow_backend_module"}
+    found = []
+
+    def look():
+        try:
+            found.append(dispatch.resolve("test.slow", registry, ("hip",), ()))
+        except Exception as e:
+            found.append(e)
+
+    first, second = threading.Thread(target=look), threading.Thread(target=look)
+    first.start()
+    assert started.wait(30)
+    second.start()
+    second.join(0.5)  # returns early only where the half-made module is taken as it is
+    go.set()
+    first.join(30)
+    second.join(30)
+    assert len(found) == 2 and all(getattr(m, "__name__", None) == "slow_backend_module" for m in found), found
