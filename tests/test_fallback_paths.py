@@ -12,7 +12,8 @@ import pytest
 import torch
 
 from oracle import scan_oracle as O
-from tsfast_amd import blocked_scan, scan
+from tsfast_amd import blocked_scan, dispatch, scan
+from tsfast_amd.dynonet import core as dcore
 from tsfast_amd.mamba import core as mcore
 
 TOL = 1e-10
@@ -151,3 +152,20 @@ def test_complex_projections_match_complex_matmul():
     )
     for g_, w_ in zip(got, want):
         assert O.rel_err(g_, w_) < TOL
+
+
+def _gblock_inputs():
+    g = torch.Generator().manual_seed(4)
+    draw = lambda *s: torch.randn(*s, generator=g, dtype=torch.float64)
+    return draw(2, 20, 2), draw(3, 2, 4), draw(3, 2, 2) * 0.1, draw(2, 3, 2), draw(2, 6, 2)  # u, b, a, u tail, x
+
+
+def test_gblock_refuses_a_state_without_its_inputs():
+    """A state dict whose input tail is missing is an error, never a run from rest."""
+    u, b, a, tail, x = _gblock_inputs()
+    for state in ({"u": None, "x": x}, {"u": None, "x": None}):
+        with pytest.raises(TypeError):
+            dcore.linear_dynamical_operator(u, b, a, state, return_state=True)
+    rest = {"u": torch.zeros_like(tail), "x": torch.zeros_like(x)}
+    for got, want in zip(dcore.linear_dynamical_operator(u, b, a, None, True), dcore.linear_dynamical_operator(u, b, a, rest, True)):
+        torch.testing.assert_close(got, want, rtol=0, atol=0)

@@ -152,9 +152,8 @@ def linear_dynamical_operator(
     na = a_coeff.shape[-1]
     P = I * O
     # plain branches, not a mapping `match`: Dynamo cannot trace mapping patterns
-    u_tail = x0 = None  # the fused backend takes absent initial conditions as zeros
     if state is None:
-        pass
+        u_tail, x0 = None, None  # zeros, which this package's backend need not read
     elif isinstance(state, dict) and "u" in state and "x" in state:
         u_tail, x0 = state["u"], state["x"]
     else:
@@ -164,7 +163,7 @@ def linear_dynamical_operator(
     if mod is not None:
         y, x_last = mod.run(u, b_coeff, a_coeff, u_tail, x0)
     else:
-        if u_tail is None:
+        if state is None:
             u_tail, x0 = u.new_zeros(B, nb - 1, I), u.new_zeros(B, P, na)
         u_buf = torch.cat((u_tail, u), dim=1)
         weight = b_coeff.permute(1, 0, 2).reshape(P, 1, nb).flip(-1)
@@ -177,5 +176,7 @@ def linear_dynamical_operator(
         y = y_pairs.view(B, I, O, L).sum(1).transpose(1, 2)
     if not return_state:
         return y
-    u_buf = torch.cat((u.new_zeros(B, nb - 1, I) if u_tail is None else u_tail, u), dim=1)
+    if state is None:
+        u_tail = u.new_zeros(B, nb - 1, I)
+    u_buf = torch.cat((u_tail, u), dim=1)
     return y, {"u": u_buf[:, u_buf.shape[1] - (nb - 1) :], "x": x_last}
