@@ -169,3 +169,27 @@ def test_gblock_refuses_a_state_without_its_inputs():
     rest = {"u": torch.zeros_like(tail), "x": torch.zeros_like(x)}
     for got, want in zip(dcore.linear_dynamical_operator(u, b, a, None, True), dcore.linear_dynamical_operator(u, b, a, rest, True)):
         torch.testing.assert_close(got, want, rtol=0, atol=0)
+
+
+def test_a_backend_in_place_of_the_gblocks_gets_whole_initial_conditions(monkeypatch):
+    """The protocol's backends take tensors; absent conditions are for this package's own only."""
+    u, b, a, tail, x = _gblock_inputs()
+    seen = []
+
+    class Backend:
+        @staticmethod
+        def supports(*args):
+            seen.append(args)
+            return None
+
+        @staticmethod
+        def run(*args):
+            seen.append(args)
+            return u.new_zeros(2, 20, 3), x
+
+    monkeypatch.setitem(dcore._GBLOCK_BACKENDS, "hip", Backend)
+    with dispatch.use_backend("hip"):
+        dcore.linear_dynamical_operator(u, b, a)
+    assert len(seen) == 2
+    for *_, tail_arg, x_arg in seen:
+        assert torch.equal(tail_arg, torch.zeros_like(tail)) and torch.equal(x_arg, torch.zeros_like(x))

@@ -154,6 +154,8 @@ def linear_dynamical_operator(
     # plain branches, not a mapping `match`: Dynamo cannot trace mapping patterns
     if state is None:
         u_tail, x0 = None, None  # zeros, which this package's backend need not read
+        if _GBLOCK_BACKENDS.get("hip") is not gblock_hip:
+            u_tail, x0 = u.new_zeros(B, nb - 1, I), u.new_zeros(B, P, na)
     elif isinstance(state, dict) and "u" in state and "x" in state:
         u_tail, x0 = state["u"], state["x"]
     else:
