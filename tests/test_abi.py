@@ -75,8 +75,9 @@ def test_size_queries(lib):
     assert lib.tsfast_hip_conv_silu_workspace_bytes(16, 4096, 1536, 4) > 0
     assert lib.tsfast_hip_conv_silu_workspace_bytes(1, 8, 4, 9) == -1  # kernel width above 8
     # counter, agg and inc [nsuper][lanes][n], grad_A partials [nsuper][lanes][n][n], Mc and Ms
-    # [lanes][n][n]: n = 2 has 16-step chunks, K = 2 here (few tiles), so nsuper = ceil(100 / 32)
-    assert lib.tsfast_hip_linrec_workspace_bytes(64, 100, 2) == 256 + 8 * (4 * 64 * (2 + 2 + 4) + 2 * 64 * 4)
+    # [lanes][n][n]: n = 2 has 16-step chunks, 8 of them a tile, so nsuper = 1 and ceil(300 / 128)
+    assert lib.tsfast_hip_linrec_workspace_bytes(64, 100, 2) == 256 + 8 * (1 * 64 * (2 + 2 + 4) + 2 * 64 * 4)
+    assert lib.tsfast_hip_linrec_workspace_bytes(64, 300, 2) == 256 + 8 * (3 * 64 * (2 + 2 + 4) + 2 * 64 * 4)
     # n = 5..8: e/f and carries [chunks][lanes][n], the lane matrices and the grad_A partials
     assert lib.tsfast_hip_linrec_workspace_bytes(4, 300, 5) == 8 * (2 * 2 * 4 * 5 + 4 * 25 + 2 * 4 * 25)
     # n = 9..16 (spread path): the same areas with the same 256-step chunks

@@ -486,8 +486,8 @@ LrPlan lr_plan(int64_t lanes, int64_t L, int64_t ns) {
   LrPlan p;
   const int64_t S = kTileT / ns;
   p.groups = (lanes + kTile - 1) / kTile;
-  const int64_t chunks = L > 0 ? (L + S - 1) / S : 0;
   if (L > 0) {
+    const int64_t chunks = (L + S - 1) / S;
     p.K = chunks < kLbWaves ? (int)chunks : kLbWaves;
     p.nsuper = (L + S * p.K - 1) / (S * p.K);
   }
@@ -497,12 +497,7 @@ LrPlan lr_plan(int64_t lanes, int64_t L, int64_t ns) {
   p.off_part = p.off_inc + vecs;
   p.off_Mc = p.off_part + vecs * ns;
   p.off_Ms = p.off_Mc + f * lanes * ns * ns;
-  // The size query keeps the bound of shorter tiles on few lanes (K halved down to 2 below 256 tiles),
-  // which this plan stays within: callers have sized buffers by it.
-  int64_t K = kLbWaves, rows = 0;
-  while (K > 2 && p.groups * ((chunks + K - 1) / K) < 256) K /= 2;
-  if (chunks > 0) rows = K < chunks ? (chunks + K - 1) / K : 1;
-  p.bytes = p.off_agg + f * (rows * lanes * ns * (2 + ns) + 2 * lanes * ns * ns);
+  p.bytes = p.off_Ms + f * lanes * ns * ns;
   return p;
 }
 
