@@ -814,9 +814,9 @@ def run_linrec(args, line):
         kernels = {"fwd": ("linrec_fwd_lb look-back scan + transfer + reset", fwd_ms, fwd_b),
                    "bwd": ("linrec_bwd_lb look-back scan + transfer + reset + finish", bwd_ms, bwd_b)}
     elif n <= 8:
-        kernels = {"fwd": ("lw_sum_fwd + lw_carry_fwd + lw_apply_fwd two-pass scan + lw_power", fwd_ms, fwd_b),
-                   "bwd": ("lw_sum_bwd + lw_carry_bwd + lw_apply_bwd two-pass scan + lw_power + finish", bwd_ms,
-                           bwd_b)}
+        kernels = {"fwd": ("lw_sum_fwd (with the powers) + lw_carry + lw_apply_fwd two-pass scan", fwd_ms, fwd_b),
+                   "bwd": ("lw_sum_bwd (with the powers) + lw_carry + lw_apply_bwd two-pass scan + finish",
+                           bwd_ms, bwd_b)}
     else:
         kernels = {"fwd": ("lsp_sum_fwd + lsp_carry_fwd + lsp_apply_fwd spread two-pass scan + lsp_power", fwd_ms,
                            fwd_b),
