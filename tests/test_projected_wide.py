@@ -51,15 +51,24 @@ def _make(B, L, H, N, O_, seed):
 
 
 @pytest.mark.parametrize("K", [1, 100, 4096 * 2 - 1, 4096 * 2, 4096 * 3 + 7, 4096 * 20 + 5])
-def test_gram_is_the_plain_product(K):
-    """Split-K sums (up to 16 row blocks and a remainder) equal a^T b."""
+def test_split_gradients_are_the_plain_products(K):
+    """The split-K partials (one, up to 16 row blocks, a remainder) and their sums in the weights' own
+    layouts: a^T b with re / im in alternate rows for W, in alternate columns (im negated) for C."""
     g = torch.Generator().manual_seed(K)
-    a = torch.randn(K, 24, generator=g, dtype=torch.float64)
-    b = torch.randn(K, 10, generator=g, dtype=torch.float64)
-    got = projected_hip._gram(a, b)
-    want = a.numpy().T @ b.numpy()
-    assert got.shape == (24, 10)
-    assert np.abs(got.numpy() - want).max() <= 1e-12 * max(1.0, np.abs(want).max()) * np.sqrt(K)
+    N, H, O_, B = 12, 10, 7, 3
+    v, u = torch.randn(K, 2 * N, generator=g, dtype=torch.float64), torch.randn(K, H, generator=g, dtype=torch.float64)
+    gy = torch.randn(K, O_, generator=g, dtype=torch.float64)
+    rows = torch.randn(B, N, generator=g, dtype=torch.complex128)
+    g_w, g_c = projected_hip._gram_parts(v, u), projected_hip._gram_parts(gy, v)
+    blocks = min(16, K // 4096)
+    parts = 1 if blocks < 2 else blocks + (K % blocks > 0)
+    assert g_w.shape == (parts, 2 * N, H) and g_c.shape == (parts, O_, 2 * N)
+    got = projected_hip._unpack(g_w, g_c, rows)
+    want_w, want_c = v.numpy().T @ u.numpy(), gy.numpy().T @ v.numpy()
+    want = (want_w[0::2], want_w[1::2], rows.numpy().sum(0), want_c[:, 0::2], -want_c[:, 1::2])
+    for a, b in zip(got, want):
+        assert a.shape == b.shape
+        assert np.abs(a.numpy() - b).max() <= 1e-12 * max(1.0, np.abs(b).max()) * np.sqrt(K)
 
 
 def test_weight_layouts():

@@ -11,7 +11,7 @@ Shapes: ``u [B, L, H]`` float32, ``W_re/W_im [N, H]``, ``lam [N]`` complex64, ``
   look-back); the complex ``v`` and ``x`` (``[B, L, N]`` each) never reach HBM.
 * wide (any other widths): each projection is one packed real GEMM (hipBLASLt) around this
   library's diagonal scan kernels, and the backward is written out by hand so that the two weight
-  gradients, products over all B L rows, run as split-K batched GEMMs (``_gram``). At these widths
+  gradients, products over all B L rows, run as split-K batched GEMMs (``_gram_parts``). At these widths
   the matrix work dominates and the library GEMMs run it at a higher share of the matrix-core peak
   than the fused kernel's scan-bound pipeline.
 """
@@ -239,16 +239,12 @@ _SPLITK_PARTS = 16  # products per split-K weight gradient ...
 _SPLITK_ROWS = 4096  # ... each over at least this many rows
 
 
-def _gram(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
-    """``a^T b`` for ``a [K, M]``, ``b [K, N]`` with K = B L rows and small M, N: the weight
-    gradients of the projections. One GEMM with K in the hundreds of thousands keeps few output
-    tiles busy (24-73 TFLOP/s measured at M, N = 512..1024, 32..128); cut into 16 batched products
-    over consecutive row blocks and summed in a fixed order, the same product runs at 110-134."""
-    return _gram_parts(a, b).sum(0)
-
-
 def _gram_parts(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
-    """``_gram``'s partial products ``[parts, M, N]``, one over each block of rows."""
+    """Partial products ``[parts, M, N]`` of ``a^T b`` for ``a [K, M]``, ``b [K, N]`` with K = B L rows
+    and small M, N, the weight gradients of the projections, one over each block of rows (``_unpack``
+    sums them in order). One GEMM with K in the hundreds of thousands keeps few output tiles busy
+    (24-73 TFLOP/s measured at M, N = 512..1024, 32..128); cut into 16 batched products over
+    consecutive row blocks the same product runs at 110-134."""
     K, M = a.shape
     parts = min(_SPLITK_PARTS, K // _SPLITK_ROWS)
     if parts < 2:
