@@ -9,6 +9,7 @@ import torch
 from oracle import scan_oracle as O
 from tests.test_gpu_mamba import _NAMES, _make, _np64, _run_hip
 from tsfast_amd import _lib
+from tsfast_amd.mamba import mamba_hip
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +44,32 @@ def test_split_rule():
     assert ws(1, 255, 64, 16) == 0 and ws(1, 256, 64, 16) == 4 * 4 * 64 * 17
     assert ws(1, 4096, 1025, 16) == 0 and ws(1, 4096, 1024, 16) > 0
     assert ws(16, 4096, 1536, 16) == 0 and ws(1, 4096, 64, 65) == -1
+
+
+def test_growing_states_at_zero_stay_there(gpu):
+    """A > 0: a segment's factor exp(A S) overflows fp32 (e^177 here); zero states and adjoints pass it as zeros."""
+    B, L, D, N = 1, 1024, 32, 8
+    draw, A = torch.zeros(B, L, D, device=gpu), torch.full((D, N), 4.0, device=gpu)
+    g = torch.Generator().manual_seed(1)
+    Bt, Ct, z, Dp = (torch.randn(*s, generator=g).to(gpu) for s in ((B, L, N), (B, L, N), (B, L, D), (D,)))
+    leaves = [t.requires_grad_() for t in (draw, A, Bt, Ct, torch.zeros(B, L, D, device=gpu), z, Dp)]
+    out, h_last = mamba_hip.run(*leaves, None)
+    grads = torch.autograd.grad(out, leaves, torch.zeros_like(out))
+    for t in (out, h_last, *grads):
+        assert torch.count_nonzero(t) == 0
+
+
+def test_growth_past_the_range_of_one_factor(gpu):
+    """A state of 1e-30 grows by e^128 over its first segment, to 3.9e25: the factor alone overflows. The
+    exponent's fp32 sum (64 steps to 128) is off by 8 ulp at most, 8 x 128 x 2^-24 of the result."""
+    B, L, D, N = 1, 1024, 32, 8
+    draw = torch.full((B, L, D), -200.0)  # delta = 0: nothing moves after the first 64 steps
+    draw[:, :64] = torch.log(torch.expm1(torch.tensor(2.0)))
+    t = dict(draw=draw, A=torch.ones(D, N), Bt=torch.ones(B, L, N), Ct=torch.ones(B, L, N), u=torch.zeros(B, L, D),
+             z=torch.ones(B, L, D), Dp=torch.ones(D), h0=torch.full((B, D, N), 1e-30))
+    with torch.no_grad():
+        out, h_last = mamba_hip.run(*(v.to(gpu) for v in t.values()))
+    want_out, want_h = O.mamba_forward(*(_np64(v) for v in t.values()))
+    assert 3e25 < want_h.max() < 5e25
+    assert O.rel_err(_np64(h_last), want_h) < 8 * 128 * 2.0**-24
+    assert O.rel_err(_np64(out), want_out) < 8 * 128 * 2.0**-24

@@ -237,7 +237,13 @@ TSF_DEV void compose_segments(const float* __restrict__ segs, int64_t first, int
     for (int q = 0; q < 4; ++q) {
       if (k == last) break;
 #pragma unroll
-      for (int j = 0; j < NPT; ++j) x[j] = fmaf(fast_exp2(A2[j] * S[q]), x[j], e[q][j]);
+      for (int j = 0; j < NPT; ++j) {
+        // a segment's factor may lie outside fp32 where its product with the state does not (a growing
+        // state at zero, as step by step, stays there): it is applied in two parts, 2^-126 .. 2^127 each
+        const float p = A2[j] * S[q], p0 = fminf(fmaxf(p, -126.0f), 127.0f);
+        const float p1 = fminf(fmaxf(p - p0, -126.0f), 127.0f);
+        x[j] = fmaf(fast_exp2(p0), x[j] * fast_exp2(p1), e[q][j]);
+      }
       k += step;
     }
   }
