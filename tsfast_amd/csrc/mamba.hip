@@ -368,8 +368,12 @@ __global__ void __launch_bounds__(FCfg<NS>::TH) mamba_segment_kernel(
 }
 
 // ------------------------------------------------------------------------------------ forward
-// SAVE: training forward (writes the checkpoints and y to chk); chk is unused otherwise.
-template <typename TIO, int NS, bool SAVE>
+// SAVE: training forward (writes the checkpoints and y to chk); chk is unused otherwise. SPLIT: the
+// workgroup walks one segment. Whole walks are instances of their own, in both directions: with the
+// segments' code in them the 64-state backward took 257 registers for 255, one wave per SIMD instead of two
+// (96 rows x 2000 steps, D 128, forward + backward 2608 -> 3417 us), and the 64-state forward 118 for 98
+// (16 rows, D 1024, 464 -> 525 us).
+template <typename TIO, int NS, bool SAVE, bool SPLIT>
 __global__ void __launch_bounds__(FCfg<NS>::TH, FCfg<NS>::WAVES >= 8 ? 3 : 1) mamba_fwd_kernel(
     const TIO* __restrict__ draw, const float* __restrict__ A, const TIO* __restrict__ Bt,
     const TIO* __restrict__ Ct, const TIO* __restrict__ u, const TIO* __restrict__ z, const float* __restrict__ Dp,
@@ -391,9 +395,9 @@ __global__ void __launch_bounds__(FCfg<NS>::TH, FCfg<NS>::WAVES >= 8 ? 3 : 1) ma
   int64_t tile, b;
   xcd_remap((D + DT - 1) / DT, tile, b);
   // this workgroup's time segment [t_begin, t_end) of its batch row (the whole row when unsplit)
-  const int64_t seg = b / B;
+  const int64_t seg = SPLIT ? b / B : 0;
   b -= seg * B;
-  const int64_t t_begin = seg * seg_len, t_end = t_begin + seg_len < L ? t_begin + seg_len : L;
+  const int64_t t_begin = seg * seg_len, t_end = SPLIT && t_begin + seg_len < L ? t_begin + seg_len : L;
   const int64_t d0 = tile * DT;
   // recurrence mapping: adjacent lanes hold the two halves of a state pair
   const int pr = tid & 1;
@@ -418,7 +422,7 @@ __global__ void __launch_bounds__(FCfg<NS>::TH, FCfg<NS>::WAVES >= 8 ? 3 : 1) ma
     h[j] = (act && h0 && n < N) ? h0[(b * D + d) * N + n] : 0.0f;
     co[j] = (uint32_t)n * Du + (uint32_t)dl;
   }
-  compose_segments<NPT>(segs, 0, seg, 1, B, b, D, d, N, [&](int j) { return n0 + j; }, act, A2, h);
+  if (SPLIT) compose_segments<NPT>(segs, 0, seg, 1, B, b, D, d, N, [&](int j) { return n0 + j; }, act, A2, h);
   const uint32_t slot_floats = Nu * Du;
   const float dp_o = oact ? Dp[d0 + od] : 0.0f;
 
@@ -567,7 +571,7 @@ __global__ void __launch_bounds__(FCfg<NS>::TH, FCfg<NS>::WAVES >= 8 ? 3 : 1) ma
     chunk((uint32_t)t0, (int)((t_end - t0) < TF ? (t_end - t0) : TF));
   }
   (void)NG;
-  if (act && t_end == L) {
+  if (act && (!SPLIT || t_end == L)) {
 #pragma unroll
     for (int j = 0; j < NPT; ++j)
       if (n0 + j < N) h_last[(b * D + d) * N + n0 + j] = h[j];
@@ -604,7 +608,7 @@ struct BCfg {
 //   D  owners prepare the previous chunk's per-(t, d) scalars in LDS (its inputs were loaded
 //      at the top of this iteration) and store grad z, which needs no recurrence
 //   -- barrier --
-template <typename TIO, int NS, int DT_>
+template <typename TIO, int NS, int DT_, bool SPLIT>
 __global__ void __launch_bounds__((BCfg<NS, DT_>::TH), (BCfg<NS, DT_>::OCC)) mamba_bwd_kernel(
     const TIO* __restrict__ draw, const float* __restrict__ A, const TIO* __restrict__ Bt,
     const TIO* __restrict__ Ct, const TIO* __restrict__ u, const TIO* __restrict__ z, const float* __restrict__ Dp,
@@ -629,9 +633,9 @@ __global__ void __launch_bounds__((BCfg<NS, DT_>::TH), (BCfg<NS, DT_>::OCC)) mam
   int64_t tile, b;
   xcd_remap((D + DT - 1) / DT, tile, b);
   // this workgroup's segment, chunks [c_begin, c_end) of its batch row (all of them when unsplit)
-  const int64_t part_row = b, seg = b / B;
+  const int64_t part_row = b, seg = SPLIT ? b / B : 0;
   b -= seg * B;
-  const int64_t c_begin = seg * seg_chunks, c_end = c_begin + seg_chunks < NC ? c_begin + seg_chunks : NC;
+  const int64_t c_begin = seg * seg_chunks, c_end = SPLIT && c_begin + seg_chunks < NC ? c_begin + seg_chunks : NC;
   const int64_t d0 = tile * DT;
   const int rw = tid >> 4, lk = tid & 15;
   const int ng = rw / RPG;
@@ -654,7 +658,7 @@ __global__ void __launch_bounds__((BCfg<NS, DT_>::TH), (BCfg<NS, DT_>::OCC)) mam
     gA[j] = 0.0f;
     lam_next[j] = 1.0f;  // no step after the last one; a segment's G starts as lam_{t+1} G_{t+1}
   }
-  compose_segments<NPT>(segs, n_segs - 1, seg, -1, B, b, D, d, N, [&](int j) { return j * NG + ng; }, act, A2, G);
+  if (SPLIT) compose_segments<NPT>(segs, n_segs - 1, seg, -1, B, b, D, d, N, [&](int j) { return j * NG + ng; }, act, A2, G);
   float gdp = 0.0f;
 
   // Row streams through buffer resources (see make_rsrc): a per-lane byte offset fixed for the
@@ -1072,14 +1076,10 @@ int launch_fwd(int64_t B, int64_t L, int64_t D, int64_t N, const void* draw, con
   const Split sp = segs ? fwd_split<NS>(B, L, D) : Split{1, L};
   if (sp.segs > 1) launch_segments<TIO, NS, false>(B, L, D, N, sp, draw, A, Bt, u, nullptr, segs, s);
   dim3 grid((unsigned)((D + C::DT - 1) / C::DT * B * sp.segs));
-  if (chk)
-    hipLaunchKernelGGL((mamba_fwd_kernel<TIO, NS, true>), grid, dim3(C::TH), 0, s, (const TIO*)draw, A,
-                       (const TIO*)Bt, (const TIO*)Ct, (const TIO*)u, (const TIO*)z, Dp, h0, (TIO*)out, h_last, chk,
-                       segs, B, L, D, (int)N, NC, sp.len, device_cus());
-  else
-    hipLaunchKernelGGL((mamba_fwd_kernel<TIO, NS, false>), grid, dim3(C::TH), 0, s, (const TIO*)draw, A,
-                       (const TIO*)Bt, (const TIO*)Ct, (const TIO*)u, (const TIO*)z, Dp, h0, (TIO*)out, h_last, chk,
-                       segs, B, L, D, (int)N, NC, sp.len, device_cus());
+  auto* const kernel = sp.segs > 1 ? (chk ? mamba_fwd_kernel<TIO, NS, true, true> : mamba_fwd_kernel<TIO, NS, false, true>)
+                                   : (chk ? mamba_fwd_kernel<TIO, NS, true, false> : mamba_fwd_kernel<TIO, NS, false, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(C::TH), 0, s, (const TIO*)draw, A, (const TIO*)Bt, (const TIO*)Ct, (const TIO*)u,
+                     (const TIO*)z, Dp, h0, (TIO*)out, h_last, chk, segs, B, L, D, (int)N, NC, sp.len, device_cus());
   return tsf_launch_status();
 }
 
@@ -1139,7 +1139,8 @@ int launch_bwd(int64_t B, int64_t L, int64_t D, int64_t N, const void* draw, con
   float* segs = gDp_part + rows * D;
   if (B > 0 && D > 0) {
     if (sp.segs > 1) launch_segments<TIO, NS, true>(B, L, D, N, sp, draw, A, Ct, gout, z, segs, s);
-    hipLaunchKernelGGL((mamba_bwd_kernel<TIO, NS, DT>), dim3((unsigned)(nT * rows)), dim3(C::TH), 0, s,
+    auto* const kernel = sp.segs > 1 ? mamba_bwd_kernel<TIO, NS, DT, true> : mamba_bwd_kernel<TIO, NS, DT, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(nT * rows)), dim3(C::TH), 0, s,
                        (const TIO*)draw, A, (const TIO*)Bt, (const TIO*)Ct, (const TIO*)u, (const TIO*)z, Dp, h0, chk,
                        (const TIO*)gout, ghlast, (TIO*)gdraw, (TIO*)gu, (TIO*)gz, gA_part, gDp_part, gBC_part, gh0,
                        segs, B, L, D, (int)N, NC, sp.segs, (sp.len + C::CHK - 1) / C::CHK, device_cus());
