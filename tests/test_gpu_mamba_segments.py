@@ -1,5 +1,5 @@
-"""The Mamba scan cut into time segments (few batch rows and channels, L >= 256) against the fp64
-oracle: segments that end off a round of 32 steps, a last segment of one step, partial channel
+"""The Mamba scan cut into time segments (few batch rows and channels; the backward from 256 steps, the
+forward from 384) against the fp64 oracle: segments that end off a round of 32 steps, a last segment of one step, partial channel
 tiles, every state tile, states padded up to one, with and without carried state and state
 gradient. Bars as for the whole walk: 1e-5 for fp32 I/O, 2e-2 for bf16."""
 
@@ -17,13 +17,13 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize(
     "B,L,D,N",
     [(1, 256, 20, 16), (2, 300, 40, 12), (1, 1000, 33, 4), (3, 515, 64, 32), (1, 700, 24, 64), (1, 1025, 16, 1),
-     (2, 2081, 70, 8), (40, 257, 160, 16), (1, 353, 1024, 16)],
+     (2, 2081, 70, 8), (40, 257, 160, 16), (1, 353, 1024, 16), (1, 385, 40, 16), (33, 769, 200, 8)],
 )
 @pytest.mark.parametrize("io", ["fp32", "bf16"])
 @pytest.mark.parametrize("carried", [True, False])
 def test_segments_match_oracle(gpu, B, L, D, N, io, carried):
     lib = _lib.load()
-    assert lib.tsfast_hip_mamba_fwd_workspace_bytes(B, L, D, N) > 0  # the shape is split
+    assert (lib.tsfast_hip_mamba_fwd_workspace_bytes(B, L, D, N) > 0) == (L >= 384)  # whether the forward is split
     io_dtype = torch.float32 if io == "fp32" else torch.bfloat16
     tol = 1e-5 if io == "fp32" else 2e-2
     t, gout, ghlast = _make(B, L, D, N, seed=L + D + N, io_dtype=io_dtype, with_h0=carried)
@@ -41,9 +41,33 @@ def test_segments_match_oracle(gpu, B, L, D, N, io, carried):
 def test_split_rule():
     lib = _lib.load()
     ws = lib.tsfast_hip_mamba_fwd_workspace_bytes
-    assert ws(1, 255, 64, 16) == 0 and ws(1, 256, 64, 16) == 4 * 4 * 64 * 17
+    assert ws(1, 383, 64, 16) == 0 and ws(1, 384, 64, 16) == 4 * 6 * 64 * 17
     assert ws(1, 4096, 1025, 16) == 0 and ws(1, 4096, 1024, 16) > 0
     assert ws(16, 4096, 1536, 16) == 0 and ws(1, 4096, 64, 65) == -1
+    # three segments: from 768 steps with a workgroup a CU (64 states: 384), never with two; never two segments
+    assert ws(64, 767, 128, 16) == 0 and ws(64, 768, 128, 16) == 4 * 3 * 64 * 128 * 17
+    assert ws(64, 383, 128, 64) == 0 and ws(64, 384, 128, 64) > 0
+    assert ws(128, 4096, 128, 4) == 0 and ws(96, 4096, 128, 4) > 0 and ws(96, 4096, 128, 16) == 0
+
+
+@pytest.mark.parametrize("D", [256, 1056])
+def test_row_alone_and_in_a_batch(gpu, D):
+    """Above 1024 channels a row gives the same bits alone and in a batch; below, where its segments
+    depend on the batch, the same values to fp32 rounding."""
+    B, L, N = 96 if D == 256 else 4, 600, 16
+    t, gout, _ = _make(B, L, D, N, seed=D, io_dtype=torch.float32, with_h0=False)
+    batch = _run_hip(t, gout, None, gpu, False)
+    one = {k: v[3:4] if v is not None and k not in ("A", "Dp") else v for k, v in t.items()}
+    alone = _run_hip(one, gout[3:4], None, gpu, False)
+    pairs = [(batch[0][3:4], alone[0]), (batch[1][3:4], alone[1])]
+    pairs += [(batch[2][k][3:4], alone[2][k]) for k in ("draw", "Bt", "Ct", "u", "z")]
+    for a, b in pairs:
+        if D > 1024:
+            assert torch.equal(a, b)
+        else:
+            assert O.rel_err(_np64(a), _np64(b)) < 1e-5
+    if D == 256:
+        assert not all(torch.equal(a, b) for a, b in pairs)  # the two were cut differently
 
 
 def test_growing_states_at_zero_stay_there(gpu):

@@ -1034,16 +1034,16 @@ struct Split {
   int64_t segs, len;
 };
 // Segments for a walk of `wgs` workgroups per segment of which `occ` fit a CU: as many as fill the
-// chip once, of at least 64 steps. Past that the maps cost more than the segments give (64 rows of
-// 1000 steps at D 256, two workgroups a CU: forward 91 us whole, 120 us in three segments).
-// Measured (fp32, N 16, whole -> split): 4 x 16384 x 256 inference 1120 -> 146 us and training
-// forward 1293 -> 184, backward 2970 -> 293 us; 8 x 2000 x 128 140 -> 31, 161 -> 32, 370 -> 54 us;
-// 64 x 512 x 128 44 -> 42, 48 -> 44, 107 -> 79 us.
-// Below 256 steps the second launch costs what the segments give. Rows of more than 1024 channels
-// are walked whole whatever the batch, so that such a row gives the same bits alone and in a batch.
-inline Split split_for(int64_t wgs, int64_t L, int64_t D, int occ) {
+// chip once, of at least 64 steps (past that the maps cost more than the segments give: 64 rows of 1000
+// steps at D 256, two workgroups a CU: forward 91 us whole, 120 us in three segments). Measured (fp32, N 16,
+// whole -> split): 4 x 16384 x 256 inference 1120 -> 146 us and training forward 1293 -> 184, backward
+// 2970 -> 293 us; 8 x 2000 x 128 140 -> 31, 161 -> 32, 370 -> 54 us. Where only two or three segments fit,
+// or the rows are short, the second pass over the inputs and its launch can cost more than they give:
+// fwd_split and bwd_split hold the lines. Rows of more than 1024 channels are walked whole whatever the
+// batch: such a row gives the same bits alone and in a batch, which narrower rows of 256 steps and more do
+// not, as their segments depend on the batch.
+inline Split split_for(int64_t segs, int64_t L, int64_t D) {
   constexpr int64_t kStep = 32, kMin = 64;
-  int64_t segs = wgs > 0 ? (int64_t)device_cus() * occ / wgs : 1;
   if (D > 1024 || segs < 2 || L < 4 * kMin) return {1, L};
   int64_t len = ((L + segs - 1) / segs + kStep - 1) / kStep * kStep;
   if (len < kMin) len = kMin;
@@ -1051,10 +1051,18 @@ inline Split split_for(int64_t wgs, int64_t L, int64_t D, int occ) {
   if (segs < 2) return {1, L};
   return {segs, len};
 }
+inline int64_t fill_segments(int64_t wgs, int occ) { return wgs > 0 ? (int64_t)device_cus() * occ / wgs : 1; }
+// Forward (kernel times, inference / training, split over whole): two segments 1.02-1.19 / 0.98-1.16 (D 128,
+// 96 rows of 256 .. 2048 steps, N 8 .. 64); three 1.02-1.12 / 0.95-1.10 up to 512 steps and 0.85-0.95 / 0.78-0.99
+// from 768 with a workgroup a CU (64 rows; N 64 0.90 / 0.87 from 384), and 0.90-1.10 / 1.04-1.16 with two (N 4,
+// 128 rows); four and more 0.66-0.97 / 0.62-0.99. Below 384 steps a call among others is bound by the host,
+// which the second launch and its workspace cost 4 us (16 x 256 x 128, inference: 27 -> 31 us).
 template <int NS>
 Split fwd_split(int64_t B, int64_t L, int64_t D) {
   using C = FCfg<NS>;
-  return split_for((D + C::DT - 1) / C::DT * B, L, D, C::OCC);
+  const int64_t wgs = (D + C::DT - 1) / C::DT * B, segs = fill_segments(wgs, C::OCC);
+  const bool pays = segs >= 4 || (segs == 3 && wgs <= (int64_t)device_cus() && L >= (NS == 64 ? 384 : 768));
+  return pays && L >= 384 ? split_for(segs, L, D) : Split{1, L};
 }
 
 template <typename TIO, int NS, bool ADJ>
@@ -1096,10 +1104,14 @@ constexpr int bwd_dt() {
   return NS >= 32 ? 16 : kBwdDT;
 }
 
+// Backward (as above): two segments 0.82-0.90 at N 16 and 0.72-0.83 at N 8 (96 rows), 0.62-0.67 at N 64 (32 rows,
+// one wave per SIMD), but 1.12-1.20 at N 32 (96 rows), where three give 0.90-0.98 from 384 steps and 1.02 at 256.
 template <int NS>
 Split bwd_split(int64_t B, int64_t L, int64_t D) {
   constexpr int DT = bwd_dt<NS>();
-  return split_for((D + DT - 1) / DT * B, L, D, NS == 64 ? 2 : BCfg<NS, DT>::OCC);  // N 64: one wave per SIMD
+  const int64_t segs = fill_segments((D + DT - 1) / DT * B, NS == 64 ? 2 : BCfg<NS, DT>::OCC);  // N 64: one wave per SIMD
+  const bool pays = NS != 32 || segs >= 4 || (segs == 3 && L >= 384);
+  return pays ? split_for(segs, L, D) : Split{1, L};
 }
 
 // Backward workspace: grad-B/C partials [nT, B, L, 2*NS] in the I/O type (padded to 256 bytes),
