@@ -17,7 +17,7 @@ import pytest
 import torch
 
 from oracle import scan_oracle as O
-from tsfast_amd import dispatch
+from tsfast_amd import _lib, dispatch
 from tsfast_amd.dynonet import core as dcore
 from tsfast_amd.dynonet import linrec_hip
 
@@ -208,3 +208,25 @@ def test_linrec_wide_row_stores(gpu, n, L):
     assert O.rel_err(_np(x), want) < TOL
     for t, w in zip(ts, (gA, gv, gx0)):
         assert O.rel_err(_np(t.grad), w) < TOL
+
+
+@pytest.mark.parametrize("n", [5, 6, 7, 8])
+@pytest.mark.parametrize("L", [1, 20, 256, 257])
+def test_linrec_wide_reads_nothing_it_has_not_written(gpu, n, L):
+    """A workspace of NaNs gives the same bits: a single chunk (L <= 256) forms no power of A and uses none."""
+    M = 9
+    A, v, x0, gx = (t.to(gpu) for t in _make(M, L, n, seed=L + n))
+    x = linrec_hip._linrec_op(A, v, x0)
+    gA, gv, gx0 = linrec_hip._linrec_bwd_op(gx, A, x, x0)
+    lib = _lib.load()
+    nbytes = lib.tsfast_hip_linrec_workspace_bytes(M, L, n)
+    got = [torch.empty_like(t) for t in (x, gA, gv, gx0)]
+    p = _lib.ptr
+    ws = torch.full((nbytes // 8,), float("nan"), dtype=torch.float64, device=gpu)
+    _lib.check(lib.tsfast_hip_linrec_fwd(M, L, n, p(A), p(v), p(x0), p(got[0]), p(ws), nbytes, _lib.stream_of(v)), "fwd")
+    ws.fill_(float("nan"))
+    _lib.check(
+        lib.tsfast_hip_linrec_bwd(M, L, n, p(gx), p(A), p(x), p(x0), p(got[1]), p(got[2]), p(got[3]), p(ws), nbytes,
+                                  _lib.stream_of(v)), "bwd")
+    for a, b in zip(got, (x, gA, gv, gx0)):
+        assert torch.equal(a, b)

@@ -931,13 +931,14 @@ __global__ void __launch_bounds__(64) lw_carry(const float* __restrict__ A, cons
   if (lane >= lanes) return;  // both threads of a pair
   double mo[NH][NH], mp[NH][NH], s[NH];
   const double* m = M + lane * NS * NS;
+  const bool chain = nchunks > 1;  // a single chunk has nothing to carry on: M is not formed then
 #pragma unroll
   for (int j = 0; j < NH; ++j) {
     const bool row = own0 + j < NS;
 #pragma unroll
     for (int i = 0; i < NH; ++i) {
-      mo[j][i] = (row && own0 + i < NS) ? m[(own0 + j) * NS + own0 + i] : 0.0;
-      mp[j][i] = (row && par0 + i < NS) ? m[(own0 + j) * NS + par0 + i] : 0.0;
+      mo[j][i] = (chain && row && own0 + i < NS) ? m[(own0 + j) * NS + own0 + i] : 0.0;
+      mp[j][i] = (chain && row && par0 + i < NS) ? m[(own0 + j) * NS + par0 + i] : 0.0;
     }
     s[j] = (!ADJ && x0 && row) ? (double)x0[lane * NS + own0 + j] : 0.0;
   }
@@ -1147,14 +1148,16 @@ int wide_out_vec(const float* p, int64_t row) {
 }
 
 // A sum kernel's grid: NS rows for M, then a row per chunk; two launches where that is more than a
-// grid's 65535 rows.
+// grid's 65535 rows. A single chunk needs no M: its 256 steps were what a short call waited for (8 lanes x
+// 20 steps, n 5, forward + backward 63 us with M in a launch of its own, 82 beside the chunk).
 template <int NS, typename F>
 void sum_launch(F kernel, unsigned gx, int64_t nchunks, hipStream_t s, const float* A, const float* in, double* out,
                 double* M, int64_t lanes, int64_t L) {
-  const bool one = nchunks + NS <= 65535;
-  if (!one) hipLaunchKernelGGL(kernel, dim3(gx, NS), dim3(kWideThreads), 0, s, A, in, out, M, lanes, L, (unsigned)NS);
-  hipLaunchKernelGGL(kernel, dim3(gx, (unsigned)nchunks + (one ? NS : 0)), dim3(kWideThreads), 0, s, A, in, out, M,
-                     lanes, L, one ? (unsigned)NS : 0u);
+  const unsigned rows = nchunks > 1 ? NS : 0;
+  const bool one = nchunks + rows <= 65535;
+  if (!one) hipLaunchKernelGGL(kernel, dim3(gx, rows), dim3(kWideThreads), 0, s, A, in, out, M, lanes, L, rows);
+  hipLaunchKernelGGL(kernel, dim3(gx, (unsigned)nchunks + (one ? rows : 0)), dim3(kWideThreads), 0, s, A, in, out, M,
+                     lanes, L, one ? rows : 0u);
 }
 
 template <int NS, int VEC>
