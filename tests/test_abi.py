@@ -78,6 +78,10 @@ def test_size_queries(lib):
     # [lanes][n][n]: n = 2 has 16-step chunks, 8 of them a tile, so nsuper = 1 and ceil(300 / 128)
     assert lib.tsfast_hip_linrec_workspace_bytes(64, 100, 2) == 256 + 8 * (1 * 64 * (2 + 2 + 4) + 2 * 64 * 4)
     assert lib.tsfast_hip_linrec_workspace_bytes(64, 300, 2) == 256 + 8 * (3 * 64 * (2 + 2 + 4) + 2 * 64 * 4)
+    # fewer chunks a tile where a tile is slow and the rows short, on each side of the lines: order 4 ..
+    lr = lib.tsfast_hip_linrec_workspace_bytes
+    for lanes, L, nsuper in ((64, 400, 7), (65, 400, 13), (65, 401, 7), (4032, 400, 13), (4033, 400, 7), (4033, 96, 3), (4033, 97, 2)):
+        assert lr(lanes, L, 4) == 256 + 8 * (nsuper * lanes * (4 + 4 + 16) + 2 * lanes * 16)
     # n = 5..8: e/f and carries [chunks][lanes][n], the lane matrices and the grad_A partials
     assert lib.tsfast_hip_linrec_workspace_bytes(4, 300, 5) == 8 * (2 * 2 * 4 * 5 + 4 * 25 + 2 * 4 * 25)
     # n = 9..16 (spread path): the same areas with the same 256-step chunks

@@ -52,6 +52,10 @@ _SHAPES = [
     (1, 20000, 1),  # one lane, a long look-back chain
     (33, 1, 2),  # L = 1
     (96, 5000, 2),
+    (65, 400, 4),  # order 4, more than one lane group up to 400 steps: 4 chunks a tile
+    (65, 401, 4),
+    (4097, 96, 4),  # 64 lane groups and more: up to 96 steps
+    (4097, 97, 4),
     # n = 5..8: the two-pass path (chunks of 256 steps)
     (5, 40, 5),
     (70, 1000, 6),  # ragged last chunk, one lane block (256 lanes per block)

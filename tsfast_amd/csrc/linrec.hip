@@ -474,7 +474,11 @@ __global__ void __launch_bounds__(256) linrec_zero(float* __restrict__ p, int64_
 }
 
 // Plan: kLbWaves chunks per tile as lb_plan (32 lanes x 1000 steps, n 4: forward / backward 76 / 83 us
-// at 2 chunks a tile, 22 / 31 at 8). Workspace: the tile counter, agg and inc [nsuper][lanes][n] (reset
+// at 2 chunks a tile, 22 / 31 at 8). Order 4's tiles are the slowest, and on short sequences half of them
+// side by side win over one look-back fewer (8 -> 4 chunks a tile, backward: 1024 lanes x 64 steps 50 -> 41
+// us, 250 steps 55 -> 45, 400 steps 51 -> 48; 800 steps of 64 .. 1024 lanes 0.91 but forward 1.09-1.17; up
+// to 64 lanes x 100 steps 1.14); full rows of lanes only up to 12 chunks (4096 x 64: 53 -> 44; 150: 1.01).
+// Workspace: the tile counter, agg and inc [nsuper][lanes][n] (reset
 // before each scan), the grad_A partials [nsuper][lanes][n][n], and Mc, Ms [lanes][n][n].
 struct LrPlan {
   int64_t groups = 0, nsuper = 0;
@@ -488,7 +492,9 @@ LrPlan lr_plan(int64_t lanes, int64_t L, int64_t ns) {
   p.groups = (lanes + kTile - 1) / kTile;
   if (L > 0) {
     const int64_t chunks = (L + S - 1) / S;
-    p.K = chunks < kLbWaves ? (int)chunks : kLbWaves;
+    const bool half = ns == 4 && p.groups > 1 && chunks <= (p.groups < kTile ? 50 : 12);
+    const int64_t most = half ? kLbWaves / 2 : kLbWaves;
+    p.K = (int)(chunks < most ? chunks : most);
     p.nsuper = (L + S * p.K - 1) / (S * p.K);
   }
   const size_t f = 8, vecs = f * p.nsuper * lanes * ns;
