@@ -82,6 +82,9 @@ def test_size_queries(lib):
     lr = lib.tsfast_hip_linrec_workspace_bytes
     for lanes, L, nsuper in ((64, 400, 7), (65, 400, 13), (65, 401, 7), (4032, 400, 13), (4033, 400, 7), (4033, 96, 3), (4033, 97, 2)):
         assert lr(lanes, L, 4) == 256 + 8 * (nsuper * lanes * (4 + 4 + 16) + 2 * lanes * 16)
+    ap = lib.tsfast_hip_allpole_workspace_bytes
+    for na, L, nsuper in ((4, 256, 2), (4, 257, 2), (3, 256, 1), (4, 129, 2), (4, 128, 1)):
+        assert ap(70, L, na) == 256 + 8 * (nsuper * 70 * 3 * na + 2 * 70 * na * na)
     # n = 5..8: e/f and carries [chunks][lanes][n], the lane matrices and the grad_A partials
     assert lib.tsfast_hip_linrec_workspace_bytes(4, 300, 5) == 8 * (2 * 2 * 4 * 5 + 4 * 25 + 2 * 4 * 25)
     # n = 9..16 (spread path): the same areas with the same 256-step chunks

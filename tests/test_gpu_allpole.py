@@ -25,6 +25,8 @@ _SHAPES = [
     (2, 4, 1, 2),
     (2, 4, 2, 4),
     (1, 1, 513, 1),
+    (2, 40, 256, 4),  # order 4 up to 256 steps: 4 chunks a tile
+    (2, 40, 257, 4),
     (2, 3, 300, 16),
     (8, 64, 16384, 3),  # config 4 with the batch reduced from 64 to 8
     # single-pass look-back path (na <= 4): many super-chunks, lanes off multiples of 64,

@@ -66,6 +66,8 @@ _SHAPES = [
     (1, 2, 2, 2, 3, 4),  # L < na
     (2, 1, 8, 8, 8, 2),  # L = 1
     (5, 1000, 2, 2, 5, 1),
+    (4, 416, 8, 8, 8, 3),  # 256 lanes, 416 steps: 4 chunks a tile
+    (4, 417, 8, 8, 8, 3),
     (6, 2049, 1, 8, 2, 3),
     (4, 4096, 8, 8, 8, 3),  # config-4 channel structure, reduced batch and length
     # lanes beyond one tile, not a multiple of 64: the second tile holds a partial lane group

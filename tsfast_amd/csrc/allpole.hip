@@ -693,11 +693,15 @@ Plan plan(int64_t lanes, int64_t L, int64_t na) {
   return p;
 }
 
+// Order 4 up to 256 steps: two tiles of at most 4 chunks beat one of 8 (296 lanes x 150 steps, forward /
+// backward 26 / 34 us for 27 / 38; 250 steps 26 / 33 for 29 / 35); orders 1 .. 3 and longer rows 0.98-1.15.
+inline int tile_chunks(int64_t L, int64_t na) { return na == 4 && L <= 8 * kTileT ? kLbWaves / 2 : kLbWaves; }
+
 template <int NA>
 void fwd_lb(int64_t lanes, int64_t L, const float* a, const float* w, const float* y0, float* y, char* ws,
             hipStream_t s) {
   static int occ[kMaxNA + 1];
-  const LbPlan p = lb_plan(lanes, L, NA);
+  const LbPlan p = lb_plan(lanes, L, NA, tile_chunks(L, NA));
   double* Mc = reinterpret_cast<double*>(ws + p.off_Mc);
   double* Ms = reinterpret_cast<double*>(ws + p.off_Ms);
   const ResetJob rj = reset_job(ws, 2 * p.nsuper * lanes * NA, 64);
@@ -714,7 +718,7 @@ template <int NA>
 void bwd_lb(int64_t lanes, int64_t L, const float* g, const float* a, const float* y, const float* y0, float* gw,
             float* ga, float* gy0, char* ws, hipStream_t s) {
   static int occ[kMaxNA + 1];
-  const LbPlan p = lb_plan(lanes, L, NA);
+  const LbPlan p = lb_plan(lanes, L, NA, tile_chunks(L, NA));
   double* part = reinterpret_cast<double*>(ws + p.off_part);
   if (L > 0) {
     double* Mc = reinterpret_cast<double*>(ws + p.off_Mc);
@@ -744,7 +748,7 @@ void transfer_launch(const Plan& p, const float* a, double* M, int64_t lanes, hi
 }
 
 size_t workspace_bytes_for(int64_t lanes, int64_t L, int64_t na) {
-  return na <= kLbNA ? lb_plan(lanes, L, na).bytes : plan(lanes, L, na).bytes;
+  return na <= kLbNA ? lb_plan(lanes, L, na, tile_chunks(L, na)).bytes : plan(lanes, L, na).bytes;
 }
 
 template <int NA>

@@ -395,9 +395,10 @@ TSF_DEV void regs_to_chunk(const float (&xb)[kTileT], float* __restrict__ dst, i
 
 // Tile plan of the single-pass path: kLbWaves chunks per tile (all of a shorter sequence's). Halving
 // them to reach one tile per CU, as few lanes once did, lengthens the chain of look-backs by more than
-// the extra workgroups shorten the tiles, at every size measured: all-pole order 3, 64 lanes x 16000
-// steps, forward / backward 222 / 233 us at 2 chunks a tile, 39 / 47 at 8; G-block 8 rows x 16000, one
-// pair, 371 / 483 and 46 / 77 us (with the anchors below). Workspace: the tile counter, agg and inc
+// the extra workgroups shorten the tiles: all-pole order 3, 64 lanes x 16000 steps, forward / backward
+// 222 / 233 us at 2 chunks a tile, 39 / 47 at 8; G-block 8 rows x 16000, one pair, 371 / 483 and 46 / 77 us
+// (with the anchors below). Where a tile is slow and the sequence a tile or two long, half the chunks
+// (`most`, the callers' rules) win. Workspace: the tile counter, agg and inc
 // [nsuper][lanes][NA] (reset before each scan), the grad_a partials [nsuper][lanes][NA], and
 // the transfer matrices Mc, Ms [lanes][NA][NA].
 struct LbPlan {
@@ -406,12 +407,12 @@ struct LbPlan {
   size_t off_agg = 0, off_inc = 0, off_part = 0, off_Mc = 0, off_Ms = 0, bytes = 0;
 };
 
-LbPlan lb_plan(int64_t lanes, int64_t L, int64_t na) {
+LbPlan lb_plan(int64_t lanes, int64_t L, int64_t na, int most) {
   LbPlan p;
   p.groups = (lanes + kTile - 1) / kTile;
   if (L > 0) {
     const int64_t chunks = (L + kTileT - 1) / kTileT;
-    p.K = chunks < kLbWaves ? (int)chunks : kLbWaves;
+    p.K = chunks < most ? (int)chunks : most;
     p.nsuper = (L + (int64_t)kTileT * p.K - 1) / ((int64_t)kTileT * p.K);
   }
   const size_t f = 8, vecs = f * p.nsuper * lanes * na;
