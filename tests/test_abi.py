@@ -85,6 +85,13 @@ def test_size_queries(lib):
     ap = lib.tsfast_hip_allpole_workspace_bytes
     for na, L, nsuper in ((4, 256, 2), (4, 257, 2), (3, 256, 1), (4, 129, 2), (4, 128, 1)):
         assert ap(70, L, na) == 256 + 8 * (nsuper * 70 * 3 * na + 2 * 70 * na * na)
+    # .. the complex backward's tiles (16 steps a chunk; words of 16 bytes), and selective rows of few lanes
+    dg, sl = lib.tsfast_hip_diag_workspace_bytes, lib.tsfast_hip_sel_workspace_bytes
+    for M, L, nsuper in ((4, 1536, 24), (4, 1537, 13), (5, 1536, 12), (16, 2560, 20), (16, 2561, 11), (17, 2560, 10)):
+        assert dg(M, L, 64, 1) == 256 + 4 * nsuper * M * 64 * 16
+    for M, L, N, nsuper in ((16, 2048, 1, 32), (16, 2049, 1, 17), (15, 2048, 1, 8), (16, 8193, 1, 33), (64, 600, 4, 10), (64, 600, 5, 5),
+                            (64, 1024, 16, 8), (64, 1025, 16, 5), (64, 256, 16, 1), (65, 600, 16, 3)):
+        assert sl(M, L, N) == 256 + nsuper * M * N * 24
     # n = 5..8: e/f and carries [chunks][lanes][n], the lane matrices and the grad_A partials
     assert lib.tsfast_hip_linrec_workspace_bytes(4, 300, 5) == 8 * (2 * 2 * 4 * 5 + 4 * 25 + 2 * 4 * 25)
     # n = 9..16 (spread path): the same areas with the same 256-step chunks

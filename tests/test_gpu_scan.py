@@ -45,6 +45,13 @@ _DIAG_SHAPES = [
     # the look-back: ragged lanes and last chunk; and a long look-back with 128 super-chunks
     ((3, 3000, 70), (70,)),
     ((6, 8192, 100), (100,)),
+    # the complex backward's fewer chunks a tile: 4 up to 256 lanes and 1536 steps, 8 up to 1024 and 2560
+    ((4, 1536, 64), (64,)),
+    ((4, 1537, 64), (64,)),
+    ((2, 1500, 129), (129,)),
+    ((16, 2560, 64), (64,)),
+    ((16, 2561, 64), (64,)),
+    ((15, 900, 69), (69,)),
 ]
 
 
@@ -113,7 +120,9 @@ def test_diag_inference_equals_grad_path(gpu):
 # (1, 3000, 24): more than 16 super-chunks (cooperative carry kernel); (16, 2048, 512): 32-step
 # forward chunks
 @pytest.mark.parametrize(
-    "shape", [(2, 7, 3), (4, 257, 8), (2, 1, 3), (3, 5000, 40), (8, 1024, 128), (1, 3000, 24), (16, 2048, 512)]
+    "shape", [(2, 7, 3), (4, 257, 8), (2, 1, 3), (3, 5000, 40), (8, 1024, 128), (1, 3000, 24), (16, 2048, 512),
+              # fewer chunks a tile: rows of few lanes (4 up to 2048 steps, 8 up to 8192), short rows (8)
+              (16, 2048, 1), (16, 2049, 1), (48, 600, 3), (65, 8193, 2), (3, 600, 40), (16, 1025, 5)]
 )
 @pytest.mark.parametrize("with_x0", [True, False])
 def test_selective_matches_oracle(gpu, shape, with_x0):

@@ -891,8 +891,8 @@ __global__ void __launch_bounds__(1024) diag_sum_shared(const typename Wide<T>::
 // kDiagWaveTarget waves. K (chunks per tile) is TSF_DIAG_KMAX, or the chunks of a shorter sequence:
 // halving it to reach a tile per CU, as few lanes once did, lengthens the chain of look-backs by more
 // than the extra workgroups shorten the tiles (4 rows x 8192 steps x 32 lanes, forward / backward:
-// complex 58 / 64 us at 4 chunks a tile, 21 / 27 at 16; real 46 / 48 and 15 / 19; no size measured was
-// slower at 16).
+// complex 58 / 64 us at 4 chunks a tile, 21 / 27 at 16; real 46 / 48 and 15 / 19), except where a tile is
+// slow by itself and the rows are short: `most`, from const_tile and sel_tile.
 #ifndef TSF_DIAG_WAVE_TARGET
 #define TSF_DIAG_WAVE_TARGET 4096
 #endif
@@ -907,14 +907,14 @@ struct DiagTile {
   int TC = 0, K = 0;
 };
 
-DiagTile diag_tile(int64_t lanes, int64_t L, int tc_max) {
+DiagTile diag_tile(int64_t lanes, int64_t L, int tc_max, int most) {
   DiagTile t;
   t.lanes = lanes;
   if (lanes < 1 || L < 1) return t;
   t.groups = (lanes + 63) / 64;
   t.TC = (t.groups * ((L + 31) / 32) < kDiagWaveTarget) ? 16 : 32;
   if (t.TC > tc_max) t.TC = tc_max;
-  t.K = TSF_DIAG_KMAX;
+  t.K = most;
   const int64_t chunks = (L + t.TC - 1) / t.TC;
   if (t.K > chunks) t.K = (int)chunks;  // no waves past the end of a short sequence
   t.SL = (int64_t)t.TC * t.K;
@@ -922,11 +922,32 @@ DiagTile diag_tile(int64_t lanes, int64_t L, int tc_max) {
   return t;
 }
 
+inline int fewer(int k) { return k < TSF_DIAG_KMAX ? k : TSF_DIAG_KMAX; }
+
+// The complex backward is the slowest tile. Chunks per tile 4 / 8 against 16, few lane groups (means over 1 ..
+// 16 rows of 3 .. 200 lanes): up to 4 groups 0.93 / 0.97 at 1000 steps, 0.80 / 0.84 at 1500, 0.94 / 0.88 at 2500
+// and 1.38 / 0.91 at 6000; 5 .. 16 groups 0.84 / 0.85, 0.96 / 0.89, 1.20 / 0.95 and 1.71 / 1.18; more groups 1.08
+// and more at 8. Forward and real lanes: 0.96-1.02 up to 1000 steps, 1.0-1.3 beyond.
 DiagTile const_tile(int64_t lanes, int64_t L, bool cplx, bool bwd) {
-  (void)bwd;
-  return diag_tile(lanes, L, cplx ? 16 : 32);
+  int most = TSF_DIAG_KMAX;
+  if (cplx && bwd && lanes <= 64 * 16 && L <= 2560) most = fewer(lanes <= 64 * 4 && L <= 1536 ? 4 : 8);
+  return diag_tile(lanes, L, cplx ? 16 : 32, most);
 }
-DiagTile sel_tile(int64_t lanes, int64_t L, bool bwd) { return diag_tile(lanes, L, bwd ? 16 : 32); }
+// Rows of few lanes (N): a wave's 64 lanes lie in as many rows as fit, its loads touch a line per row and
+// step, and one CU's address unit bounds the tile; smaller tiles use more CUs. 16 and more rows a wave, chunks
+// per tile 4 / 8 / 16, forward and backward: 64 x 600 steps, N 1 21 / 25 / 36 and 27 / 34 / 52 us; 48 x 1000, N 3
+// 22 / 22 / 29 and 25 / 28 / 41; x 2500 28 / 25 / 30 and 31 / 31 / 42; 64 x 8000, N 1 54 / 38 / 42 and 59 / 47 / 61.
+// Other rows: 8 for 16 0.95-0.98 backward and 0.98-1.0 forward from 300 to 1000 steps up to 16 lane groups, 1.0-1.3
+// beyond either.
+DiagTile sel_tile(int64_t lanes, int64_t L, int64_t N, bool bwd) {
+  const bool many_rows = 16 * N <= (lanes < 64 ? lanes : 64);
+  int most = TSF_DIAG_KMAX;
+  if (many_rows)
+    most = fewer(L <= 2048 ? 4 : L <= 8192 ? 8 : TSF_DIAG_KMAX);
+  else if (lanes <= 64 * 16 && L > 256 && L <= 1024)
+    most = fewer(8);
+  return diag_tile(lanes, L, bwd ? 16 : 32, most);
+}
 
 inline bool grid_fits(const DiagTile& t) { return t.groups * t.nsuper <= INT32_MAX; }
 
@@ -1257,7 +1278,7 @@ int tsfast_hip_diag_fwd_noalloc(int64_t M, int64_t L, int64_t N, int is_complex,
 int64_t tsfast_hip_sel_workspace_bytes(int64_t M, int64_t L, int64_t N) {
   // counter, then fp64 look-back maps (P, e) and states, 3 words per lane and super-chunk, for
   // the larger of the forward / backward tilings
-  const DiagTile f = sel_tile(M * N, L, false), b = sel_tile(M * N, L, true);
+  const DiagTile f = sel_tile(M * N, L, N, false), b = sel_tile(M * N, L, N, true);
   return kCounterBytes + (f.nsuper > b.nsuper ? f.nsuper : b.nsuper) * M * N * 24;
 }
 
@@ -1267,7 +1288,7 @@ int tsfast_hip_sel_fwd(int64_t M, int64_t L, int64_t N, const float* a, const fl
   if (M == 0 || L == 0 || N == 0) return TSF_OK;
   if (!a || !v || !out) return TSF_ERR_ARG;
   if (workspace_bytes < tsfast_hip_sel_workspace_bytes(M, L, N) || !workspace) return TSF_ERR_WORKSPACE;
-  const DiagTile t = sel_tile(M * N, L, false);
+  const DiagTile t = sel_tile(M * N, L, N, false);
   if (!grid_fits(t)) return TSF_ERR_UNSUPPORTED;
   hipStream_t s = static_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
@@ -1292,7 +1313,7 @@ int tsfast_hip_sel_bwd(int64_t M, int64_t L, int64_t N, const float* g, const fl
   }
   if (!g || !a || !out || !gv || !glam) return TSF_ERR_ARG;
   if (workspace_bytes < tsfast_hip_sel_workspace_bytes(M, L, N) || !workspace) return TSF_ERR_WORKSPACE;
-  const DiagTile t = sel_tile(lanes, L, true);
+  const DiagTile t = sel_tile(lanes, L, N, true);
   if (!grid_fits(t)) return TSF_ERR_UNSUPPORTED;
   sel_bwd_launch(t, g, a, out, x0, glam, gv, gx0, static_cast<char*>(workspace), L, N, s);
   return tsf_launch_status();
