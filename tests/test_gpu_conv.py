@@ -134,26 +134,46 @@ def test_conv_supports_reasons(gpu):
     assert "GPU-only" in conv_hip.supports(x.cpu(), tail.cpu(), w.cpu(), None)
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("K", [2, 4, 5])
-@pytest.mark.parametrize("D", [3, 4, 5, 7, 8, 9, 17, 254, 255, 257, 263, 509])
-def test_conv_rows_of_any_alignment(gpu, D, K, dtype):
-    """16-byte pieces at any alignment (channel stride 1) against the element path (any other channel
-    stride): the same arithmetic in the same order, so the same bits. The view ends where its storage
-    ends, and its rows start at every alignment; widths from under one piece to several blocks."""
-    B, L, off = 2, 131, 1
+def _rows_and_columns(gpu, B, L, D, K, dtype):
+    """The conv's outputs and gradients on the same values in rows at every alignment (a view that ends
+    where its storage ends) and with a channel stride other than 1 (the element path)."""
     g = torch.Generator().manual_seed(D * 10 + K)
-    wide = torch.randn(B, L, off + D, generator=g).to(gpu, dtype)
-    rows = wide[..., off:]
+    rows = torch.randn(B, L, 1 + D, generator=g).to(gpu, dtype)[..., 1:]
     columns = rows.transpose(1, 2).contiguous().transpose(1, 2)
+    assert rows.stride(2) == 1 and columns.stride(2) != 1
     tail = torch.randn(B, D, K - 1, generator=g).to(gpu, dtype)
     weight, bias = (torch.randn(D, 1, K, generator=g) * 0.5).to(gpu), torch.randn(D, generator=g).to(gpu)
     gy = torch.randn(B, L, D, generator=g).to(gpu, dtype)
     results = []
     for x in (rows, columns):
-        assert x.stride(2) == 1 or x is columns
         leaves = [t.detach().requires_grad_() for t in (x, tail, weight, bias)]
         y = conv_hip.run(*leaves)
         results.append((y, *torch.autograd.grad(y, leaves, gy)))
-    for a, b in zip(*results):
+    return (rows, tail, weight, bias, gy), results
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("K", [2, 4, 5])
+@pytest.mark.parametrize("D", [3, 4, 5, 7, 8, 9, 17, 254, 255, 257, 263, 509])
+def test_conv_rows_of_any_alignment(gpu, D, K, dtype):
+    """Widths from under one 16-byte piece to several blocks against the oracle, and bit for bit against
+    the element path: the same arithmetic in the same order (bf16 goes by pieces at these sizes, fp32 by
+    one channel a thread or by elements)."""
+    (x, tail, weight, bias, gy), (rows, columns) = _rows_and_columns(gpu, 2, 131, D, K, dtype)
+    for a, b in zip(rows, columns):
+        assert torch.equal(a, b)
+    x, tail, weight, bias, gy = (_np(t) for t in (x, tail, weight[:, 0], bias, gy))
+    tol = 1e-5 if dtype == torch.float32 else 2e-2
+    assert O.rel_err(_np(rows[0]), O.conv_silu_forward(x, tail, weight, bias)) < tol
+    for name, a, b in zip(("x", "tail", "weight", "bias"), rows[1:], O.conv_silu_backward(gy, x, tail, weight, bias)):
+        assert O.rel_err(_np(a).reshape(b.shape), b) < tol, name
+
+
+@pytest.mark.parametrize("K", [2, 4, 5, 7])
+@pytest.mark.parametrize("D", [254, 255, 509])
+def test_conv_fp32_by_pieces_on_many_rows(gpu, D, K):
+    """fp32 rows of any alignment with enough workgroups for the CUs, where both directions go by pieces
+    (the backward of K 5 and 7 beyond 256 channels): the element path's bits."""
+    _, (rows, columns) = _rows_and_columns(gpu, 64, 397, D, K, torch.float32)
+    for a, b in zip(rows, columns):
         assert torch.equal(a, b)

@@ -674,13 +674,24 @@ ConvPlan conv_plan(int64_t L, int64_t D) {
   return p;
 }
 
-// y, z: the contiguous [B, L, D] tensors read or written the same way, or NULL.
+// y, z: the contiguous [B, L, D] tensors read or written the same way, or NULL. The fp32 tiled backward (5 and
+// more taps) takes unaligned rows by pieces only beyond 256 channels and one workgroup a CU: there they run
+// 0.83-0.95 of the element loads' time (means over D 257 .. 1025 by grid size; K 8 0.78-0.89), with fewer
+// workgroups 1.09-1.16, and at 256 channels and less 1.0-1.3 (64 x 2000 steps, D 129, K 5 83 -> 100 us). bf16
+// rows, twice the channels a piece, gain at every size (0.40-0.98).
 template <typename TIO>
 Rows rows_of(const void* x, int64_t D, int64_t sxb, int64_t sxl, int64_t sxd, const void* y, const void* z) {
   constexpr int64_t VE = 16 / sizeof(TIO);
   const uintptr_t a = (uintptr_t)x | (uintptr_t)y | (uintptr_t)z;
   if (sxd != 1 || D < VE) return kElements;
   return D % VE == 0 && sxl % VE == 0 && sxb % VE == 0 && a % 16 == 0 ? kAligned : kRuns;
+}
+Rows rows_of_f32_bwd(int64_t B, int64_t L, int64_t D, const void* x, int64_t sxb, int64_t sxl, int64_t sxd, const void* y,
+                     const void* z) {
+  const Rows rows = rows_of<float>(x, D, sxb, sxl, sxd, y, z);
+  const ConvPlan p = conv_plan(L, D);
+  const bool runs = D > kCh && p.cblocks * p.nseg * B > (int64_t)device_cus();
+  return rows == kRuns && !runs ? kElements : rows;
 }
 
 template <typename TIO, int K>
@@ -728,16 +739,27 @@ RegPlan reg_plan(int64_t L, int64_t D, int vec, int run_len, int runs_per_group)
 
 // Vector width 4 (both passes) when rows of x are runs of at least one channel group. Rows that are not
 // whole aligned groups went one channel a thread before: at 16 x 4096 steps, D 1531, K 4, forward and
-// forward + backward took 233 and 568 us, now 185 and 480 (157 and 407 at D 1536). They still do where the
-// wider groups would leave more than a third of the lanes without a channel: 170 us against 192 at 50 x
-// 2000 steps, D 303 (320 lanes of one channel, or 128 of four for 76 groups), K 3. The tail, weights and
-// bias are read per channel either way.
-int vec_for(const void* x, int64_t D, int64_t sxb, int64_t sxl, int64_t sxd, const void* y, const void* z) {
+// forward + backward took 233 and 568 us, now 185 and 480 (157 and 407 at D 1536). They still do
+//  - where the wider groups would leave more than a third of the lanes without a channel: 170 us against
+//    192 at 50 x 2000 steps, D 303 (320 lanes of one channel, or 128 of four for 76 groups), K 3;
+//  - where their workgroups, blocks at least half full counted, reach no more than three CUs in four, or
+//    six in four beside a last block of fewer lanes, whose workgroups are the slowest (`fills` false):
+//    forward 0.94-2.4 of the time by channel (1 x 1000 steps, K 4, D 255 3.3 us by channel and 4.4 by groups,
+//    D 771 3.7 and 9.0; 16 x 500 x 255 4.9 and 5.3; 1 x 4000 x 1025, K 8, 8.8 and 12.1), backward 1.0-2.6
+//    (4 x 500, K 4, D 513 17 and 43 us; 16 x 500 x 771 32 and 37). Beyond, 0.64-1.02 and 0.8-1.07.
+// The tail, weights and bias are read per channel either way.
+int vec_for(const void* x, int64_t D, int64_t sxb, int64_t sxl, int64_t sxd, const void* y, const void* z, bool fills) {
   if (sxd != 1 || D < 4) return 1;
   const uintptr_t a = (uintptr_t)x | (uintptr_t)y | (uintptr_t)z;
   if (D % 4 == 0 && sxl % 4 == 0 && sxb % 4 == 0 && a % 16 == 0) return 4;
   const int64_t lanes4 = (D + 4 * kCgWg - 1) / (4 * kCgWg) * 4 * kCgWg, lanes1 = (D + kCgWg - 1) / kCgWg * kCgWg;
-  return 2 * lanes4 <= 3 * lanes1 ? 4 : 1;
+  return fills && 2 * lanes4 <= 3 * lanes1 ? 4 : 1;
+}
+bool groups_fill(int64_t B, int64_t L, int64_t D, bool bwd) {
+  constexpr int64_t kWide = 4 * kCgWg;
+  const RegPlan p = bwd ? reg_plan(L, D, 4, kRunB, kRunsWg * kRpt) : reg_plan(L, D, 4, kRun, kRunsWg);
+  const int64_t rest = D % kWide, need = rest > 0 && rest < kWide / 2 ? 6 : 3;
+  return 4 * ((D + kWide / 2) / kWide * p.run_groups * B) > need * (int64_t)device_cus();
 }
 
 template <typename TIO, int K, int VEC>
@@ -841,7 +863,7 @@ int tsfast_hip_conv_silu_fwd(int64_t B, int64_t L, int64_t D, int64_t K, int io_
   if (const int st = conv_layout_status(L, D, sxl, sxd, io_dtype == TSF_DTYPE_BF16 ? 2 : 4)) return st;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (io_dtype == TSF_DTYPE_F32) {
-    const int vec = vec_for(x, D, sxb, sxl, sxd, out, nullptr);
+    const int vec = vec_for(x, D, sxb, sxl, sxd, out, nullptr, groups_fill(B, L, D, false));
 #define CALL(KK) fwd_reg<float, KK>(vec, B, L, D, x, sxb, sxl, sxd, tail, weight, bias, out, s)
     TSF_CONV_K_SWITCH(K, CALL)
 #undef CALL
@@ -877,12 +899,12 @@ int tsfast_hip_conv_silu_bwd(int64_t B, int64_t L, int64_t D, int64_t K, int io_
   if (const int st = conv_layout_status(L, D, sxl, sxd, io_dtype == TSF_DTYPE_BF16 ? 2 : 4)) return st;
   float* part = static_cast<float*>(workspace);
   if (io_dtype == TSF_DTYPE_F32 && K >= TSF_CONV_F32_TILED_K) {
-    const Rows rows = rows_of<float>(x, D, sxb, sxl, sxd, gy, gx);
+    const Rows rows = rows_of_f32_bwd(B, L, D, x, sxb, sxl, sxd, gy, gx);
 #define CALL(KK) bwd_k<float, KK>(rows, B, L, D, x, sxb, sxl, sxd, tail, weight, bias, gy, gx, gtail, gw, gb, part, s)
     TSF_CONV_K_SWITCH(K, CALL)
 #undef CALL
   } else if (io_dtype == TSF_DTYPE_F32) {
-    const int vec = vec_for(x, D, sxb, sxl, sxd, gy, gx);
+    const int vec = vec_for(x, D, sxb, sxl, sxd, gy, gx, groups_fill(B, L, D, true));
 #define CALL(KK) bwd_reg<float, KK>(vec, B, L, D, x, sxb, sxl, sxd, tail, weight, bias, gy, gx, gtail, gw, gb, part, s)
     TSF_CONV_K_SWITCH(K, CALL)
 #undef CALL
