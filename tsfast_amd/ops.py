@@ -18,7 +18,14 @@ __all__ = ["custom_op"]
 import torch
 from torch.autograd import forward_ad
 
-_C = torch._C
+# bound once: every call asks all of these (0.5 us of a call of four tensors, on the build machine)
+_dispatch_keys = torch._C._dispatch_keys
+_len_dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_mode = torch._C._is_torch_function_mode_enabled
+_transform = torch._C._functorch.peek_interpreter_stack
+_tracing_state = torch._C._get_tracing_state
+_profiler = torch._C._autograd._profiler_enabled
+_registered = torch.library._impls  # what Python code has registered on any op, as "namespace/op/key"
 # dispatch keys of a plain dense GPU tensor (made in and outside inference mode); any other key
 # (conjugate or negative views, subclasses, functional, sparse, nested, batched ..) needs the dispatcher
 _plain_keys: set[int] = set()
@@ -30,7 +37,7 @@ def _keys_of_plain(device: torch.device) -> set[int]:
     keys = set()
     for mode in (False, True):
         with torch.inference_mode(mode):
-            keys.add(_C._dispatch_keys(torch.empty(0, device=device)).raw_repr())
+            keys.add(_dispatch_keys(torch.empty(0, device=device)).raw_repr())
     return keys
 
 
@@ -39,18 +46,18 @@ def _plain(t) -> bool:
         return False
     if not _plain_keys and t.is_cuda:
         _plain_keys.update(_keys_of_plain(t.device))
-    return _C._dispatch_keys(t).raw_repr() in _plain_keys
+    return _dispatch_keys(t).raw_repr() in _plain_keys
 
 
 def _unobserved() -> bool:
     """No trace, transform, mode or profiler would see an op called now."""
     return (
-        _C._len_torch_dispatch_stack() == 0
-        and not _C._is_torch_function_mode_enabled()
-        and _C._functorch.peek_interpreter_stack() is None
-        and _C._get_tracing_state() is None
+        _len_dispatch_modes() == 0
+        and not _function_mode()
+        and _transform() is None
+        and _tracing_state() is None
         and forward_ad._current_level < 0
-        and not _C._autograd._profiler_enabled()
+        and not _profiler()
     )
 
 
@@ -94,7 +101,7 @@ class _Op:
         self._function, self._backward = Direct, self._def._backward_fn
 
     def _overridden(self) -> bool:
-        return not self._overrides.isdisjoint(torch.library._impls) or self._def._backward_fn is not self._backward
+        return not self._overrides.isdisjoint(_registered) or self._def._backward_fn is not self._backward
 
     def __call__(self, *args, **kwargs):
         if kwargs or torch.compiler.is_compiling() or not _unobserved() or self._overridden():
