@@ -158,7 +158,8 @@ int tsfast_hip_mamba_fwd(int64_t B, int64_t L, int64_t D, int64_t N, int io_dtyp
                          const float* h0, void* out, float* h_last, float* chk, void* stream);
 /* The same forward with a workspace: where B x ceil(D / 32) workgroups leave the chip idle and D <= 1024
  * the rows are cut into time segments that run side by side, and the workspace holds the segments'
- * state maps (0 bytes where the rows are walked whole; workspace == NULL always walks them whole). */
+ * state maps (0 bytes where the rows are walked whole; workspace == NULL always walks them whole). A
+ * row that is cut agrees with the same row in another batch, or walked whole, to fp32 rounding. */
 int64_t tsfast_hip_mamba_fwd_workspace_bytes(int64_t B, int64_t L, int64_t D, int64_t N);
 int tsfast_hip_mamba_fwd_ws(int64_t B, int64_t L, int64_t D, int64_t N, int io_dtype, const void* draw, const float* A,
                             const void* Bt, const void* Ct, const void* u, const void* z, const float* Dp,

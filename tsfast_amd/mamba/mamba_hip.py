@@ -290,6 +290,10 @@ def run(draw, A, Bt, Ct, u, z, Dp, h0):
     Returns ``(out [B, L, D], h_last [B, D, N] float32)``; differentiable in all inputs. Without
     grad the inference op (no checkpoints) runs. (Contract of ``mamba_triton.py:523-534``.)
 
+    Rows of more than 1024 channels give the same bits alone and in a batch. Narrower rows may be cut
+    into time segments whose number depends on the batch beside them: their results agree to float32
+    rounding (before rounding to bfloat16 I/O).
+
     A launch serves at most 64 states. Larger N runs the states in groups of up to 64: the states
     evolve independently, and the output is linear in the per-state sum ``h . C`` for fixed
     draw, u, z (``out = (sum over groups of h_g . C_g + Dp u) * silu(z)``), so the groups' outputs
