@@ -80,7 +80,7 @@ MEASURED_TRAFFIC = {
 MEASURED_VALU = {
     (3, "bf16"): {
         "fwd": (230_092_800, "profiles/mamba_scan_config3_valu.md"),
-        "bwd": (501_884_608, "profiles/mamba_scan_config3_valu.md"),
+        "bwd": (501_946_264, "profiles/mamba_scan_config3_valu.md"),
     },
 }
 VALU_PEAK_CLOCK_HZ = 2.4e9  # MI355X peak engine clock
